@@ -301,6 +301,7 @@ QNode4 quantize_node(const Node4 &n, bool tlas) {
     const float *hi[3] = {n.hi_x, n.hi_y, n.hi_z};
     uint8_t *qlo[3] = {q.lo_x, q.lo_y, q.lo_z};
     uint8_t *qhi[3] = {q.hi_x, q.hi_y, q.hi_z};
+    float *steps[3] = {&q.step_x, &q.step_y, &q.step_z};
     bool any = false;
     float nlo[3] = {0, 0, 0}, nhi[3] = {0, 0, 0};
     for (int i = 0; i < 4; ++i) {
@@ -320,8 +321,8 @@ QNode4 quantize_node(const Node4 &n, bool tlas) {
             e = std::max(-126, static_cast<int>(std::ceil(std::log2(extent / 255.0))));
             while (e < 127 && std::ceil(extent / std::ldexp(1.0, e)) > 255.0) ++e;
         }
-        q.exp[a] = static_cast<int8_t>(e);
         const double step = std::ldexp(1.0, e);
+        *steps[a] = static_cast<float>(step);
         for (int i = 0; i < 4; ++i) {
             if (n.count[i] == kEmptySlot) continue;
             // outward rounding, checked in exact arithmetic

@@ -56,16 +56,16 @@ constexpr uint32_t kKindInstance = 0xc0000000u;  // instance index
 
 // The node record the kernels traverse: a Node4 quantised to 64 bytes, so a
 // node fetch moves half the bytes and the L2 holds twice the nodes.  Child
-// bound = origin + q * 2^exp per axis, with q an 8-bit integer rounded
-// outward (bounds only grow, so culling stays conservative).  ref[i] is the
-// child's traversal entry (kind | index), kEmptySlot for an unused slot.
+// bound = origin + q * step per axis, with step a power of two and q an 8-bit
+// integer rounded outward (bounds only grow, so culling stays conservative).
+// ref[i] is the child's traversal entry (kind | index), kEmptySlot for an
+// unused slot.
 struct alignas(16) QNode4 {
     float origin[3];
-    int8_t exp[3];
-    uint8_t pad0;
+    float step_x;
     uint8_t lo_x[4], hi_x[4], lo_y[4], hi_y[4];
     uint8_t lo_z[4], hi_z[4];
-    uint32_t pad1[2];
+    float step_y, step_z;
     uint32_t ref[4];
 };
 static_assert(sizeof(QNode4) == 64, "QNode4 must be 64 bytes");

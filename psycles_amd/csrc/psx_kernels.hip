@@ -117,7 +117,7 @@ __global__ __launch_bounds__(kBlock) void render_kernel(SceneView s, KernelParam
                                                          const float *filter, FilmView film, uint32_t first,
                                                          uint32_t count, Counters *counters, uint32_t *spill,
                                                          uint32_t *cursor) {
-    __shared__ uint32_t lds[kShortStack * kBlock];
+    __shared__ uint32_t lds[kTraversalLds * kBlock];
     __shared__ float4 lamp_sphere[kLampCache];
     __shared__ uint32_t lamp_bits[kLampCache];
     const LampView lv = stage_lamps(s, lamp_sphere, lamp_bits);
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kBlock) void render_kernel(SceneView s, KernelParam
 __global__ __launch_bounds__(kBlock) void trace_kernel(SceneView s, KernelParams k, const float4 *sobol,
                                                         const float *filter, uint32_t sample, uint32_t *records,
                                                         uint32_t *spill) {
-    __shared__ uint32_t lds[kShortStack * kBlock];
+    __shared__ uint32_t lds[kTraversalLds * kBlock];
     __shared__ float4 lamp_sphere[kLampCache];
     __shared__ uint32_t lamp_bits[kLampCache];
     const LampView lv = stage_lamps(s, lamp_sphere, lamp_bits);
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(kBlock) void path_trace_kernel(SceneView s, KernelP
                                                              const float *filter, uint32_t sample, uint32_t px,
                                                              uint32_t py, float4 *slots, uint32_t *records,
                                                              uint32_t *spill) {
-    __shared__ uint32_t lds[kShortStack * kBlock];
+    __shared__ uint32_t lds[kTraversalLds * kBlock];
     __shared__ float4 lamp_sphere[kLampCache];
     __shared__ uint32_t lamp_bits[kLampCache];
     const LampView lv = stage_lamps(s, lamp_sphere, lamp_bits);
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kBlock) void path_trace_kernel(SceneView s, KernelP
 __global__ __launch_bounds__(kBlock) void primary_kernel(SceneView s, KernelParams k, const float4 *sobol,
                                                           const float *filter, uint32_t sample, uint32_t *records,
                                                           uint32_t *spill) {
-    __shared__ uint32_t lds[kShortStack * kBlock];
+    __shared__ uint32_t lds[kTraversalLds * kBlock];
     Stack st = block_stack(lds, spill);
     const uint32_t tiles = tile_count(k);
     const uint32_t waves = gridDim.x * (kBlock / 64u);

@@ -289,48 +289,73 @@ struct Hit {
     bool valid;
 };
 
+// Words of a query that the traversal touches a few times per ray: they live
+// in LDS beside the stack, so that the registers a step carries are few and
+// its predicated writes are stores instead of register copies.
+enum ColdWord : uint32_t {
+    kColdOrigin = 0u, kColdDirection = 3u, kColdTmax = 6u, kColdVisibility = 7u, kColdSource = 8u, kColdLight = 10u,
+    kColdWeights = 12u, kColdHit = 15u, kColdWords = 18u
+};
+constexpr uint32_t kTraversalLds = kShortStack + kColdWords;  // LDS words per lane
+
+// LDS accesses through this type stay LDS instructions where a plain pointer
+// may become a generic one.
+typedef __attribute__((address_space(3))) uint32_t LdsWord;
+
 // Per-lane traversal stack: the top kShortStack entries live in LDS laid out
 // [entry][lane] (bank-conflict free), older entries move to a per-lane column
 // of an HBM spill buffer laid out [entry][lane of the grid].  Scene
 // compilation bounds the depth by kTraversalStackDepth.
 struct Stack {
-    uint32_t *lds;    // block base of the LDS ring
+    LdsWord *lds;     // this lane's column of the LDS ring; the cold words follow
     uint32_t *spill;  // this lane's spill column
     uint32_t lanes;   // LDS row stride (lanes per block)
-    uint32_t lane;    // lane within the block
     uint32_t stride;  // spill row stride (lanes of the grid)
     int sp, bottom;   // entries [bottom, sp) are in LDS, [0, bottom) spilled
 
-    __device__ __forceinline__ void push(uint32_t e) {
-        if (sp >= kStackDepth) return;
-        if (sp - bottom == static_cast<int>(kShortStack)) {
-            spill[static_cast<size_t>(bottom) * stride] = lds[(bottom & (kShortStack - 1u)) * lanes + lane];
+    // makes room for three entries in the ring
+    __device__ __forceinline__ void reserve3() {
+        while (sp + 3 - bottom > static_cast<int>(kShortStack)) {
+            if (bottom < kStackDepth)
+                spill[static_cast<size_t>(bottom) * stride] = lds[(bottom & (kShortStack - 1u)) * lanes];
             ++bottom;
         }
-        lds[(sp & (kShortStack - 1u)) * lanes + lane] = e;
-        ++sp;
+    }
+    // After reserve3(): the slot is written either way and kept when `keep`,
+    // so three pushes are straight-line code.
+    __device__ __forceinline__ void push_if(uint32_t e, bool keep) {
+        lds[(sp & (kShortStack - 1u)) * lanes] = e;
+        sp += keep ? 1 : 0;
     }
     __device__ __forceinline__ uint32_t pop() {
         --sp;
-        // the LDS slot is read unconditionally (the index is always in the
-        // ring), so the common case stays an LDS access instead of one
-        // generic load that selects between LDS and the spill column
-        uint32_t e = lds[(sp & (kShortStack - 1u)) * lanes + lane];
+        // the LDS slot is read unconditionally (the index is always in the ring)
+        uint32_t e = lds[(sp & (kShortStack - 1u)) * lanes];
         if (sp < bottom) {
             bottom = sp;
             e = spill[static_cast<size_t>(sp) * stride];
         }
         return e;
     }
+    __device__ __forceinline__ uint32_t word(uint32_t i) const { return lds[(kShortStack + i) * lanes]; }
+    __device__ __forceinline__ void set_word(uint32_t i, uint32_t v) const { lds[(kShortStack + i) * lanes] = v; }
+    __device__ __forceinline__ float number(uint32_t i) const { return __uint_as_float(word(i)); }
+    __device__ __forceinline__ void set_number(uint32_t i, float v) const { set_word(i, __float_as_uint(v)); }
+    __device__ __forceinline__ f3 vec(uint32_t i) const { return V(number(i), number(i + 1u), number(i + 2u)); }
+    __device__ __forceinline__ void set_vec(uint32_t i, f3 v) const {
+        set_number(i, v.x);
+        set_number(i + 1u, v.y);
+        set_number(i + 2u, v.z);
+    }
 };
 
+// `lds` holds kTraversalLds * `lanes` words
 __device__ __forceinline__ Stack make_stack(uint32_t *lds, uint32_t *spill, uint32_t lanes, uint32_t lane,
                                             uint32_t global_lane, uint32_t stride) {
     Stack st;
-    st.lds = lds;
+    st.lds = (LdsWord *)(lds + lane);
     st.spill = spill + global_lane;
     st.lanes = lanes;
-    st.lane = lane;
     st.stride = stride;
     st.sp = 0;
     st.bottom = 0;
@@ -347,9 +372,13 @@ __device__ __forceinline__ f3 pluecker_cross(f3 a, f3 b) {
 }
 __device__ __forceinline__ float pluecker_dot(f3 a, f3 b) { return fmaf(a.x, b.x, fmaf(a.y, b.y, a.z * b.z)); }
 
+// Candidate of the exact Pluecker test: distance and the raw edge weights.
+struct Candidate {
+    float t, u, v, sum;
+};
+
 // d is already clamped with clamp_bvh_dir
-__device__ __forceinline__ bool pluecker(f3 o, f3 d, float tmin, float tmax, f3 p0, f3 p1, f3 p2,
-                                         float &t, float &bu, float &bv) {
+__device__ __forceinline__ bool pluecker(f3 o, f3 d, float tmin, float tmax, f3 p0, f3 p1, f3 p2, Candidate &c) {
     const f3 v0 = p0 - o, v1 = p1 - o, v2 = p2 - o;
     const f3 e0 = v2 - v0, e1 = v0 - v1, e2 = v1 - v2;
     const float u = pluecker_dot(pluecker_cross(e0, v2 + v0), d);
@@ -363,25 +392,22 @@ __device__ __forceinline__ bool pluecker(f3 o, f3 d, float tmin, float tmax, f3 
     const f3 n2 = pluecker_cross(e1, e0) * 2.0f;
     const float den = pluecker_dot(n2, d);
     const float safe_den = den != 0.0f ? den : 1.0f;
-    t = pluecker_dot(v0, n2) / safe_den;
-    const bool in_range = (t >= tmin) && (t <= tmax);
+    const float t = pluecker_dot(v0, n2) / safe_den;
+    c = Candidate{t, u, v, sum};
+    return inside && den != 0.0f && t >= tmin && t <= tmax;
+}
+
+// barycentrics of an accepted candidate
+__device__ __forceinline__ void pluecker_uv(float u, float v, float sum, float &bu, float &bv) {
     const float rs = fabsf(sum) >= 1.0e-18f ? 1.0f / sum : 0.0f;
     bu = fminf(u * rs, 1.0f);
     bv = fminf(v * rs, 1.0f);
-    return inside && den != 0.0f && in_range;
 }
 
 struct TraceQuery {
     uint32_t visibility;
     uint32_t src_obj, src_prim, light_obj, light_prim;
 };
-
-__device__ __forceinline__ bool order_accepts(const Hit &best, float t, uint32_t object, uint32_t prim) {
-    if (!best.valid) return true;
-    if (t < best.t) return true;
-    if (t == best.t) return object > best.object || (object == best.object && prim > best.cprim);
-    return false;
-}
 
 // compare-exchange of a sorting network on (distance, entry) pairs
 __device__ __forceinline__ void sort_pair(float &ka, uint32_t &ea, float &kb, uint32_t &eb) {
@@ -415,151 +441,124 @@ __device__ __forceinline__ uint32_t hit_material(const SceneView &s, uint32_t in
 // padded at build time and the far distance is widened), so traversal order
 // never changes the result, only its cost.
 //
-// The traversal is a resumable state machine (begin, then step until it
-// reports completion) so that persistent kernels can refill lanes whose ray
-// has finished while the rest of the wave keeps traversing.
+// The traversal is a resumable state machine that the lanes of a wave run
+// together.  A lane's next work is of one of three kinds: a node, a leaf
+// triangle, or a change of space (into an instance, or back to the world).
+// traversal_advance() counts the lanes ready for each kind and runs one kind
+// for the lanes that wait for it.  A lane that reaches a leaf sets it aside in
+// `leaf` and goes on with its stack, so it is ready for both kinds.
+//
+// What bounds it is VALU issue, then random fetches: with all three kinds in
+// one divergent step the trace kernel issued VALU work on 84 % of the SIMD's
+// cycles with 26 of 64 lanes on (instanced frame; 21 many-light, 22 slabs).
+// One kind at a time has 37 lanes on and three quarters of the instructions:
+// trace kernel 83.2 -> 63.9 ms (instanced frame, 1920x1080x64), 210 -> 150
+// (many lights, x32), 107 -> 81 (13 slabs, 773x773x37).
 struct Traversal {
-    Ray ray;        // world ray of the query
-    TraceQuery q;
-    f3 o, d, inv, oi;  // ray in the current intersection space; oi = o * inv
-    float lower;
-    Hit best;
-    uint32_t current;
+    f3 o, d, inv, oi;   // ray in the current intersection space; oi = o * inv
+    float tmin, lower;  // lower: tmin widened for the box tests
+    float best_t;       // tmax until a hit is found
+    uint32_t cur;       // next entry, or kEmptySlot
+    uint32_t leaf;      // leaf set aside, or kEmptySlot
     uint32_t inst_index, inst_prim_offset;
-    bool in_blas;
-    // Any-hit traversal (traversal_step<COUNT, true>, for shadow queries)
-    // ends at the first accepted candidate on an instance whose every
-    // material is opaque to shadow rays (`stop` while inside such an
-    // instance; `opaque` once ended): the transparent shadow loop's
-    // transmittance is then exactly zero whatever else lies on the ray, so
-    // the early end changes no result bit.
+    // stack level at which the current instance was entered, 0 in the world,
+    // kStale when the stack is back in the world and o and d still an instance's
+    int base;
+    // Any-hit traversal (ANYHIT, for shadow queries) ends at the first
+    // accepted candidate on an instance whose every material is opaque to
+    // shadow rays (`stop` while inside such an instance; `opaque` once
+    // ended): the transparent shadow loop's transmittance is then exactly
+    // zero whatever else lies on the ray, so the early end changes no result
+    // bit.
     bool stop, opaque;
 };
+constexpr int kStale = -1;
 
 __device__ __forceinline__ f3 clamped_dir(f3 d) {
     return V(clamp_bvh_dir(d.x), clamp_bvh_dir(d.y), clamp_bvh_dir(d.z));
 }
 
-__device__ __forceinline__ void traversal_world_space(Traversal &t) {
-    t.in_blas = false;
-    t.o = t.ray.o;
-    t.d = clamped_dir(t.ray.d);
-    t.inv = V(1.0f / t.d.x, 1.0f / t.d.y, 1.0f / t.d.z);
-    t.oi = t.o * t.inv;  // slab distances are fma(bound, inv, -o * inv)
+// Slab distances are fma(bound, inv, -o * inv).  They only prune, under
+// margins of 1e-5, so the hardware reciprocal (1 ulp) serves: it costs an
+// instruction where the correctly rounded division costs ten.
+__device__ __forceinline__ void traversal_space(Traversal &t, f3 o, f3 d) {
+    t.o = o;
+    t.d = clamped_dir(d);
+    t.inv = V(__builtin_amdgcn_rcpf(t.d.x), __builtin_amdgcn_rcpf(t.d.y), __builtin_amdgcn_rcpf(t.d.z));
+    t.oi = t.o * t.inv;
 }
 
-__device__ __forceinline__ void traversal_begin(const SceneView &s, Traversal &t, Stack &st) {
-    t.best.valid = false;
-    t.best.t = t.ray.tmax;
-    t.best.inst = t.best.prim = t.best.object = t.best.cprim = 0xffffffffu;
-    t.best.u = t.best.v = 0.0f;
-    t.lower = t.ray.tmin > 0.0f ? t.ray.tmin * 0.99999f : t.ray.tmin - 1.0e-30f;
-    t.inst_index = t.inst_prim_offset = 0u;
-    t.stop = t.opaque = false;
-    traversal_world_space(t);
+__device__ __forceinline__ void traversal_idle(Traversal &t, Stack &st) {
+    t.cur = t.leaf = kEmptySlot;
+    t.base = 0;
     st.sp = 0;
     st.bottom = 0;
-    t.current = s.has_tlas ? (s.tlas_root | kKindTlas) : kEmptySlot;
 }
 
-// One traversal iteration: an instance entry, a leaf or an inner node.
-// Returns false once the query is complete (t.best holds the result).
-template <bool COUNT, bool ANYHIT = false>
-__device__ __forceinline__ bool traversal_step(const SceneView &s, Traversal &t, Stack &st, uint32_t &node_count,
-                                               uint32_t &tri_count) {
-    if (t.current == kEmptySlot) {
-        if (st.sp == 0) return false;
-        t.current = st.pop();
+// starts the search of the ray (o, d) from `tmin` up to `tmax`
+__device__ __forceinline__ void traversal_start(const SceneView &s, Traversal &t, Stack &st, f3 o, f3 d, float tmin,
+                                                float tmax) {
+    t.tmin = tmin;
+    t.lower = tmin > 0.0f ? tmin * 0.99999f : tmin - 1.0e-30f;
+    t.best_t = tmax;
+    st.set_word(kColdHit, kNone);
+    t.inst_index = t.inst_prim_offset = 0u;
+    t.stop = t.opaque = false;
+    traversal_space(t, o, d);
+    traversal_idle(t, st);
+    // a NaN anywhere in the ray fails every triangle test: nothing to search
+    const bool nan = __builtin_isunordered(o.x, d.x) || __builtin_isunordered(o.y, d.y) ||
+                     __builtin_isunordered(o.z, d.z) || __builtin_isunordered(tmin, tmax);
+    if (s.has_tlas && !nan) t.cur = s.tlas_root | kKindTlas;
+}
+
+__device__ __forceinline__ void traversal_begin(const SceneView &s, Traversal &t, Stack &st, const Ray &ray,
+                                                const TraceQuery &q) {
+    st.set_vec(kColdOrigin, ray.o);
+    st.set_vec(kColdDirection, ray.d);
+    st.set_number(kColdTmax, ray.tmax);
+    st.set_word(kColdVisibility, q.visibility);
+    st.set_word(kColdSource, q.src_obj);
+    st.set_word(kColdSource + 1u, q.src_prim);
+    st.set_word(kColdLight, q.light_obj);
+    st.set_word(kColdLight + 1u, q.light_prim);
+    traversal_start(s, t, st, ray.o, ray.d, ray.tmin, ray.tmax);
+}
+
+// the same query again, from `tmin`
+__device__ __forceinline__ void traversal_resume(const SceneView &s, Traversal &t, Stack &st, float tmin) {
+    traversal_start(s, t, st, st.vec(kColdOrigin), st.vec(kColdDirection), tmin, st.number(kColdTmax));
+}
+
+__device__ __forceinline__ bool traversal_busy(const Traversal &t, const Stack &st) {
+    return (t.cur & t.leaf) != kEmptySlot || st.sp > 0;
+}
+
+__device__ __forceinline__ Hit traversal_result(const Traversal &t, const Stack &st) {
+    Hit h;
+    h.inst = h.object = st.word(kColdHit);
+    h.valid = h.inst != kNone;
+    h.prim = h.cprim = kNone;
+    h.u = h.v = 0.0f;
+    h.t = t.best_t;
+    if (h.valid) {
+        h.prim = st.word(kColdHit + 1u);
+        h.cprim = st.word(kColdHit + 2u);
+        pluecker_uv(st.number(kColdWeights), st.number(kColdWeights + 1u), st.number(kColdWeights + 2u), h.u, h.v);
     }
-    const uint32_t entry = t.current;
-    t.current = kEmptySlot;
-    const uint32_t kind = entry & kKindMask;
-    const uint32_t index = entry & ~kKindMask;
-    // back at the top level: world ray again
-    if (t.in_blas && (kind == kKindTlas || kind == kKindInstance)) traversal_world_space(t);
-    if (kind == kKindInstance) {
-        // enter an instance: object-space ray with the Cycles FMA transform
-        const Instance &inst = s.instances[index];
-        if ((inst.visibility & t.q.visibility) == 0u) return true;
-        t.inst_index = index;
-        t.inst_prim_offset = inst.prim_offset;
-        t.in_blas = true;
-        if (ANYHIT) t.stop = s.instance_opaque[index] != 0u;
-        if (!inst.applied) {
-            t.o = affine_point(inst.w2o, t.ray.o);
-            t.d = clamped_dir(affine_dir(inst.w2o, t.ray.d));
-            t.inv = V(1.0f / t.d.x, 1.0f / t.d.y, 1.0f / t.d.z);
-            t.oi = t.o * t.inv;
-        }
-        t.current = inst.blas_root | kKindBlas;
-        return true;
-    }
-    // One 64-byte fetch serves both kinds of step: a node record, or a leaf
-    // triangle (48 bytes, the next 16 read and ignored; the triangle array
-    // carries one record of padding).  Lanes of a wave that sit on nodes and
-    // on triangles then wait on one memory round trip per step, not two.
-    const bool is_leaf = kind == kKindLeaf;
-    const uint4 *rec = is_leaf ? reinterpret_cast<const uint4 *>(s.tris + (index >> 3))
-                               : reinterpret_cast<const uint4 *>(s.nodes + index);
-    const uint4 r0 = rec[0], r1 = rec[1], r2 = rec[2], r3 = rec[3];
-    if (is_leaf) {
-        // one triangle per step: a wave whose lanes sit on leaves of
-        // different sizes then runs one intersection test per step instead
-        // of the longest leaf's loop; the rest of the leaf is the next step
-        const uint32_t first = index >> 3;
-        const uint32_t n = (index & 7u) + 1u;
-        if (n > 1u) t.current = (((first + 1u) << 3) | (n - 2u)) | kKindLeaf;
-        {
-            if (COUNT) tri_count++;
-            float th, bu, bv;
-            const bool ok = pluecker(t.o, t.d, t.ray.tmin, t.ray.tmax,
-                                     V(__uint_as_float(r0.x), __uint_as_float(r0.y), __uint_as_float(r0.z)),
-                                     V(__uint_as_float(r1.x), __uint_as_float(r1.y), __uint_as_float(r1.z)),
-                                     V(__uint_as_float(r2.x), __uint_as_float(r2.y), __uint_as_float(r2.z)), th, bu, bv);
-            if (!ok) return true;
-            const uint32_t prim = r0.w;
-            const uint32_t cprim = t.inst_prim_offset + prim;
-            const bool excluded = (t.inst_index == t.q.src_obj && cprim == t.q.src_prim) ||
-                                  (t.inst_index == t.q.light_obj && cprim == t.q.light_prim);
-            if (excluded) return true;
-            if (ANYHIT && t.stop) {
-                // any opaque candidate in [tmin, tmax] zeroes the shadow
-                t.opaque = true;
-                t.best.valid = true;
-                t.best.t = th;
-                t.best.u = bu;
-                t.best.v = bv;
-                t.best.inst = t.best.object = t.inst_index;
-                t.best.prim = prim;
-                t.best.cprim = cprim;
-                t.current = kEmptySlot;
-                st.sp = 0;
-                st.bottom = 0;
-                return true;
-            }
-            if (!order_accepts(t.best, th, t.inst_index, cprim)) return true;
-            t.best.valid = true;
-            t.best.t = th;
-            t.best.u = bu;
-            t.best.v = bv;
-            t.best.inst = t.inst_index;
-            t.best.prim = prim;
-            t.best.object = t.inst_index;
-            t.best.cprim = cprim;
-        }
-        return true;
-    }
-    // inner node: test the four child boxes, continue with the nearest hit
-    // child and push the others far-to-near
-    const uint4 head = r0, qxy = r1, qz = r2, refs = r3;
+    return h;
+}
+
+// the four child boxes of a node: continue with the nearest hit child, push
+// the others far to near
+template <bool COUNT>
+__device__ __forceinline__ void traversal_node(const SceneView &s, Traversal &t, Stack &st, uint32_t &node_count) {
+    const uint4 *rec = reinterpret_cast<const uint4 *>(s.nodes + (t.cur & ~kKindMask));
+    const uint4 head = rec[0], qxy = rec[1], qz = rec[2], refs = rec[3];
     if (COUNT) node_count++;
-    const float upper = (t.best.valid ? t.best.t : t.ray.tmax) * 1.00001f + 1.0e-30f;
-    // slab distance of origin + q * 2^e is fma(q, 2^e * inv, origin * inv - o * inv)
-    auto pow2 = [](uint32_t bits, int shift) {
-        const int e = static_cast<int>(static_cast<int8_t>((bits >> shift) & 0xffu));
-        return __uint_as_float(static_cast<uint32_t>(e + 127) << 23);
-    };
-    const float sx = pow2(head.w, 0) * t.inv.x, sy = pow2(head.w, 8) * t.inv.y, sz = pow2(head.w, 16) * t.inv.z;
+    // slab distance of origin + q * step is fma(q, step * inv, origin * inv - o * inv)
+    const float sx = __uint_as_float(head.w) * t.inv.x, sy = __uint_as_float(qz.z) * t.inv.y,
+                sz = __uint_as_float(qz.w) * t.inv.z;
     const float bx = fmaf(__uint_as_float(head.x), t.inv.x, -t.oi.x);
     const float by = fmaf(__uint_as_float(head.y), t.inv.y, -t.oi.y);
     const float bz = fmaf(__uint_as_float(head.z), t.inv.z, -t.oi.z);
@@ -577,8 +576,8 @@ __device__ __forceinline__ bool traversal_step(const SceneView &s, Traversal &t,
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         // conservative: boxes are padded by 1e-5 of their coordinate
-        // magnitude before quantisation, which rounds outward, and `far` is
-        // widened by 1e-5, all far above the rounding of these slab terms
+        // magnitude before quantisation, which rounds outward, and the far end
+        // is widened by 1e-5, all far above the rounding of these slab terms
         const int sh = 8 * i;
         const float t0x = fmaf(static_cast<float>((nx >> sh) & 0xffu), sx, bx);
         const float t1x = fmaf(static_cast<float>((fx >> sh) & 0xffu), sx, bx);
@@ -586,11 +585,10 @@ __device__ __forceinline__ bool traversal_step(const SceneView &s, Traversal &t,
         const float t1y = fmaf(static_cast<float>((fy >> sh) & 0xffu), sy, by);
         const float t0z = fmaf(static_cast<float>((nz >> sh) & 0xffu), sz, bz);
         const float t1z = fmaf(static_cast<float>((fz >> sh) & 0xffu), sz, bz);
-        const float near = fmaxf(fmaxf(t0x, t0y), t0z);
-        const float far = fminf(fminf(t1x, t1y), t1z);
-        const float far_safe = far * 1.00001f + 1.0e-30f;
+        const float near = fmaxf(fmaxf(fmaxf(t0x, t0y), t0z), t.lower);
+        const float far = fminf(fminf(fminf(t1x, t1y), t1z), t.best_t);
         const uint32_t ref = ref_arr[i];
-        const bool hit = ref != kEmptySlot && near <= far_safe && far_safe >= t.lower && near <= upper;
+        const bool hit = ref != kEmptySlot && near <= fmaf(far, 1.00001f, 1.0e-30f);
         key[i] = hit ? near : INFINITY;
         ent[i] = ref;
     }
@@ -599,24 +597,121 @@ __device__ __forceinline__ bool traversal_step(const SceneView &s, Traversal &t,
     sort_pair(key[0], ent[0], key[2], ent[2]);
     sort_pair(key[1], ent[1], key[3], ent[3]);
     sort_pair(key[1], ent[1], key[2], ent[2]);
-    if (key[3] != INFINITY) st.push(ent[3]);
-    if (key[2] != INFINITY) st.push(ent[2]);
-    if (key[1] != INFINITY) st.push(ent[1]);
-    if (key[0] != INFINITY) t.current = ent[0];
-    return true;
+    st.reserve3();
+    st.push_if(ent[3], key[3] != INFINITY);
+    st.push_if(ent[2], key[2] != INFINITY);
+    st.push_if(ent[1], key[1] != INFINITY);
+    t.cur = key[0] != INFINITY ? ent[0] : kEmptySlot;
+}
+
+// One triangle of the leaf set aside; the rest of the leaf stays there.
+template <bool COUNT, bool ANYHIT>
+__device__ __forceinline__ void traversal_leaf(const SceneView &s, Traversal &t, Stack &st, uint32_t &tri_count) {
+    const uint32_t index = t.leaf & ~kKindMask;
+    const uint32_t first = index >> 3, more = index & 7u;
+    const uint4 *rec = reinterpret_cast<const uint4 *>(s.tris + first);
+    const uint4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
+    t.leaf = more != 0u ? ((((first + 1u) << 3) | (more - 1u)) | kKindLeaf) : kEmptySlot;
+    if (COUNT) tri_count++;
+    Candidate c;
+    const bool ok = pluecker(t.o, t.d, t.tmin, t.best_t,
+                             V(__uint_as_float(r0.x), __uint_as_float(r0.y), __uint_as_float(r0.z)),
+                             V(__uint_as_float(r1.x), __uint_as_float(r1.y), __uint_as_float(r1.z)),
+                             V(__uint_as_float(r2.x), __uint_as_float(r2.y), __uint_as_float(r2.z)), c);
+    if (!ok) return;
+    const uint32_t prim = r0.w, inst = t.inst_index;
+    const uint32_t cprim = t.inst_prim_offset + prim;
+    const bool excluded = (inst == st.word(kColdSource) && cprim == st.word(kColdSource + 1u)) ||
+                          (inst == st.word(kColdLight) && cprim == st.word(kColdLight + 1u));
+    // at the best distance so far the greatest (object, primitive) wins
+    const uint32_t best_inst = st.word(kColdHit), best_cprim = st.word(kColdHit + 2u);
+    const bool loses = c.t == t.best_t && best_inst != kNone &&
+                       (inst < best_inst || (inst == best_inst && cprim <= best_cprim));
+    if (excluded || loses) return;
+    t.best_t = c.t;
+    st.set_number(kColdWeights, c.u);
+    st.set_number(kColdWeights + 1u, c.v);
+    st.set_number(kColdWeights + 2u, c.sum);
+    st.set_word(kColdHit, inst);
+    st.set_word(kColdHit + 1u, prim);
+    st.set_word(kColdHit + 2u, cprim);
+    if (ANYHIT && t.stop) {
+        // any opaque candidate in [tmin, tmax] zeroes the shadow
+        t.opaque = true;
+        traversal_idle(t, st);
+    }
+}
+
+// A lane that enters an instance, or whose stack came back to the world.
+template <bool ANYHIT>
+__device__ __forceinline__ void traversal_change_space(const SceneView &s, Traversal &t, Stack &st) {
+    f3 o = st.vec(kColdOrigin), d = st.vec(kColdDirection);
+    int base = 0;
+    if (t.cur >= kKindInstance) {
+        const uint32_t index = t.cur & ~kKindMask;
+        const Instance &inst = s.instances[index];
+        const Affine w2o = inst.w2o;
+        // an invisible instance leaves the lane in its space with nothing to
+        // do there, which is the state of a lane that came back from it
+        const bool visible = (inst.visibility & st.word(kColdVisibility)) != 0u;
+        const bool applied = inst.applied != 0u;
+        t.cur = visible ? inst.blas_root | kKindBlas : kEmptySlot;
+        base = visible ? st.sp : kStale;
+        t.inst_index = index;
+        t.inst_prim_offset = inst.prim_offset;
+        if (ANYHIT) t.stop = s.instance_opaque[index] != 0u;
+        // object-space ray with the Cycles FMA transform
+        const f3 oo = affine_point(w2o, o), od = affine_dir(w2o, d);
+        o = sel(oo, o, applied);
+        d = sel(od, d, applied);
+    }
+    t.base = base;
+    traversal_space(t, o, d);
+}
+
+// Advances the wave's lanes by one step of the kind that most of them wait
+// for.  Called by the lanes of a wave together; idle lanes take no part.  The
+// three kinds are three predicated blocks in a row, not branches: as branches
+// the compiler copied the ray's registers around each of them (17 moves a
+// step).
+template <bool COUNT, bool ANYHIT = false>
+__device__ __forceinline__ void traversal_advance(const SceneView &s, Traversal &t, Stack &st, uint32_t &node_count,
+                                                  uint32_t &tri_count) {
+    // set a leaf aside, then take the next entry from the stack; as signed
+    // words, nodes are >= 0 and leaves the least
+    if (t.leaf == kEmptySlot && t.base >= 0 && static_cast<int>(t.cur) < static_cast<int>(kKindInstance)) {
+        t.leaf = t.cur;
+        t.cur = kEmptySlot;
+    }
+    if (t.cur == kEmptySlot && st.sp > 0) {
+        if (st.sp == t.base) t.base = kStale;
+        t.cur = st.pop();
+    }
+    const bool leaf = t.leaf != kEmptySlot;
+    const bool stale = t.base < 0;
+    const bool node = static_cast<int>(t.cur) >= 0 && !stale;
+    const bool changes = t.cur != kEmptySlot && !leaf && (stale || t.cur >= kKindInstance);
+    const uint32_t n_node = static_cast<uint32_t>(__popcll(__builtin_amdgcn_ballot_w64(node)));
+    const uint32_t n_leaf = static_cast<uint32_t>(__popcll(__builtin_amdgcn_ballot_w64(leaf)));
+    const uint32_t n_change = static_cast<uint32_t>(__popcll(__builtin_amdgcn_ballot_w64(changes)));
+    // Lanes that wait for a change of space can do nothing else, while most
+    // lanes with a leaf aside have a node too, so a change counts double.
+    // Weights of 1 or 4 for it and of 0.75 to 1.5 for leaves are within 2 %.
+    const bool run_change = n_change > 0u && 2u * n_change >= n_node && 2u * n_change >= n_leaf;
+    const bool run_leaf = !run_change && n_leaf >= n_node;
+    if (changes && run_change) traversal_change_space<ANYHIT>(s, t, st);
+    if (leaf && run_leaf) traversal_leaf<COUNT, ANYHIT>(s, t, st, tri_count);
+    if (node && !run_change && !run_leaf) traversal_node<COUNT>(s, t, st, node_count);
 }
 
 template <bool COUNT, bool ANYHIT = false>
 __device__ Hit closest_hit(const SceneView &s, const Ray &ray, const TraceQuery &q, Stack &st,
                            uint32_t &node_count, uint32_t &tri_count, bool *opaque = nullptr) {
     Traversal t;
-    t.ray = ray;
-    t.q = q;
-    traversal_begin(s, t, st);
-    while (traversal_step<COUNT, ANYHIT>(s, t, st, node_count, tri_count)) {
-    }
+    traversal_begin(s, t, st, ray, q);
+    while (traversal_busy(t, st)) traversal_advance<COUNT, ANYHIT>(s, t, st, node_count, tri_count);
     if (opaque) *opaque = t.opaque;
-    return t.best;
+    return traversal_result(t, st);
 }
 
 // ===========================================================================

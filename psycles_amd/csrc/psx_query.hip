@@ -75,7 +75,7 @@ __device__ void run_query(const SceneView &s, const psx_ray_query &q, Stack &st,
 __global__ __launch_bounds__(kQueryBlock) void intersect_kernel(SceneView s, const psx_ray_query *queries,
                                                                 uint32_t count, psx_ray_hit *hits, uint32_t *cursor,
                                                                 uint32_t *spill) {
-    __shared__ uint32_t lds[kShortStack * kQueryBlock];
+    __shared__ uint32_t lds[kTraversalLds * kQueryBlock];
     Stack st = make_stack(lds, spill, kQueryBlock, threadIdx.x, blockIdx.x * kQueryBlock + threadIdx.x,
                           gridDim.x * kQueryBlock);
     const uint32_t lane = __lane_id();

@@ -211,7 +211,7 @@ __global__ __launch_bounds__(kShadeBlock) void generate_kernel(KernelParams k, c
 template <bool COUNT, bool SEGMENTED = false>
 __global__ __launch_bounds__(kTraceBlock, 4) void wf_trace_kernel(SceneView s, KernelParams k, WavefrontView w,
                                                                uint32_t it, Counters *counters, uint32_t *spill) {
-    __shared__ uint32_t lds[kShortStack * kTraceBlock];
+    __shared__ uint32_t lds[kTraversalLds * kTraceBlock];
     Stack st = make_stack(lds, spill, kTraceBlock, threadIdx.x, blockIdx.x * kTraceBlock + threadIdx.x,
                           gridDim.x * kTraceBlock);
     WavefrontCounters *c = w.counters + it;
@@ -221,6 +221,8 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wf_trace_kernel(SceneView s, K
     const unsigned long long below = (1ull << lane) - 1ull;
     uint32_t rays = 0u, nodes = 0u, tris = 0u;
     Traversal t;
+    traversal_idle(t, st);
+    // active: the lane owns a query; it is done once its traversal is no longer busy
     bool active = false, exhausted = false, shadow = false;
     uint32_t path = 0u, tdepth = 0u;
     f3 transmittance = V(1.0f, 1.0f, 1.0f);
@@ -289,60 +291,57 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wf_trace_kernel(SceneView s, K
                 if (entry != kSkip) {
                     path = entry >> 1;
                     shadow = (entry & 1u) != 0u;
+                    Ray ray;
+                    TraceQuery q;
                     if (shadow) {
                         const float4 o = w.shadow_o[path], d = w.shadow_d[path];
                         const uint4 sq = w.shadow_q[path];
-                        t.ray.o = V(o.x, o.y, o.z);
-                        t.ray.tmax = o.w;
-                        t.ray.d = V(d.x, d.y, d.z);
-                        t.ray.tmin = 0.0f;
-                        t.q.visibility = VIS_SHADOW;
-                        t.q.src_obj = sq.x;
-                        t.q.src_prim = sq.y;
-                        t.q.light_obj = sq.z;
-                        t.q.light_prim = sq.w;
+                        ray = Ray{V(o.x, o.y, o.z), V(d.x, d.y, d.z), 0.0f, o.w};
+                        q = TraceQuery{VIS_SHADOW, sq.x, sq.y, sq.z, sq.w};
                         tdepth = __float_as_uint(w.shadow_l[path].w);
                         transmittance = V(1.0f, 1.0f, 1.0f);
                     } else {
                         const float4 o = w.ray_o[path], d = w.ray_d[path];
                         const uint4 a = w.aux[path];
-                        t.ray.o = V(o.x, o.y, o.z);
-                        t.ray.tmin = o.w;
-                        t.ray.d = V(d.x, d.y, d.z);
-                        t.ray.tmax = d.w;
-                        t.q.visibility = contract_visibility(w.state0[path].y);
-                        t.q.src_obj = a.x;
-                        t.q.src_prim = a.y;
-                        t.q.light_obj = t.q.light_prim = 0xffffffffu;
+                        ray = Ray{V(o.x, o.y, o.z), V(d.x, d.y, d.z), o.w, d.w};
+                        q = TraceQuery{contract_visibility(w.state0[path].y), a.x, a.y, kNone, kNone};
                     }
-                    traversal_begin(s, t, st);
+                    traversal_begin(s, t, st, ray, q);
                     active = true;
                 }
             }
         }
-        if (__ballot(active) == 0ull) {
+        const unsigned long long owned = __ballot(active);
+        if (owned == 0ull) {
             if (exhausted && res == res_end) break;
             continue;
         }
-        // traverse until enough lanes are idle to refill (or all are, at the end)
-        for (;;) {
-            if (active && !traversal_step<COUNT>(s, t, st, nodes, tris)) {
-                ++rays;
-                if (!shadow) {
-                    const Hit &h = t.best;
-                    w.hit[path] = make_uint4(h.valid ? h.inst : kNone, h.prim, h.cprim, __float_as_uint(h.t));
-                    w.hit_uv[path] = make_float2(h.u, h.v);
-                    active = false;
-                } else if (shadow_hit(s, k.transparent_max, t.best, t.ray, tdepth, transmittance)) {
+        // Traverse until enough lanes are idle to refill.  With nothing left
+        // to refill from, stop when half of the owned lanes are done, so that
+        // a shadow ray past a transparent surface does not wait for the
+        // longest ray of its wave.
+        const uint32_t busy_min = !exhausted || res < res_end ? 64u - refill
+                                                              : static_cast<uint32_t>(__popcll(owned)) >> 1u;
+        do {
+            traversal_advance<COUNT>(s, t, st, nodes, tris);
+        } while (static_cast<uint32_t>(__popcll(__ballot(traversal_busy(t, st)))) > busy_min);
+        if (active && !traversal_busy(t, st)) {
+            ++rays;
+            const Hit h = traversal_result(t, st);
+            if (!shadow) {
+                w.hit[path] = make_uint4(h.inst, h.prim, h.cprim, __float_as_uint(h.t));
+                w.hit_uv[path] = make_float2(h.u, h.v);
+                active = false;
+            } else {
+                Ray rest;
+                if (shadow_hit(s, k.transparent_max, h, rest, tdepth, transmittance)) {
                     w.shadow_t[path] = make_float4(transmittance.x, transmittance.y, transmittance.z, 0.0f);
                     active = false;
                 } else {
                     // past a transparent surface: same shadow ray from the next float
-                    traversal_begin(s, t, st);
+                    traversal_resume(s, t, st, rest.tmin);
                 }
             }
-            const uint32_t idle = static_cast<uint32_t>(__popcll(__ballot(!active)));
-            if (idle == 64u || ((!exhausted || res < res_end) && idle >= refill)) break;
         }
     }
     add_counter(&counters->rays, rays);

@@ -1,0 +1,92 @@
+"""The phased traversal against the oracle where its bookkeeping can go wrong.
+
+Waves that are partly filled, stacks deeper than the LDS ring (entries spill
+to HBM and come back), lanes that enter, leave and skip instances while
+others are inside one, rays with NaN.  Closest hits identical, shadow
+transmittance bit-identical.
+"""
+import sys
+
+import numpy as np
+import pytest
+
+import oracle_binding as ob
+from psycles_amd import abi, scenes
+from psycles_amd.render import RendererBackend
+
+pytestmark = pytest.mark.gpu
+
+
+def heap_of_triangles(count=3000, seed=11):
+    """Large triangles through one ball: no split separates them, so a ray
+    visits most of the tree and its stack grows past the LDS ring."""
+    rng = np.random.RandomState(seed)
+    p = rng.uniform(-1.0, 1.0, (3 * count, 3)).astype(np.float32)
+    t = np.arange(3 * count, dtype=np.uint32).reshape(-1, 3)
+    return scenes.MeshData(p, t, [0])
+
+
+def mixed_scene():
+    """Triangle heaps shared by overlapping instances of different
+    visibility, one single-user mesh and a floor; opaque and part
+    transparent materials."""
+    rng = np.random.RandomState(5)
+    small = heap_of_triangles(40, 3)
+    ball_p, ball_t = scenes.geodesic_icosphere(4)
+    fp, ft = scenes.quad([[-6, -2, -6], [-6, -2, 6], [6, -2, 6], [6, -2, -6]])
+    meshes = [small, scenes.MeshData(ball_p, ball_t, [0]), scenes.MeshData(fp, ft, [1]), heap_of_triangles(60, 4)]
+    materials = [scenes.mix_diffuse_transparent((0.5, 0.6, 0.7), 0.7), scenes.diffuse_material((0.5, 0.5, 0.5))]
+    instances = []
+    for k in range(24):
+        m = scenes.translation(*rng.uniform(-2.5, 2.5, 3)) @ scenes.rotation_y(float(rng.uniform(0, 360)))
+        instances.append(scenes.InstanceData(k % 2, m, material_overrides=[k % 3 == 0],
+                                             visibility=[abi.VIS_ALL, abi.VIS_SHADOW, abi.VIS_ALL & ~abi.VIS_SHADOW][k % 3]))
+    instances += [scenes.InstanceData(2, scenes.identity()), scenes.InstanceData(3, scenes.translation(0.5, 0.0, 0.5))]
+    camera = scenes.CameraData(scenes.translation(0, 0, 6))
+    return scenes.SceneSnapshot(materials, meshes, instances, camera, name="mixed")
+
+
+def heap_scene():
+    camera = scenes.CameraData(scenes.translation(0, 0, 4))
+    return scenes.SceneSnapshot([scenes.mix_diffuse_transparent((0.5, 0.5, 0.5), 0.9)], [heap_of_triangles()],
+                                [scenes.InstanceData(0, scenes.identity())], camera, name="heap")
+
+
+def queries(n, reach, seed, kind):
+    rng = np.random.RandomState(seed)
+    out = []
+    for i in range(n):
+        a, b = rng.uniform(-reach, reach, 3), rng.uniform(-reach, reach, 3)
+        d = (b - a) / np.linalg.norm(b - a)
+        q = {"origin": a, "direction": d, "kind": kind, "tmin": float(rng.choice([0.0, 0.1])),
+             "tmax": float(rng.choice([0.5, 100.0])), "transparent_max": 40}
+        q["visibility"] = abi.VIS_SHADOW if kind == abi.QUERY_SHADOW else int(rng.choice([abi.VIS_ALL, abi.VIS_CAMERA]))
+        if i % 13 == 5:
+            q["direction"] = [0.0, 1.0, 0.0]
+        if i % 17 == 3:
+            q["origin"] = [a[0], float("nan"), a[2]]
+        out.append(q)
+    return out
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1500])
+@pytest.mark.parametrize("name", ["heap", "mixed"])
+def test_queries_match_oracle(name, n):
+    print(f"case: traversal of {name}, {n} queries", flush=True)
+    sys.stdout.flush()
+    snap = heap_scene() if name == "heap" else mixed_scene()
+    backend = RendererBackend(0)
+    dev = backend.compile_scene(snap).scene
+    ora = ob.OracleScene(snap)
+    reach = 1.5 if name == "heap" else 4.0
+    closest = queries(n, reach, 100 + n, abi.QUERY_CLOSEST)
+    for x, y in zip(dev.intersect(closest), ora.intersect(closest)):
+        assert (x.hit, x.object, x.primitive) == (y.hit, y.object, y.primitive)
+        if x.hit:
+            assert np.float32([x.t, x.u, x.v]).tobytes() == np.float32([y.t, y.u, y.v]).tobytes()
+    shadow = queries(n, reach, 200 + n, abi.QUERY_SHADOW)
+    for x, y in zip(dev.intersect(shadow), ora.intersect(shadow)):
+        assert np.float32(x.transmittance).tobytes() == np.float32(y.transmittance).tobytes()
+        assert x.hit == y.hit
+    dev.close()
+    backend.close()
