@@ -90,3 +90,23 @@ def test_queries_match_oracle(name, n):
         assert x.hit == y.hit
     dev.close()
     backend.close()
+
+
+@pytest.mark.parametrize("width,height,spp", [(1, 1, 1), (8, 8, 1), (17, 3, 2), (64, 64, 1), (257, 129, 3), (640, 400, 9)])
+def test_short_queues(width, height, spp):
+    """Queues from one entry to several reservations a wave (4096 waves, 16 to
+    128 entries each): the trace kernel deals them out; film and ray count are
+    those of the one-lane-per-path kernel."""
+    print(f"case: short queues {width}x{height}x{spp}", flush=True)
+    snap = scenes.cornell_lamps()
+    films = []
+    for integrator in (abi.INTEGRATOR_MEGAKERNEL, abi.INTEGRATOR_WAVEFRONT):
+        backend = RendererBackend(0, integrator=integrator, max_samples_per_dispatch=spp)
+        scene = backend.compile_scene(snap).scene
+        session = backend.create_session(scene, scenes.cornell_settings(width, height))
+        session.render_device(0, spp, spp)
+        films.append([a.tobytes() for a in session.read_film()] + [session.stats().rays])
+        session.close()
+        scene.close()
+        backend.close()
+    assert films[0] == films[1]
