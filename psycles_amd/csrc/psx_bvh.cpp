@@ -94,7 +94,10 @@ class BinaryBuilder {
             nodes_[t.node].box = box;
             max_depth_ = std::max(max_depth_, t.depth);
             const uint32_t n = t.end - t.begin;
-            if (n <= leaf_size_) {
+            bool leaf = n <= leaf_size_;
+            for (uint32_t i = t.begin; leaf && n > 1u && i < t.end; ++i)
+                leaf = items_[order_[i]].instance_weight == 0u;
+            if (leaf) {
                 nodes_[t.node].first = t.begin;
                 nodes_[t.node].count = n;
                 continue;
@@ -129,7 +132,7 @@ class BinaryBuilder {
                 const uint32_t id = order_[i];
                 int b = static_cast<int>((centroids_[3 * id + a] - cbox.lo[a]) * scale);
                 b = std::min(std::max(b, 0), kBins - 1);
-                counts[b]++;
+                counts[b] += std::max(1u, items_[id].instance_weight);
                 Box ib;
                 std::memcpy(ib.lo, items_[id].lo, sizeof(ib.lo));
                 std::memcpy(ib.hi, items_[id].hi, sizeof(ib.hi));
@@ -295,7 +298,7 @@ Bvh4 build_bvh4(const std::vector<BuildItem> &items, uint32_t node_base, uint32_
     return out;
 }
 
-QNode4 quantize_node(const Node4 &n, bool tlas) {
+QNode4 quantize_node(const Node4 &n) {
     QNode4 q{};
     const float *lo[3] = {n.lo_x, n.lo_y, n.lo_z};
     const float *hi[3] = {n.hi_x, n.hi_y, n.hi_z};
@@ -341,13 +344,75 @@ QNode4 quantize_node(const Node4 &n, bool tlas) {
         if (c == kEmptySlot)
             q.ref[i] = kEmptySlot;
         else if (c == 0u)
-            q.ref[i] = child | (tlas ? kKindTlas : kKindBlas);
-        else if (tlas)
+            q.ref[i] = child | kKindNode;
+        else if (c == kInstanceSlot)
             q.ref[i] = child | kKindInstance;
         else
             q.ref[i] = kKindLeaf | (child << 3) | (c - 1u);
     }
     return q;
+}
+
+std::vector<QNode4> quantize_nodes(const std::vector<Node4> &nodes) {
+    std::vector<QNode4> out(nodes.size());
+    for (size_t i = 0; i < nodes.size(); ++i) out[i] = quantize_node(nodes[i]);
+    return out;
+}
+
+void transformed_bounds(const std::vector<Node4> &nodes, const std::vector<LeafTri> &tris, uint32_t root,
+                        const float *transform, double lo[3], double hi[3]) {
+    std::vector<uint32_t> stack;
+    for (int side = 0; side < 6; ++side) {
+        const int axis = side >> 1;
+        const double sign = (side & 1) != 0 ? -1.0 : 1.0;
+        const double m[3] = {sign * transform[axis], sign * transform[4 + axis], sign * transform[8 + axis]};
+        double best = -HUGE_VAL, tolerance = 0.0;
+        stack.assign(1, root);
+        while (!stack.empty()) {
+            const Node4 &n = nodes[stack.back()];
+            stack.pop_back();
+            const float *nlo[3] = {n.lo_x, n.lo_y, n.lo_z}, *nhi[3] = {n.hi_x, n.hi_y, n.hi_z};
+            double reach[4];
+            int order[4], k = 0;
+            double widest = 0.0;
+            for (int i = 0; i < 4; ++i) {
+                if (n.count[i] == kEmptySlot) continue;
+                reach[i] = 0.0;
+                double magnitude = 0.0, extent = 0.0;
+                for (int a = 0; a < 3; ++a) {
+                    reach[i] += std::max(m[a] * nlo[a][i], m[a] * nhi[a][i]);
+                    magnitude += std::max(std::fabs(m[a] * nlo[a][i]), std::fabs(m[a] * nhi[a][i]));
+                    extent += std::fabs(m[a] * nhi[a][i] - m[a] * nlo[a][i]);
+                }
+                widest = std::max(widest, 1.0e-4 * extent + 4.0e-5 * magnitude);
+                order[k++] = i;
+            }
+            // a flat mesh has all its boxes, which are padded, reach past
+            // its vertices: what is this near is not searched but allowed for
+            if (tolerance == 0.0) tolerance = widest;
+            // the furthest child is searched first: it is pushed last
+            std::sort(order, order + k, [&](int a, int b) { return reach[a] < reach[b]; });
+            for (int j = 0; j < k; ++j) {
+                const int i = order[j];
+                if (reach[i] <= best + tolerance) continue;
+                if (n.count[i] == 0u) {
+                    stack.push_back(n.child[i]);
+                    continue;
+                }
+                for (uint32_t t = n.child[i]; t < n.child[i] + n.count[i]; ++t) {
+                    const LeafTri &l = tris[t];
+                    best = std::max(best, m[0] * l.p0x + m[1] * l.p0y + m[2] * l.p0z);
+                    best = std::max(best, m[0] * l.p1x + m[1] * l.p1y + m[2] * l.p1z);
+                    best = std::max(best, m[0] * l.p2x + m[1] * l.p2y + m[2] * l.p2z);
+                }
+            }
+        }
+        best += tolerance;
+        if (sign > 0.0)
+            hi[axis] = transform[12 + axis] + best;
+        else
+            lo[axis] = transform[12 + axis] - best;
+    }
 }
 
 }  // namespace psx

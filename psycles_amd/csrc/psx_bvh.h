@@ -11,6 +11,9 @@ namespace psx {
 struct BuildItem {
     float lo[3];
     float hi[3];
+    // an instance makes a leaf of its own and weighs as many triangles as
+    // entering it costs; 0: a triangle
+    uint32_t instance_weight = 0;
 };
 
 struct Bvh4 {
@@ -28,19 +31,17 @@ Bvh4 build_bvh4(const std::vector<BuildItem> &items, uint32_t node_base, uint32_
 
 // The traversal form of a node array: node i becomes QNode4 i with 8-bit
 // outward-rounded child bounds and child references encoded as traversal
-// entries.  `is_tlas(i)` tells whether node i belongs to the instance level
-// (its leaves hold one instance index) or to a mesh level (its leaves hold
-// count triangles from child[i]).
-template <typename IsTlas>
-std::vector<QNode4> quantize_nodes(const std::vector<Node4> &nodes, IsTlas is_tlas);
+// entries.
+std::vector<QNode4> quantize_nodes(const std::vector<Node4> &nodes);
 
-QNode4 quantize_node(const Node4 &n, bool tlas);
+QNode4 quantize_node(const Node4 &n);
 
-template <typename IsTlas>
-std::vector<QNode4> quantize_nodes(const std::vector<Node4> &nodes, IsTlas is_tlas) {
-    std::vector<QNode4> out(nodes.size());
-    for (size_t i = 0; i < nodes.size(); ++i) out[i] = quantize_node(nodes[i], is_tlas(static_cast<uint32_t>(i)));
-    return out;
-}
+// Bounds of the triangles under `root` (leaves hold triangles only) after the
+// affine map `transform` (column-major 4x4), in double precision: six support
+// searches that descend only where a node's box reaches past the best vertex
+// so far.  A box of eight transformed corners is up to sqrt(3) times as wide
+// for a rotated instance.
+void transformed_bounds(const std::vector<Node4> &nodes, const std::vector<LeafTri> &tris, uint32_t root,
+                        const float *transform, double lo[3], double hi[3]);
 
 }  // namespace psx

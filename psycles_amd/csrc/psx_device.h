@@ -32,10 +32,10 @@ namespace psx {
 
 // 4-wide BVH node, one 128-byte line.  Child boxes are stored structure-of-
 // arrays so one node fetch feeds four slab tests.  count[i]:
-//   0            inner child, child[i] = node index
-//   1..          leaf: BLAS nodes hold count[i] triangles starting at
-//                child[i]; TLAS nodes hold one instance, child[i] = instance
-//   kEmptySlot   unused slot
+//   0              inner child, child[i] = node index
+//   1..            leaf of count[i] triangles starting at child[i]
+//   kInstanceSlot  an instance, child[i] = instance (world tree only)
+//   kEmptySlot     unused slot
 struct alignas(16) Node4 {
     float lo_x[4], hi_x[4];
     float lo_y[4], hi_y[4];
@@ -45,12 +45,12 @@ struct alignas(16) Node4 {
 };
 static_assert(sizeof(Node4) == 128, "Node4 must be one 128-byte line");
 constexpr uint32_t kEmptySlot = 0xffffffffu;
+constexpr uint32_t kInstanceSlot = 0xfffffffeu;
 
 // Traversal entries (stack entries and quantised child references) carry
 // their kind in the two top bits.
 constexpr uint32_t kKindMask = 0xc0000000u;
-constexpr uint32_t kKindBlas = 0x00000000u;      // BLAS inner node index
-constexpr uint32_t kKindTlas = 0x40000000u;      // TLAS inner node index
+constexpr uint32_t kKindNode = 0x00000000u;      // inner node index
 constexpr uint32_t kKindLeaf = 0x80000000u;      // first triangle << 3 | (count - 1)
 constexpr uint32_t kKindInstance = 0xc0000000u;  // instance index
 
@@ -72,13 +72,25 @@ static_assert(sizeof(QNode4) == 64, "QNode4 must be 64 bytes");
 
 // Leaf triangle in intersection space (object space for shared meshes, final
 // world space for single-user meshes).  p0.w carries the local primitive
-// index as raw bits.
+// index as raw bits.  A triangle of the world tree carries what an instance
+// entry would have set: `owner` is its instance and visibility, `prim_offset`
+// its mesh's Cycles primitive offset; in a mesh's own tree `owner` is kNone
+// and `prim_offset` 0.
 struct alignas(16) LeafTri {
-    float p0x, p0y, p0z, prim_bits;
-    float p1x, p1y, p1z, pad1;
-    float p2x, p2y, p2z, pad2;
+    float p0x, p0y, p0z;
+    uint32_t prim;
+    float p1x, p1y, p1z;
+    uint32_t owner;
+    float p2x, p2y, p2z;
+    uint32_t prim_offset;
 };
 static_assert(sizeof(LeafTri) == 48, "LeafTri must be 48 bytes");
+
+// LeafTri::owner: instance in the low bits, then the six visibility bits and
+// one for a mask of all ones.  Instances that do not fit (a larger index, or
+// other bits in the mask) keep a tree of their own.
+constexpr uint32_t kOwnerBits = 25u;
+constexpr uint32_t kOwnerAnyVisibility = 0x40u;
 
 // Affine transform stored column-major without the constant last row:
 // m[0..2] column 0, m[3..5] column 1, m[6..8] column 2, m[9..11] translation.

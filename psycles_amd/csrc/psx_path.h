@@ -460,7 +460,8 @@ struct Traversal {
     float best_t;       // tmax until a hit is found
     uint32_t cur;       // next entry, or kEmptySlot
     uint32_t leaf;      // leaf set aside, or kEmptySlot
-    uint32_t inst_index, inst_prim_offset;
+    uint32_t inst_index;  // kNone in the world
+    uint32_t inst_prim_offset;
     // stack level at which the current instance was entered, 0 in the world,
     // kStale when the stack is back in the world and o and d still an instance's
     int base;
@@ -502,14 +503,15 @@ __device__ __forceinline__ void traversal_start(const SceneView &s, Traversal &t
     t.lower = tmin > 0.0f ? tmin * 0.99999f : tmin - 1.0e-30f;
     t.best_t = tmax;
     st.set_word(kColdHit, kNone);
-    t.inst_index = t.inst_prim_offset = 0u;
+    t.inst_index = kNone;
+    t.inst_prim_offset = 0u;
     t.stop = t.opaque = false;
     traversal_space(t, o, d);
     traversal_idle(t, st);
     // a NaN anywhere in the ray fails every triangle test: nothing to search
     const bool nan = __builtin_isunordered(o.x, d.x) || __builtin_isunordered(o.y, d.y) ||
                      __builtin_isunordered(o.z, d.z) || __builtin_isunordered(tmin, tmax);
-    if (s.has_tlas && !nan) t.cur = s.tlas_root | kKindTlas;
+    if (s.has_tlas && !nan) t.cur = s.tlas_root;
 }
 
 __device__ __forceinline__ void traversal_begin(const SceneView &s, Traversal &t, Stack &st, const Ray &ray,
@@ -619,8 +621,11 @@ __device__ __forceinline__ void traversal_leaf(const SceneView &s, Traversal &t,
                              V(__uint_as_float(r1.x), __uint_as_float(r1.y), __uint_as_float(r1.z)),
                              V(__uint_as_float(r2.x), __uint_as_float(r2.y), __uint_as_float(r2.z)), c);
     if (!ok) return;
-    const uint32_t prim = r0.w, inst = t.inst_index;
-    const uint32_t cprim = t.inst_prim_offset + prim;
+    const bool world = t.inst_index == kNone;
+    const uint32_t prim = r0.w, owner = r1.w, mask = owner >> kOwnerBits, seen = st.word(kColdVisibility);
+    if (world && (mask & seen & 0x3fu) == 0u && ((mask & kOwnerAnyVisibility) == 0u || seen == 0u)) return;
+    const uint32_t inst = world ? owner & ((1u << kOwnerBits) - 1u) : t.inst_index;
+    const uint32_t cprim = t.inst_prim_offset + r2.w + prim;
     const bool excluded = (inst == st.word(kColdSource) && cprim == st.word(kColdSource + 1u)) ||
                           (inst == st.word(kColdLight) && cprim == st.word(kColdLight + 1u));
     // at the best distance so far the greatest (object, primitive) wins
@@ -635,7 +640,7 @@ __device__ __forceinline__ void traversal_leaf(const SceneView &s, Traversal &t,
     st.set_word(kColdHit, inst);
     st.set_word(kColdHit + 1u, prim);
     st.set_word(kColdHit + 2u, cprim);
-    if (ANYHIT && t.stop) {
+    if (ANYHIT && (world ? s.instance_opaque[inst] != 0u : t.stop)) {
         // any opaque candidate in [tmin, tmax] zeroes the shadow
         t.opaque = true;
         traversal_idle(t, st);
@@ -647,7 +652,10 @@ template <bool ANYHIT>
 __device__ __forceinline__ void traversal_change_space(const SceneView &s, Traversal &t, Stack &st) {
     f3 o = st.vec(kColdOrigin), d = st.vec(kColdDirection);
     int base = 0;
-    if (t.cur >= kKindInstance) {
+    if (t.cur < kKindInstance) {
+        t.inst_index = kNone;
+        t.inst_prim_offset = 0u;
+    } else {
         const uint32_t index = t.cur & ~kKindMask;
         const Instance &inst = s.instances[index];
         const Affine w2o = inst.w2o;
@@ -655,7 +663,7 @@ __device__ __forceinline__ void traversal_change_space(const SceneView &s, Trave
         // do there, which is the state of a lane that came back from it
         const bool visible = (inst.visibility & st.word(kColdVisibility)) != 0u;
         const bool applied = inst.applied != 0u;
-        t.cur = visible ? inst.blas_root | kKindBlas : kEmptySlot;
+        t.cur = visible ? inst.blas_root : kEmptySlot;
         base = visible ? st.sp : kStale;
         t.inst_index = index;
         t.inst_prim_offset = inst.prim_offset;

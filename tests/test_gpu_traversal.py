@@ -2,7 +2,8 @@
 
 Waves that are partly filled, stacks deeper than the LDS ring (entries spill
 to HBM and come back), lanes that enter, leave and skip instances while
-others are inside one, rays with NaN.  Closest hits identical, shadow
+others are inside one, single-user meshes in and outside the world tree,
+rays with NaN.  Closest hits identical, shadow
 transmittance bit-identical.
 """
 import sys
@@ -34,14 +35,19 @@ def mixed_scene():
     small = heap_of_triangles(40, 3)
     ball_p, ball_t = scenes.geodesic_icosphere(4)
     fp, ft = scenes.quad([[-6, -2, -6], [-6, -2, 6], [6, -2, 6], [6, -2, -6]])
-    meshes = [small, scenes.MeshData(ball_p, ball_t, [0]), scenes.MeshData(fp, ft, [1]), heap_of_triangles(60, 4)]
+    meshes = [small, scenes.MeshData(ball_p, ball_t, [0]), scenes.MeshData(fp, ft, [1]), heap_of_triangles(60, 4),
+              heap_of_triangles(50, 6)]
     materials = [scenes.mix_diffuse_transparent((0.5, 0.6, 0.7), 0.7), scenes.diffuse_material((0.5, 0.5, 0.5))]
     instances = []
     for k in range(24):
         m = scenes.translation(*rng.uniform(-2.5, 2.5, 3)) @ scenes.rotation_y(float(rng.uniform(0, 360)))
         instances.append(scenes.InstanceData(k % 2, m, material_overrides=[k % 3 == 0],
                                              visibility=[abi.VIS_ALL, abi.VIS_SHADOW, abi.VIS_ALL & ~abi.VIS_SHADOW][k % 3]))
-    instances += [scenes.InstanceData(2, scenes.identity()), scenes.InstanceData(3, scenes.translation(0.5, 0.0, 0.5))]
+    # single-user meshes: with a plain mask and with all bits set they join
+    # the world tree, with other bits they keep a tree of their own
+    instances += [scenes.InstanceData(2, scenes.identity()),
+                  scenes.InstanceData(3, scenes.translation(0.5, 0.0, 0.5), visibility=0xffffffff),
+                  scenes.InstanceData(4, scenes.translation(-0.5, 0.3, 0.0), visibility=0x50)]
     camera = scenes.CameraData(scenes.translation(0, 0, 6))
     return scenes.SceneSnapshot(materials, meshes, instances, camera, name="mixed")
 
@@ -52,6 +58,24 @@ def heap_scene():
                                 [scenes.InstanceData(0, scenes.identity())], camera, name="heap")
 
 
+def nested_scales():
+    """Three meshes of triangles whose sizes fall by powers of two, each mesh
+    every third power.  One tree over all of them has about 22 levels of four,
+    too many for the traversal stack, so each mesh keeps its own (about 12)."""
+    meshes = []
+    for m in range(3):
+        sizes = 2.0 ** (60.0 - np.arange(m, 131, 3))
+        corners = np.array([[1.0, 1.0, 1.0], [1.3, 1.0, 1.15], [1.1, 1.3, 1.3]])
+        p = (sizes[:, None, None] * corners[None]).reshape(-1, 3).astype(np.float32)
+        meshes.append(scenes.MeshData(p, np.arange(len(p), dtype=np.uint32).reshape(-1, 3), [0]))
+    return scenes.SceneSnapshot([scenes.diffuse_material((0.5, 0.5, 0.5))], meshes,
+                                [scenes.InstanceData(m, scenes.identity()) for m in range(3)],
+                                scenes.CameraData(scenes.translation(0, 0, 4)), name="scales")
+
+
+SCENES = {"heap": (heap_scene, 1.5), "mixed": (mixed_scene, 4.0), "scales": (nested_scales, 2.0)}
+
+
 def queries(n, reach, seed, kind):
     rng = np.random.RandomState(seed)
     out = []
@@ -60,9 +84,13 @@ def queries(n, reach, seed, kind):
         d = (b - a) / np.linalg.norm(b - a)
         q = {"origin": a, "direction": d, "kind": kind, "tmin": float(rng.choice([0.0, 0.1])),
              "tmax": float(rng.choice([0.5, 100.0])), "transparent_max": 40}
-        q["visibility"] = abi.VIS_SHADOW if kind == abi.QUERY_SHADOW else int(rng.choice([abi.VIS_ALL, abi.VIS_CAMERA]))
+        q["visibility"] = (abi.VIS_SHADOW if kind == abi.QUERY_SHADOW
+                           else int(rng.choice([abi.VIS_ALL, abi.VIS_CAMERA, 0x40])))
         if i % 13 == 5:
             q["direction"] = [0.0, 1.0, 0.0]
+        if i % 3 == 1:  # a ray near the diagonal, where the scales are nested
+            b = np.ones(3) * rng.uniform(0.9, 1.5) + rng.uniform(0.0, 0.3, 3)
+            q["origin"], q["direction"] = b * 2.0 ** rng.randint(-8, 8), -b / np.linalg.norm(b) + rng.uniform(-0.1, 0.1, 3)
         if i % 17 == 3:
             q["origin"] = [a[0], float("nan"), a[2]]
         out.append(q)
@@ -70,15 +98,15 @@ def queries(n, reach, seed, kind):
 
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 1500])
-@pytest.mark.parametrize("name", ["heap", "mixed"])
+@pytest.mark.parametrize("name", sorted(SCENES))
 def test_queries_match_oracle(name, n):
     print(f"case: traversal of {name}, {n} queries", flush=True)
     sys.stdout.flush()
-    snap = heap_scene() if name == "heap" else mixed_scene()
+    make, reach = SCENES[name]
+    snap = make()
     backend = RendererBackend(0)
     dev = backend.compile_scene(snap).scene
     ora = ob.OracleScene(snap)
-    reach = 1.5 if name == "heap" else 4.0
     closest = queries(n, reach, 100 + n, abi.QUERY_CLOSEST)
     for x, y in zip(dev.intersect(closest), ora.intersect(closest)):
         assert (x.hit, x.object, x.primitive) == (y.hit, y.object, y.primitive)
