@@ -334,6 +334,20 @@ struct FilmView {
     float *light;      // kLightPasses float4 per pixel, or null
 };
 
+// How a requested pass is made from the film's sums.
+enum class PassRule : uint32_t {
+    kCombined,      // exposed mean and alpha
+    kNormal,        // mean
+    kAlbedo,        // mean
+    kSampleCount,   // the count in every channel
+    kLight,         // exposed mean of a light-pass sum
+    kLightColor,    // mean of a light-pass colour
+    kOverAlbedo,    // light-pass sum over the albedo sum, exposed
+    kOverGlossy,    // light-pass sum over the glossy colour sum, exposed
+    kOverTransmission,  // the same over the transmission colour sum
+    kZero           // a light pass of a film without light sums
+};
+
 struct Counters {
     unsigned long long rays;
     unsigned long long nodes;

@@ -32,6 +32,7 @@
 #include "psx_device.h"
 #include "psx_light_tree.h"
 #include "psx_rtc.h"
+#include "psx_sobol.h"
 
 namespace psx {
 
@@ -72,6 +73,12 @@ hipError_t launch_wavefront(const SceneView &s, const KernelParams &k, const flo
                             const uint32_t *first_at, Counters *counters, bool count_nodes, uint32_t *spill,
                             hipEvent_t *events, const GeneratedShade *generated, hipStream_t stream);
 hipError_t launch_store_word(uint32_t *dst, uint32_t value, hipStream_t stream);
+// psx_passes.hip
+hipError_t launch_sobol_table(float4 *table, uint32_t size, hipStream_t stream);
+hipError_t launch_count_check(const uint32_t *counts, uint64_t pixels, uint32_t expected, uint32_t *wrong,
+                              hipStream_t stream);
+hipError_t launch_pass(const FilmView &film, uint64_t pixels, PassRule rule, uint32_t slot, uint32_t channels,
+                       float exposure, float *out, hipStream_t stream);
 uint32_t shade_variant(const SceneView &s, bool light_passes);
 
 namespace {
@@ -198,32 +205,6 @@ void transpose4(const float *a, float *r) {
 // ---------------------------------------------------------------------------
 // tabulated Sobol LUT (src/sampling/tabulated_sobol.cpp:24-199)
 // ---------------------------------------------------------------------------
-const uint32_t kSobolXors[4][32] = {
-    {0u},
-    {0x00000000u, 0x00000001u, 0x00000001u, 0x00000007u, 0x00000001u, 0x00000013u, 0x00000015u, 0x0000007fu,
-     0x00000001u, 0x00000103u, 0x00000105u, 0x0000070fu, 0x00000111u, 0x00001333u, 0x00001555u, 0x00007fffu,
-     0x00000001u, 0x00010003u, 0x00010005u, 0x0007000fu, 0x00010011u, 0x00130033u, 0x00150055u, 0x007f00ffu,
-     0x00010101u, 0x01030303u, 0x01050505u, 0x070f0f0fu, 0x01111111u, 0x13333333u, 0x15555555u, 0x7fffffffu},
-    {0x00000000u, 0x00000001u, 0x00000003u, 0x00000001u, 0x00000005u, 0x0000001fu, 0x0000002bu, 0x0000003du,
-     0x00000011u, 0x00000133u, 0x00000377u, 0x00000199u, 0x00000445u, 0x00001ccfu, 0x00002ddbu, 0x0000366du,
-     0x00000101u, 0x00010303u, 0x00030707u, 0x00010909u, 0x00051515u, 0x001f3f3fu, 0x002b6b6bu, 0x003dbdbdu,
-     0x00101011u, 0x01303033u, 0x03707077u, 0x01909099u, 0x04515145u, 0x1cf3f3cfu, 0x2db6b6dbu, 0x36dbdb6du},
-    {0x00000000u, 0x00000001u, 0x00000000u, 0x00000003u, 0x0000000du, 0x0000000cu, 0x00000005u, 0x0000004fu,
-     0x00000014u, 0x000000e7u, 0x00000329u, 0x0000039cu, 0x00000011u, 0x00001033u, 0x00000044u, 0x000030bbu,
-     0x0000d1cdu, 0x0000c2ecu, 0x00005415u, 0x0004fc3fu, 0x00015054u, 0x000e5c97u, 0x0032e5b9u, 0x0039725cu,
-     0x00000101u, 0x01000303u, 0x00000404u, 0x03000b0bu, 0x0d001d1du, 0x0c002c2cu, 0x05004545u, 0x4f00cfcfu}};
-
-uint32_t hash_hp(uint32_t v) {
-    v ^= v >> 16u;
-    v *= 0x21f0aaadu;
-    v ^= v >> 15u;
-    v *= 0xd35a2d97u;
-    v ^= v >> 15u;
-    return v ^ 0xe6fe3bebu;
-}
-
-float hash_hp_float(uint32_t v) { return static_cast<float>(hash_hp(v)) * (1.0f / 4294967808.0f); }
-
 uint32_t sequence_size_for(uint32_t samples) {
     const uint32_t c = std::min(std::max(samples, 1u), 8192u);
     uint32_t u = 1u;
@@ -235,10 +216,7 @@ std::vector<float> sobol_table(uint32_t size) {
     std::vector<float> t(static_cast<size_t>(size) * 256u * 4u);
     for (uint32_t pattern = 0; pattern < 256u; ++pattern) {
         float *p = t.data() + static_cast<size_t>(pattern) * size * 4u;
-        // hash_hp_seeded_uint(pattern, 0x44605a73): the seed is pre-mixed
-        uint32_t seed = 0x44605a73u;
-        seed ^= seed << 19u;
-        uint32_t rng = hash_hp(pattern ^ seed);
+        uint32_t rng = sobol_pattern_seed(pattern);
         for (int c = 0; c < 4; ++c) p[c] = hash_hp_float(rng++);
         uint32_t log_n = 0;
         for (uint32_t n = 1; n < size; ++log_n, n *= 2u) {
@@ -565,9 +543,82 @@ uint64_t structure_signature(const HostMaterial &m) {
 // ---------------------------------------------------------------------------
 // handles
 // ---------------------------------------------------------------------------
+// What a pass download needs: a stream, device memory for the pass pixels and
+// pinned host memory that the sink reads.
+struct PassStaging {
+    hipStream_t stream = nullptr;
+    std::vector<hipEvent_t> events;
+    DeviceBuffer device;
+    void *pinned = nullptr;
+    size_t pinned_bytes = 0;
+
+    PassStaging() = default;
+    PassStaging(const PassStaging &) = delete;
+    PassStaging &operator=(const PassStaging &) = delete;
+    ~PassStaging() {
+        if (stream) (void)hipStreamSynchronize(stream);
+        for (hipEvent_t e : events) (void)hipEventDestroy(e);
+        if (pinned) (void)hipHostFree(pinned);
+        if (stream) (void)hipStreamDestroy(stream);
+    }
+    void reserve(size_t bytes, size_t event_count) {
+        if (!stream) hip_check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+        while (events.size() < event_count) {
+            hipEvent_t e = nullptr;
+            hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            events.push_back(e);
+        }
+        if (device.bytes() < bytes) device.allocate(bytes);
+        if (pinned_bytes < bytes) {
+            if (pinned) (void)hipHostFree(pinned);
+            pinned = nullptr;
+            pinned_bytes = 0;
+            hip_check(hipHostMalloc(&pinned, bytes, hipHostMallocDefault));
+            pinned_bytes = bytes;
+        }
+    }
+};
+
+// Stagings between downloads: pinning 90 MB takes longer than filling it, so
+// a backend keeps up to two of at most kStagingBytes each; concurrent
+// downloads beyond that make their own and free them.
+constexpr size_t kStagingBytes = 256u << 20;
+struct StagingPool {
+    std::mutex mutex;
+    std::vector<std::unique_ptr<PassStaging>> idle;
+};
+
+class StagingLease {
+  public:
+    explicit StagingLease(StagingPool &pool) : pool_(pool) {
+        std::lock_guard<std::mutex> lock(pool_.mutex);
+        if (!pool_.idle.empty()) {
+            held_ = std::move(pool_.idle.back());
+            pool_.idle.pop_back();
+        } else {
+            held_ = std::make_unique<PassStaging>();
+        }
+    }
+    ~StagingLease() {
+        // whatever an error left in flight ends before the memory is reused
+        if (held_->stream) (void)hipStreamSynchronize(held_->stream);
+        if (held_->pinned_bytes > kStagingBytes) return;
+        std::lock_guard<std::mutex> lock(pool_.mutex);
+        if (pool_.idle.size() < 2u) pool_.idle.push_back(std::move(held_));
+    }
+    StagingLease(const StagingLease &) = delete;
+    StagingLease &operator=(const StagingLease &) = delete;
+    PassStaging &operator*() { return *held_; }
+
+  private:
+    StagingPool &pool_;
+    std::unique_ptr<PassStaging> held_;
+};
+
 struct Backend {
     int device = 0;
     psx_backend_options options{};
+    StagingPool staging;  // pass downloads
     ProgramCache programs;  // generated shade kernels (PSX_BACKEND_GENERATED_PROGRAMS)
     // Held while a session captures a dispatch graph, and by the render
     // server's worker while it makes device calls: a synchronous upload
@@ -1124,7 +1175,9 @@ struct Session {
     bool light_passes = false;
     WavefrontState wavefront;
     uint32_t wavefront_iterations = 0;
-    uint32_t sobol_size = 0;
+    uint32_t sobol_size = 0;  // the table depends on nothing else
+    uint32_t filter_kind = 0;  // what `filter` was made for
+    float filter_width = 0.0f;
     uint32_t total_aa = 0;
     uint32_t rendered = 0;
     std::atomic<bool> cancelled{false};
@@ -1168,37 +1221,6 @@ int light_pass_slot(uint32_t kind) {
     case PSX_PASS_TRANSMISSION_COLOR: return kLpTransmissionColor;
     default: return -1;
     }
-}
-
-// Cycles' safe_divide_even_color (src/luisa/path_tracer_common.cpp:516-548):
-// channels with a zero denominator take the other channels' quotients.
-void divide_even_color(const float *n, const float *d, float *out) {
-    float x = d[0] != 0.0f ? n[0] / d[0] : 0.0f;
-    float y = d[1] != 0.0f ? n[1] / d[1] : 0.0f;
-    float z = d[2] != 0.0f ? n[2] / d[2] : 0.0f;
-    if (d[0] == 0.0f) {
-        if (d[1] == 0.0f) {
-            x = z;
-            y = z;
-        } else if (d[2] == 0.0f) {
-            x = y;
-            z = y;
-        } else {
-            x = 0.5f * (y + z);
-        }
-    } else if (d[1] == 0.0f) {
-        if (d[2] == 0.0f) {
-            y = x;
-            z = x;
-        } else {
-            y = 0.5f * (x + z);
-        }
-    } else if (d[2] == 0.0f) {
-        z = 0.5f * (x + y);
-    }
-    out[0] = x;
-    out[1] = y;
-    out[2] = z;
 }
 
 // Kernel parameters of one render request: the host part of
@@ -1292,18 +1314,22 @@ void initialize_session(Session &s, const psx_render_settings &rs) {
     } else {
         s.light.reset();
     }
-    s.filter.upload(pixel_filter_table(rs.pixel_filter, rs.filter_width));
+    if (!s.filter.bytes() || s.filter_kind != rs.pixel_filter || s.filter_width != rs.filter_width) {
+        s.filter.upload(pixel_filter_table(rs.pixel_filter, rs.filter_width));
+        s.filter_kind = rs.pixel_filter;
+        s.filter_width = rs.filter_width;
+    }
     if (!s.counters.bytes()) s.counters.allocate(sizeof(Counters));
     s.total_aa = 0;
     s.rendered = 0;
-    s.sobol_size = 0;
 }
 
 // prepare_sobol_table (src/luisa/path_tracer_session.cpp:41-69)
 void prepare_sobol(Session &s, uint32_t total) {
     const uint32_t size = sequence_size_for(total);
     if (size != s.sobol_size) {
-        s.sobol.upload(sobol_table(size));
+        s.sobol.allocate(static_cast<size_t>(size) * kSobolPatterns * sizeof(float4));
+        hip_check(launch_sobol_table(s.sobol.as<float4>(), size, s.stream));
         s.sobol_size = size;
     }
     s.params.sequence_size = size;
@@ -1501,77 +1527,105 @@ int dispatch_samples(Session &s, uint32_t first, uint32_t count) {
     return PSX_OK;
 }
 
-// write_passes (src/luisa/path_tracer_session.cpp:71-254)
-int write_passes(Session &s, const psx_sink *sink) {
+// The rule that makes a pass of `kind`, and its light-pass slot.
+PassRule pass_rule(uint32_t kind, bool light, uint32_t &slot) {
+    slot = 0u;
+    switch (kind) {
+    case PSX_PASS_COMBINED:
+        return PassRule::kCombined;
+    case PSX_PASS_NORMAL:
+    case PSX_PASS_DENOISING_NORMAL:
+        return PassRule::kNormal;
+    case PSX_PASS_ALBEDO:
+    case PSX_PASS_DENOISING_ALBEDO:
+        return PassRule::kAlbedo;
+    case PSX_PASS_SAMPLE_COUNT:
+        return PassRule::kSampleCount;
+    default:
+        break;
+    }
+    const int s = light_pass_slot(kind);
+    if (s < 0 || !light) return PassRule::kZero;
+    slot = static_cast<uint32_t>(s);
+    switch (slot) {
+    case kLpDiffuseDirect:
+    case kLpDiffuseIndirect:
+        return PassRule::kOverAlbedo;
+    case kLpGlossyDirect:
+    case kLpGlossyIndirect:
+        return PassRule::kOverGlossy;
+    case kLpTransmissionDirect:
+    case kLpTransmissionIndirect:
+        return PassRule::kOverTransmission;
+    case kLpGlossyColor:
+    case kLpTransmissionColor:
+        return PassRule::kLightColor;
+    default:
+        return PassRule::kLight;
+    }
+}
+
+// write_passes (src/luisa/path_tracer_session.cpp:71-254).  Kernels make the
+// pass pixels, and copies into pinned memory run ahead of the sink's calls.
+// The film of a finished render does not change, so the work goes on the
+// staging's own stream.
+int write_passes(Backend &backend, Session &s, const psx_sink *sink) {
     const size_t n = static_cast<size_t>(s.window_w) * s.window_h;
-    std::vector<float> combined(n * 4u), normal(n * 4u), albedo(n * 4u);
-    std::vector<uint32_t> counts(n);
-    hip_check(hipMemcpy(combined.data(), s.combined.as<void>(), n * 16u, hipMemcpyDeviceToHost));
-    hip_check(hipMemcpy(normal.data(), s.normal.as<void>(), n * 16u, hipMemcpyDeviceToHost));
-    hip_check(hipMemcpy(albedo.data(), s.albedo.as<void>(), n * 16u, hipMemcpyDeviceToHost));
-    hip_check(hipMemcpy(counts.data(), s.sample_count.as<void>(), n * 4u, hipMemcpyDeviceToHost));
-    std::vector<float> light;
-    if (s.light_passes) {
-        light.resize(n * kLightPasses * 4u);
-        hip_check(hipMemcpy(light.data(), s.light.as<void>(), n * kLightPasses * 16u, hipMemcpyDeviceToHost));
-    }
-    for (size_t i = 0; i < n; ++i)
-        if (counts[i] != s.rendered) return PSX_ERROR_INCOMPLETE;
-    if (sink && sink->begin) sink->begin(sink->user, &s.settings);
+    const FilmView film{s.combined.as<float>(), s.normal.as<float>(), s.albedo.as<float>(),
+                        s.sample_count.as<uint32_t>(), s.light_passes ? s.light.as<float>() : nullptr};
     const float exposure = s.settings.integrator.film_exposure;
-    std::vector<float> pixels;
-    for (uint32_t p = 0; p < s.passes.size(); ++p) {
-        const uint32_t kind = s.passes[p];
-        const uint32_t channels = std::max(1u, std::min(s.pass_channels[p], 4u));
-        pixels.assign(n * channels, 0.0f);
-        for (size_t i = 0; i < n; ++i) {
-            const float den = static_cast<float>(std::max(counts[i], 1u));
-            float v[4] = {0, 0, 0, 0};
-            switch (kind) {
-            case PSX_PASS_COMBINED:
-                for (int c = 0; c < 3; ++c) v[c] = combined[4 * i + c] * (exposure / den);
-                v[3] = std::min(std::max(1.0f - combined[4 * i + 3] / den, 0.0f), 1.0f);
-                break;
-            case PSX_PASS_NORMAL:
-            case PSX_PASS_DENOISING_NORMAL:
-                for (int c = 0; c < 4; ++c) v[c] = normal[4 * i + c] / den;
-                break;
-            case PSX_PASS_ALBEDO:
-            case PSX_PASS_DENOISING_ALBEDO:
-                for (int c = 0; c < 4; ++c) v[c] = albedo[4 * i + c] / den;
-                break;
-            case PSX_PASS_SAMPLE_COUNT:
-                v[0] = v[1] = v[2] = v[3] = static_cast<float>(counts[i]);
-                break;
-            default: {
-                // light passes (src/luisa/path_tracer_session.cpp:150-230)
-                const int slot = light_pass_slot(kind);
-                if (slot < 0 || light.empty()) break;
-                const float *lp = light.data() + i * kLightPasses * 4u;
-                const float *sum = lp + 4 * slot;
-                const float *color = nullptr;
-                if (slot == kLpDiffuseDirect || slot == kLpDiffuseIndirect) color = albedo.data() + 4 * i;
-                if (slot == kLpGlossyDirect || slot == kLpGlossyIndirect) color = lp + 4 * kLpGlossyColor;
-                if (slot == kLpTransmissionDirect || slot == kLpTransmissionIndirect)
-                    color = lp + 4 * kLpTransmissionColor;
-                if (color) {
-                    divide_even_color(sum, color, v);
-                    for (int c = 0; c < 3; ++c) v[c] *= exposure;
-                    v[3] = 1.0f;
-                } else if (slot == kLpGlossyColor || slot == kLpTransmissionColor) {
-                    for (int c = 0; c < 4; ++c) v[c] = sum[c] / den;
-                } else {
-                    for (int c = 0; c < 4; ++c) v[c] = sum[c] * (exposure / den);
-                }
-                break;
-            }
-            }
-            for (uint32_t c = 0; c < channels; ++c) pixels[i * channels + c] = v[std::min(c, 3u)];
+    const bool write = sink && sink->write;
+    StagingLease lease(backend.staging);
+    PassStaging &stage = *lease;
+    constexpr size_t kHead = 256u;  // the count check's word
+    auto pass_bytes = [&](size_t p) {
+        return n * std::max(1u, std::min(s.pass_channels[p], 4u)) * sizeof(float);
+    };
+    size_t done = 0u;
+    bool checked = false;
+    do {
+        // as many passes as the staging holds, at least one
+        size_t end = done, bytes = kHead;
+        while (write && end < s.passes.size() && (end == done || bytes + pass_bytes(end) <= kStagingBytes))
+            bytes += pass_bytes(end++);
+        stage.reserve(bytes, end - done + 1u);
+        if (!checked) {
+            hip_check(launch_count_check(film.sample_count, n, s.rendered, stage.device.as<uint32_t>(), stage.stream));
+            hip_check(hipMemcpyAsync(stage.pinned, stage.device.as<void>(), sizeof(uint32_t), hipMemcpyDeviceToHost,
+                                     stage.stream));
+            hip_check(hipEventRecord(stage.events[0], stage.stream));
         }
-        if (sink && sink->write)
-            sink->write(sink->user, kind, channels, s.settings.window_x, s.settings.window_y, s.window_w, s.window_h,
-                        s.settings.width, s.settings.height, pixels.data());
-    }
+        size_t at = kHead;
+        for (size_t p = done; p < end; ++p) {
+            uint32_t slot;
+            const PassRule rule = pass_rule(s.passes[p], s.light_passes, slot);
+            char *out = stage.device.as<char>() + at;
+            hip_check(launch_pass(film, n, rule, slot, std::max(1u, std::min(s.pass_channels[p], 4u)), exposure,
+                                  reinterpret_cast<float *>(out), stage.stream));
+            hip_check(hipMemcpyAsync(static_cast<char *>(stage.pinned) + at, out, pass_bytes(p),
+                                     hipMemcpyDeviceToHost, stage.stream));
+            hip_check(hipEventRecord(stage.events[p - done + 1u], stage.stream));
+            at += pass_bytes(p);
+        }
+        if (!checked) {
+            hip_check(hipEventSynchronize(stage.events[0]));
+            checked = true;
+            if (*static_cast<const uint32_t *>(stage.pinned) != 0u) {
+                hip_check(hipStreamSynchronize(stage.stream));
+                return PSX_ERROR_INCOMPLETE;
+            }
+            if (sink && sink->begin) sink->begin(sink->user, &s.settings);
+        }
+        at = kHead;
+        for (size_t p = done; p < end; ++p) {
+            hip_check(hipEventSynchronize(stage.events[p - done + 1u]));
+            sink->write(sink->user, s.passes[p], std::max(1u, std::min(s.pass_channels[p], 4u)), s.settings.window_x,
+                        s.settings.window_y, s.window_w, s.window_h, s.settings.width, s.settings.height,
+                        reinterpret_cast<const float *>(static_cast<const char *>(stage.pinned) + at));
+            at += pass_bytes(p);
+        }
+        done = end;
+    } while (write && done < s.passes.size());
     if (sink && sink->end) sink->end(sink->user, s.cancelled.load() ? 1 : 0);
     return PSX_OK;
 }
@@ -3001,7 +3055,7 @@ int psx_session_render(psx_session *handle, uint32_t first, uint32_t count, uint
         const int d = dispatch_samples(*s, first + offset, count);
         if (d != PSX_OK) return d;
         if (s->cancelled.load()) return static_cast<int>(PSX_ERROR_CANCELLED);
-        return write_passes(*s, sink);
+        return write_passes(*s->scene->backend, *s, sink);
     });
 }
 
@@ -3659,7 +3713,7 @@ int psx_server_write_passes(psx_server *server, uint64_t id, const psx_sink *sin
     }
     return guarded([&] {
         hip_check(hipSetDevice(server->backend->device));
-        return write_passes(r->film, sink);
+        return write_passes(*server->backend, r->film, sink);
     });
 }
 
