@@ -356,8 +356,8 @@ struct Counters {
 };
 
 // ---------------------------------------------------------------------------
-// wavefront integrator: per-path state in HBM, structure of arrays indexed by
-// path = sample_in_batch * padded_pixels + tile * 64 + lane (tiles of 64
+// wavefront integrator: per-path state in HBM, indexed by path =
+// sample_in_batch * padded_pixels + tile * 64 + lane (tiles of 64
 // pixels, 8x8 unless the view's tile_shift says otherwise)
 // ---------------------------------------------------------------------------
 // trace_count and shade_count share one 8-byte word, so that a shade wave
@@ -385,25 +385,44 @@ struct BatchItem {
     uint32_t pixel_base, pad0, pad1, pad2;
 };
 
+// A path's live state is one 128-byte record, so that a step moves one line
+// whatever the paths beside it do: as 13 arrays of 16 bytes a path, the lines
+// of dead neighbours came along, 589 bytes a step at 4.5 TB/s.  The words are
+// float4s:
+enum PathWord : uint32_t {
+    kPathOrigin,      // origin.xyz, tmin
+    kPathDirection,   // direction.xyz, tmax
+    kPathSource,      // source object, source primitive, flag | visibility << 20 | bits << 25, step
+    kPathThroughput,  // xyz, previous BSDF pdf
+    kPathIdentity,    // sample, pixel rng hash, bounce | diffuse << 16, glossy | transmission << 16
+    kPathHit,         // instance (kNone = miss), primitive, Cycles primitive, t bits
+    kPathUv,          // hit u, v, transparent bounces, 0
+    kPathMisNormal,   // shading normal of the last non-transparent scatter (scenes with lights)
+    kPathWords
+};
+// the same for a pending shadow ray, 64 bytes
+enum ShadowWord : uint32_t {
+    kShadowOrigin,     // origin.xyz, tmax
+    kShadowDirection,  // direction.xyz, clamp depth bits
+    kShadowIdentity,   // source object, source primitive, light object, light primitive
+    kShadowLight,      // light estimate xyz, transparent depth bits
+    kShadowWords
+};
+// bounce counts take 16 bits: a path has at most kMaxPathSteps steps
+constexpr uint32_t kMaxPathSteps = 1024u;
+
 struct WavefrontView {
-    float4 *ray_o;       // origin.xyz, tmin
-    float4 *ray_d;       // direction.xyz, tmax
-    uint4 *aux;          // source object, source primitive, step, bits
-    float4 *throughput;  // xyz, previous BSDF pdf
-    float4 *mis_normal;  // shading normal of the last non-transparent scatter
+    float4 *path;        // kPathWords per path
+    float4 *shadow;      // kShadowWords per path
+    // film sums of a path; before the first shade step they hold the camera
+    // ray instead: origin and tmin, direction and tmax, and (sample, pixel rng
+    // hash, hit u, hit v).  All paths are live then, and dense arrays are
+    // written and read at full rate where records would be filled in part.
     float4 *radiance;    // xyz, transparency
     float4 *normal;      // primary normal AOV
     float4 *albedo;      // primary albedo AOV
-    uint4 *state0;       // flag, visibility, bounce, diffuse bounce
-    uint4 *state1;       // glossy, transmission, transparent bounce, rng offset
-    uint2 *ident;        // sample index, pixel rng hash
-    uint4 *hit;          // instance (kNone = miss), primitive, Cycles primitive, t bits
-    float2 *hit_uv;
-    float4 *shadow_o;    // origin.xyz, tmax
-    float4 *shadow_d;    // direction.xyz, clamp depth bits
-    uint4 *shadow_q;     // source object, source primitive, light object, light primitive
-    float4 *shadow_l;    // light estimate xyz, transparent depth bits
-    float4 *shadow_t;    // transmittance xyz
+    float4 *first_hit;   // the camera ray's hit, as kPathHit
+    float4 *shadow_t;    // light passes: transmittance xyz of the shadow ray, or null
     uint32_t *queue[2];  // trace entries: path << 1 | is_shadow
     uint32_t *list[2];   // shade entries: path
     WavefrontCounters *counters;  // one per iteration

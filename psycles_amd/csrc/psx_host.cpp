@@ -1051,11 +1051,13 @@ void Scene::rebuild_emitters(ParamTables &t) {
     view.triangle_area_pdf = tri_pdf;
 }
 
+// Bytes of a path's state: records, film sums, first hit, two queues and two lists.
+constexpr size_t kPathBytes = (kPathWords + kShadowWords + 4u) * 16u + 2u * 2u * 4u + 2u * 4u;
+
 // Wavefront path state of one session (psx_device.h, WavefrontView), sized
 // for max_samples_per_dispatch samples of every window pixel.
 struct WavefrontState {
-    DeviceBuffer ray_o, ray_d, aux, throughput, mis_normal, radiance, normal, albedo, state0, state1, ident, hit, hit_uv,
-        shadow_o, shadow_d, shadow_q, shadow_l, shadow_t, queue0, queue1, list0, list1, counters, lp, shadow_split;
+    DeviceBuffer path, shadow, radiance, normal, albedo, first_hit, shadow_t, queue0, queue1, list0, list1, counters, lp, shadow_split;
     WavefrontView view{};
 
     bool light = false;  // light-pass arrays allocated
@@ -1066,28 +1068,18 @@ struct WavefrontState {
         if (light_passes) {
             lp.allocate(n * 10u * 16u);
             shadow_split.allocate(n * 2u * 16u);
+            shadow_t.allocate(n * 16u);
         } else {
             lp.reset();
             shadow_split.reset();
+            shadow_t.reset();
         }
-        ray_o.allocate(n * 16u);
-        ray_d.allocate(n * 16u);
-        aux.allocate(n * 16u);
-        throughput.allocate(n * 16u);
-        mis_normal.allocate(n * 16u);
+        path.allocate(n * kPathWords * 16u);
+        shadow.allocate(n * kShadowWords * 16u);
         radiance.allocate(n * 16u);
         normal.allocate(n * 16u);
         albedo.allocate(n * 16u);
-        state0.allocate(n * 16u);
-        state1.allocate(n * 16u);
-        ident.allocate(n * 8u);
-        hit.allocate(n * 16u);
-        hit_uv.allocate(n * 8u);
-        shadow_o.allocate(n * 16u);
-        shadow_d.allocate(n * 16u);
-        shadow_q.allocate(n * 16u);
-        shadow_l.allocate(n * 16u);
-        shadow_t.allocate(n * 16u);
+        first_hit.allocate(n * 16u);
         // a live path queues at most a continuation ray and a shadow ray;
         // shade waves leave partly used reservations as skip entries
         const size_t qh = wavefront_queue_headroom(), lh = wavefront_list_headroom();
@@ -1097,24 +1089,13 @@ struct WavefrontState {
         list1.allocate((n + lh) * 4u);
         counters.allocate((iterations + 1u) * sizeof(WavefrontCounters));
         WavefrontView &v = view;
-        v.ray_o = ray_o.as<float4>();
-        v.ray_d = ray_d.as<float4>();
-        v.aux = aux.as<uint4>();
-        v.throughput = throughput.as<float4>();
-        v.mis_normal = mis_normal.as<float4>();
+        v.path = path.as<float4>();
+        v.shadow = shadow.as<float4>();
         v.radiance = radiance.as<float4>();
         v.normal = normal.as<float4>();
         v.albedo = albedo.as<float4>();
-        v.state0 = state0.as<uint4>();
-        v.state1 = state1.as<uint4>();
-        v.ident = ident.as<uint2>();
-        v.hit = hit.as<uint4>();
-        v.hit_uv = hit_uv.as<float2>();
-        v.shadow_o = shadow_o.as<float4>();
-        v.shadow_d = shadow_d.as<float4>();
-        v.shadow_q = shadow_q.as<uint4>();
-        v.shadow_l = shadow_l.as<float4>();
-        v.shadow_t = shadow_t.as<float4>();
+        v.first_hit = first_hit.as<float4>();
+        v.shadow_t = light_passes ? shadow_t.as<float4>() : nullptr;
         v.queue[0] = queue0.as<uint32_t>();
         v.queue[1] = queue1.as<uint32_t>();
         v.list[0] = list0.as<uint32_t>();
@@ -1246,7 +1227,7 @@ KernelParams kernel_params(const Scene &scene, const SceneView &view, const psx_
     k.transparent_min = synced(in.transparent_min_bounces);
     k.transparent_max = in.transparent_max_bounces;
     const uint64_t req = 2ull * k.max_bounces + std::max(in.transparent_max_bounces, 1u) + 1ull;
-    k.max_path_steps = static_cast<uint32_t>(std::min<uint64_t>(req, 1024ull));
+    k.max_path_steps = static_cast<uint32_t>(std::min<uint64_t>(req, kMaxPathSteps));
     k.transparent_background = rs.transparent_background;
     k.clamp_direct = in.sample_clamp_direct > 0.0f ? in.sample_clamp_direct * 3.0f : 0.0f;
     k.clamp_indirect = in.sample_clamp_indirect > 0.0f ? in.sample_clamp_indirect * 3.0f : 0.0f;
@@ -3561,7 +3542,7 @@ int psx_server_create(psx_backend *b, const psx_server_options *options, psx_ser
             std::memset(a->host_queues, 0, (kMaxIterations + 1u) * sizeof(WavefrontCounters));
             // the upper half of the streams takes viewport batches only
             a->viewport_only = i >= o.streams - std::max(o.streams / 2u, 1u);
-            a->bytes = static_cast<size_t>(o.path_capacity) * 288u + a->items.bytes() + a->spill.bytes();
+            a->bytes = static_cast<size_t>(o.path_capacity) * kPathBytes + a->items.bytes() + a->spill.bytes();
             server->fixed_bytes += a->bytes;
             server->arenas.push_back(std::move(a));
         }

@@ -2579,7 +2579,25 @@ struct PathVars {
     uint32_t sample, rng_hash, step, bits;
     LightSums lp;   // only read and written by the light-pass kernels
     float min_pdf;  // path traces only: smallest non-transparent BSDF pdf so far
+    // where the radiance and transparency still are, or null once they are in
+    // `radiance` and `transparency`: most steps add nothing to them
+    const float4 *stored;
 };
+
+__device__ __forceinline__ void path_radiance(PathVars &p) {
+    if (!p.stored) return;
+    const float4 r = *p.stored;
+    p.radiance = V(r.x, r.y, r.z);
+    p.transparency = r.w;
+    p.stored = nullptr;
+}
+
+// adds a contribution; adding zeros changes no bit (the sum is never -0)
+__device__ __forceinline__ void path_add(PathVars &p, f3 c) {
+    if (!any_nonzero(c)) return;
+    path_radiance(p);
+    p.radiance = p.radiance + c;
+}
 
 struct ShadowRay {
     Ray ray;
@@ -2643,10 +2661,8 @@ __device__ __forceinline__ TraceQuery path_query(const PathVars &p) {
     return q;
 }
 
-// camera ray and initial state (src/luisa/path_kernel_setup.cpp)
-__device__ __forceinline__ void init_path(const KernelParams &k, const float4 *sobol, const float *filter,
-                                          uint32_t fx, uint32_t fy, uint32_t sample, PathVars &p) {
-    p.ray = camera_ray(k, sobol, filter, fx, fy, sample, p.rng_hash);
+// state of a path that has taken no step, but for its ray and sample
+__device__ __forceinline__ void new_path_state(PathVars &p) {
     p.src_obj = p.src_prim = 0xffffffffu;
     p.throughput = V(1.0f, 1.0f, 1.0f);
     p.prev_pdf = 0.0f;
@@ -2659,10 +2675,21 @@ __device__ __forceinline__ void init_path(const KernelParams &k, const float4 *s
     p.ps.visibility = CVIS_CAMERA;
     p.ps.bounce = p.ps.diffuse_bounce = p.ps.glossy_bounce = p.ps.transmission_bounce = p.ps.transparent_bounce = 0u;
     p.ps.rng_offset = 16u;
-    p.sample = sample;
     p.step = 0u;
-    p.bits = PATH_PREV_DELTA | (k.max_path_steps == 0u ? PATH_DONE : 0u);
+    p.bits = PATH_PREV_DELTA;
+    p.lp.dd = p.lp.di = p.lp.gd = p.lp.gi = p.lp.td = p.lp.ti = p.lp.emission = p.lp.environment = p.lp.path_dw =
+        p.lp.path_gw = V(0.0f, 0.0f, 0.0f);
     p.min_pdf = FLT_MAX;
+    p.stored = nullptr;
+}
+
+// camera ray and initial state (src/luisa/path_kernel_setup.cpp)
+__device__ __forceinline__ void init_path(const KernelParams &k, const float4 *sobol, const float *filter,
+                                          uint32_t fx, uint32_t fy, uint32_t sample, PathVars &p) {
+    new_path_state(p);
+    p.ray = camera_ray(k, sobol, filter, fx, fy, sample, p.rng_hash);
+    p.sample = sample;
+    if (k.max_path_steps == 0u) p.bits |= PATH_DONE;
 }
 
 // transparent shadow continuation (src/luisa/path_tracer_geometry.cpp:75-174):
@@ -2700,7 +2727,7 @@ __device__ __forceinline__ void apply_shadow(const KernelParams &k, PathVars &p,
                                              f3 transmittance, f3 dw, f3 gw) {
     if (transmittance.x > 0.0f || transmittance.y > 0.0f || transmittance.z > 0.0f) {
         const f3 c = film_clamp(L * transmittance, depth, k.clamp_direct, k.clamp_indirect);
-        p.radiance = p.radiance + c;
+        path_add(p, c);
         if (LP) lp_scattered(p.lp, c, dw, gw, depth == 0u);
     }
 }
@@ -2866,7 +2893,7 @@ __device__ bool path_step(const SceneView &s, const LampView &lv, const KernelPa
             const f3 light_radiance = lamp3(l.color) * (l.power * best_eval);
             const f3 lc = film_clamp((p.throughput * light_radiance) * mis, p.ps.bounce > 1u ? 1u : 0u,
                                      k.clamp_direct, k.clamp_indirect);
-            p.radiance = p.radiance + lc;
+            path_add(p, lc);
             if (LP) lp_route(p.lp, false, lc, p.ps.flag, p.ps.bounce);
             p.ps.transparent_bounce += 1u;
             p.ray.tmin = next_float_up(event_distance);
@@ -2884,9 +2911,10 @@ __device__ bool path_step(const SceneView &s, const LampView &lv, const KernelPa
         const bool transparent_bg =
             k.transparent_background != 0u && (p.ps.flag & FLAG_TRANSPARENT_BACKGROUND) != 0u;
         if (transparent_bg) {
+            path_radiance(p);
             p.transparency += (p.throughput.x + p.throughput.y + p.throughput.z) * (1.0f / 3.0f);
         } else if (world_visible) {
-            p.radiance = p.radiance + c;
+            path_add(p, c);
         }
         if (LP) lp_route(p.lp, true, world_visible ? c : V(0.0f, 0.0f, 0.0f), p.ps.flag, p.ps.bounce);
         return false;
@@ -2924,7 +2952,7 @@ __device__ bool path_step(const SceneView &s, const LampView &lv, const KernelPa
     }
     const f3 emitted = film_clamp((p.throughput * cs.emission) * emission_weight, p.ps.bounce > 1u ? 1u : 0u,
                                   k.clamp_direct, k.clamp_indirect);
-    p.radiance = p.radiance + emitted;
+    path_add(p, emitted);
     if (LP) lp_route(p.lp, false, emitted, p.ps.flag, p.ps.bounce);
     if (terminate_on_next_surface) return false;
     // Russian roulette (cycles_path_state.h:416-446)

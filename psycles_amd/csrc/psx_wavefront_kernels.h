@@ -36,39 +36,41 @@ __device__ __forceinline__ void add_counter(unsigned long long *dst, uint32_t va
     if ((threadIdx.x & 63) == 0 && v != 0ull) atomicAdd(dst, v);
 }
 
-// The state a shade step can change: the sample identity never changes
-// after generation, and the primary Normal / Albedo only while the path is
-// at bounce 0 (`aov`).  The MIS normal is read only by light sampling and
-// forward-hit MIS, so a scene without lights (MIS = false) neither loads nor
-// stores it.
-template <bool MIS>
-__device__ __forceinline__ void store_step(const WavefrontView &w, uint32_t i, const PathVars &p, bool aov) {
-    w.ray_o[i] = make_float4(p.ray.o.x, p.ray.o.y, p.ray.o.z, p.ray.tmin);
-    w.ray_d[i] = make_float4(p.ray.d.x, p.ray.d.y, p.ray.d.z, p.ray.tmax);
-    w.aux[i] = make_uint4(p.src_obj, p.src_prim, p.step, p.bits);
-    w.throughput[i] = make_float4(p.throughput.x, p.throughput.y, p.throughput.z, p.prev_pdf);
-    if (MIS) w.mis_normal[i] = make_float4(p.mis_normal.x, p.mis_normal.y, p.mis_normal.z, 0.0f);
-    w.radiance[i] = make_float4(p.radiance.x, p.radiance.y, p.radiance.z, p.transparency);
-    if (aov) {
-        w.normal[i] = make_float4(p.normal.x, p.normal.y, p.normal.z, 0.0f);
-        w.albedo[i] = make_float4(p.albedo.x, p.albedo.y, p.albedo.z, 0.0f);
-    }
-    w.state0[i] = make_uint4(p.ps.flag, p.ps.visibility, p.ps.bounce, p.ps.diffuse_bounce);
-    w.state1[i] = make_uint4(p.ps.glossy_bounce, p.ps.transmission_bounce, p.ps.transparent_bounce, p.ps.rng_offset);
+// float4 number `word` of a path's and of a shadow ray's record
+__device__ __forceinline__ float4 &path_word(const WavefrontView &w, uint32_t i, uint32_t word) {
+    return w.path[static_cast<size_t>(i) * kPathWords + word];
+}
+__device__ __forceinline__ float4 &shadow_word(const WavefrontView &w, uint32_t i, uint32_t word) {
+    return w.shadow[static_cast<size_t>(i) * kShadowWords + word];
+}
+__device__ __forceinline__ uint32_t bits_of(float v) { return __float_as_uint(v); }
+__device__ __forceinline__ float4 bit_words(uint32_t x, uint32_t y, uint32_t z, uint32_t w) {
+    return make_float4(__uint_as_float(x), __uint_as_float(y), __uint_as_float(z), __uint_as_float(w));
 }
 
-__device__ __forceinline__ void store_path(const WavefrontView &w, uint32_t i, const PathVars &p) {
-    w.ray_o[i] = make_float4(p.ray.o.x, p.ray.o.y, p.ray.o.z, p.ray.tmin);
-    w.ray_d[i] = make_float4(p.ray.d.x, p.ray.d.y, p.ray.d.z, p.ray.tmax);
-    w.aux[i] = make_uint4(p.src_obj, p.src_prim, p.step, p.bits);
-    w.throughput[i] = make_float4(p.throughput.x, p.throughput.y, p.throughput.z, p.prev_pdf);
-    w.mis_normal[i] = make_float4(p.mis_normal.x, p.mis_normal.y, p.mis_normal.z, 0.0f);
-    w.radiance[i] = make_float4(p.radiance.x, p.radiance.y, p.radiance.z, p.transparency);
-    w.normal[i] = make_float4(p.normal.x, p.normal.y, p.normal.z, 0.0f);
-    w.albedo[i] = make_float4(p.albedo.x, p.albedo.y, p.albedo.z, 0.0f);
-    w.state0[i] = make_uint4(p.ps.flag, p.ps.visibility, p.ps.bounce, p.ps.diffuse_bounce);
-    w.state1[i] = make_uint4(p.ps.glossy_bounce, p.ps.transmission_bounce, p.ps.transparent_bounce, p.ps.rng_offset);
-    w.ident[i] = make_uint2(p.sample, p.rng_hash);
+// What generation stores: the camera ray and the sample's identity, in the
+// film sums' arrays.  The rest of a new path is constant (new_path_state).
+__device__ __forceinline__ void store_camera_path(const WavefrontView &w, uint32_t i, const PathVars &p) {
+    w.radiance[i] = make_float4(p.ray.o.x, p.ray.o.y, p.ray.o.z, p.ray.tmin);
+    w.normal[i] = make_float4(p.ray.d.x, p.ray.d.y, p.ray.d.z, p.ray.tmax);
+    w.albedo[i] = bit_words(p.sample, p.rng_hash, 0u, 0u);
+}
+
+// The state of a path that goes on.  The MIS normal is read only by light
+// sampling and forward-hit MIS, so a scene without lights (MIS = false)
+// neither loads nor stores it.
+template <bool MIS>
+__device__ __forceinline__ void store_step(const WavefrontView &w, uint32_t i, const PathVars &p) {
+    path_word(w, i, kPathOrigin) = make_float4(p.ray.o.x, p.ray.o.y, p.ray.o.z, p.ray.tmin);
+    path_word(w, i, kPathDirection) = make_float4(p.ray.d.x, p.ray.d.y, p.ray.d.z, p.ray.tmax);
+    path_word(w, i, kPathSource) =
+        bit_words(p.src_obj, p.src_prim, p.ps.flag | (p.ps.visibility << 20) | (p.bits << 25), p.step);
+    path_word(w, i, kPathThroughput) = make_float4(p.throughput.x, p.throughput.y, p.throughput.z, p.prev_pdf);
+    path_word(w, i, kPathIdentity) =
+        bit_words(p.sample, p.rng_hash, p.ps.bounce | (p.ps.diffuse_bounce << 16),
+                  p.ps.glossy_bounce | (p.ps.transmission_bounce << 16));
+    path_word(w, i, kPathUv).z = __uint_as_float(p.ps.transparent_bounce);
+    if (MIS) path_word(w, i, kPathMisNormal) = make_float4(p.mis_normal.x, p.mis_normal.y, p.mis_normal.z, 0.0f);
 }
 
 // light-pass sums of a path, field-major: field f of path i at f * capacity + i
@@ -101,55 +103,69 @@ __device__ __forceinline__ LightSums load_lp(const WavefrontView &w, uint32_t i)
     return lp;
 }
 
-// A path's state for one shade step.  The primary Normal / Albedo are read
-// only while the path is at bounce 0, the only steps that change them, and
-// the MIS normal only with MIS (see store_step).
+// A path's state for one shade step and the hit of its ray.  The first step
+// (`first`) takes the constants of a new path; later ones leave the radiance
+// where it is until something is added, and read the primary Albedo only at
+// bounce 0, the only steps that change it.
 template <bool MIS>
-__device__ __forceinline__ PathVars load_path(const WavefrontView &w, uint32_t i) {
+__device__ __forceinline__ PathVars load_path(const WavefrontView &w, uint32_t i, bool first, Hit &h) {
     PathVars p;
-    const float4 o = w.ray_o[i], d = w.ray_d[i];
+    const float4 o = first ? w.radiance[i] : path_word(w, i, kPathOrigin);
+    const float4 d = first ? w.normal[i] : path_word(w, i, kPathDirection);
+    const float4 id = first ? w.albedo[i] : path_word(w, i, kPathIdentity);
+    const float4 hv = first ? w.first_hit[i] : path_word(w, i, kPathHit);
+    const float4 uv = first ? make_float4(id.z, id.w, 0.0f, 0.0f) : path_word(w, i, kPathUv);
     p.ray.o = V(o.x, o.y, o.z);
     p.ray.tmin = o.w;
     p.ray.d = V(d.x, d.y, d.z);
     p.ray.tmax = d.w;
-    const uint4 a = w.aux[i];
-    p.src_obj = a.x;
-    p.src_prim = a.y;
-    p.step = a.z;
-    p.bits = a.w;
-    const float4 t = w.throughput[i];
+    p.sample = bits_of(id.x);
+    p.rng_hash = bits_of(id.y);
+    h.inst = h.object = bits_of(hv.x);
+    h.valid = h.inst != kNone;
+    h.prim = bits_of(hv.y);
+    h.cprim = bits_of(hv.z);
+    h.t = hv.w;
+    h.u = uv.x;
+    h.v = uv.y;
+    if (first) {
+        new_path_state(p);
+        return p;
+    }
+    const float4 a = path_word(w, i, kPathSource), t = path_word(w, i, kPathThroughput);
+    p.src_obj = bits_of(a.x);
+    p.src_prim = bits_of(a.y);
+    p.ps.flag = bits_of(a.z) & 0xfffffu;
+    p.ps.visibility = (bits_of(a.z) >> 20) & 0x1fu;
+    p.bits = bits_of(a.z) >> 25;
+    p.step = bits_of(a.w);
     p.throughput = V(t.x, t.y, t.z);
     p.prev_pdf = t.w;
+    p.mis_normal = V(0.0f, 0.0f, 0.0f);
     if (MIS) {
-        const float4 mn = w.mis_normal[i];
+        const float4 mn = path_word(w, i, kPathMisNormal);
         p.mis_normal = V(mn.x, mn.y, mn.z);
-    } else {
-        p.mis_normal = V(0.0f, 0.0f, 0.0f);
     }
-    const float4 r = w.radiance[i];
-    p.radiance = V(r.x, r.y, r.z);
-    p.transparency = r.w;
-    const uint4 s0 = w.state0[i], s1 = w.state1[i];
-    if (s0.z == 0u) {
-        const float4 n = w.normal[i];
-        p.normal = V(n.x, n.y, n.z);
+    p.ps.bounce = bits_of(id.z) & 0xffffu;
+    p.ps.diffuse_bounce = bits_of(id.z) >> 16;
+    p.ps.glossy_bounce = bits_of(id.w) & 0xffffu;
+    p.ps.transmission_bounce = bits_of(id.w) >> 16;
+    p.ps.transparent_bounce = bits_of(uv.z);
+    p.ps.rng_offset = 16u * (p.step + 1u);
+    p.radiance = p.normal = p.albedo = V(0.0f, 0.0f, 0.0f);
+    p.transparency = 0.0f;
+    p.stored = w.radiance + i;
+    if (p.ps.bounce == 0u) {
         const float4 al = w.albedo[i];
         p.albedo = V(al.x, al.y, al.z);
-    } else {
-        p.normal = p.albedo = V(0.0f, 0.0f, 0.0f);
     }
-    p.ps.flag = s0.x;
-    p.ps.visibility = s0.y;
-    p.ps.bounce = s0.z;
-    p.ps.diffuse_bounce = s0.w;
-    p.ps.glossy_bounce = s1.x;
-    p.ps.transmission_bounce = s1.y;
-    p.ps.transparent_bounce = s1.z;
-    p.ps.rng_offset = s1.w;
-    const uint2 id = w.ident[i];
-    p.sample = id.x;
-    p.rng_hash = id.y;
     return p;
+}
+
+// film sums of a path that has none
+__device__ __forceinline__ void store_empty_film(const WavefrontView &w, uint32_t i) {
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    w.radiance[i] = w.normal[i] = w.albedo[i] = zero;
 }
 
 __global__ void reset_kernel(WavefrontCounters *counters, uint32_t n) {
@@ -171,24 +187,17 @@ __global__ __launch_bounds__(kShadeBlock) void generate_kernel(KernelParams k, c
         const uint32_t sample = first + i / w.padded_pixels;
         uint32_t px, py;
         tile_pixel(i % w.padded_pixels, k.window_width, w.tile_shift, px, py);
-        PathVars p;
         if (px < k.window_width && py < k.window_height) {
+            PathVars p;
             init_path(k, sobol, filter, px + k.window_x, py + k.window_y, sample, p);
             live = (p.bits & PATH_DONE) == 0u;
-        } else {
-            p.bits = PATH_DONE;
-            p.ray.o = p.ray.d = V(0.0f, 0.0f, 0.0f);
-            p.ray.tmin = p.ray.tmax = 0.0f;
-            p.src_obj = p.src_prim = 0xffffffffu;
-            p.throughput = p.radiance = p.normal = p.albedo = p.mis_normal = V(0.0f, 0.0f, 0.0f);
-            p.prev_pdf = p.transparency = 0.0f;
-            p.ps = PathState{0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-            p.sample = sample;
-            p.rng_hash = 0u;
-            p.step = 0u;
+            if (live) {
+                store_camera_path(w, i, p);
+            } else {
+                store_empty_film(w, i);
+            }
         }
-        store_path(w, i, p);
-        if (w.lp) {
+        if (w.lp && !live) {
             LightSums z;
             z.dd = z.di = z.gd = z.gi = z.td = z.ti = z.emission = z.environment = z.path_dw = z.path_gw =
                 V(0.0f, 0.0f, 0.0f);
@@ -230,6 +239,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wf_trace_kernel(SceneView s, K
     bool active = false, exhausted = false, shadow = false;
     uint32_t path = 0u, tdepth = 0u;
     f3 transmittance = V(1.0f, 1.0f, 1.0f);
+    const f3 no_split = V(0.0f, 0.0f, 0.0f);
     // The wave's reservation [res, res_end) of queue entries.  One atomic on
     // the shared cursor reserves w.trace_chunk entries, which the wave hands to its
     // idle lanes over several refills: a returning atomic on one address
@@ -321,17 +331,23 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wf_trace_kernel(SceneView s, K
                     Ray ray;
                     TraceQuery q;
                     if (shadow) {
-                        const float4 o = w.shadow_o[path], d = w.shadow_d[path];
-                        const uint4 sq = w.shadow_q[path];
+                        const float4 o = shadow_word(w, path, kShadowOrigin), d = shadow_word(w, path, kShadowDirection);
+                        const float4 sq = shadow_word(w, path, kShadowIdentity);
                         ray = Ray{V(o.x, o.y, o.z), V(d.x, d.y, d.z), 0.0f, o.w};
-                        q = TraceQuery{VIS_SHADOW, sq.x, sq.y, sq.z, sq.w};
-                        tdepth = __float_as_uint(w.shadow_l[path].w);
+                        q = TraceQuery{VIS_SHADOW, bits_of(sq.x), bits_of(sq.y), bits_of(sq.z), bits_of(sq.w)};
+                        tdepth = bits_of(shadow_word(w, path, kShadowLight).w);
                         transmittance = V(1.0f, 1.0f, 1.0f);
                     } else {
-                        const float4 o = w.ray_o[path], d = w.ray_d[path];
-                        const uint4 a = w.aux[path];
+                        const float4 o = it == 0u ? w.radiance[path] : path_word(w, path, kPathOrigin);
+                        const float4 d = it == 0u ? w.normal[path] : path_word(w, path, kPathDirection);
                         ray = Ray{V(o.x, o.y, o.z), V(d.x, d.y, d.z), o.w, d.w};
-                        q = TraceQuery{contract_visibility(w.state0[path].y), a.x, a.y, kNone, kNone};
+                        q = TraceQuery{contract_visibility(CVIS_CAMERA), kNone, kNone, kNone, kNone};
+                        if (it > 0u) {
+                            const float4 a = path_word(w, path, kPathSource);
+                            q.visibility = contract_visibility((bits_of(a.z) >> 20) & 0x1fu);
+                            q.src_obj = bits_of(a.x);
+                            q.src_prim = bits_of(a.y);
+                        }
                     }
                     traversal_begin(s, t, st, ray, q);
                     active = true;
@@ -356,13 +372,33 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wf_trace_kernel(SceneView s, K
             ++rays;
             const Hit h = traversal_result(t, st);
             if (!shadow) {
-                w.hit[path] = make_uint4(h.inst, h.prim, h.cprim, __float_as_uint(h.t));
-                w.hit_uv[path] = make_float2(h.u, h.v);
+                float4 *hit = it == 0u ? w.first_hit + path : &path_word(w, path, kPathHit);
+                float2 *uv = it == 0u ? reinterpret_cast<float2 *>(w.albedo + path) + 1
+                                      : reinterpret_cast<float2 *>(&path_word(w, path, kPathUv));
+                *hit = bit_words(h.inst, h.prim, h.cprim, __float_as_uint(h.t));
+                *uv = make_float2(h.u, h.v);
                 active = false;
             } else {
                 Ray rest;
                 if (shadow_hit(s, k.transparent_max, h, rest, tdepth, transmittance)) {
-                    w.shadow_t[path] = make_float4(transmittance.x, transmittance.y, transmittance.z, 0.0f);
+                    if (w.shadow_t) {
+                        // light passes: the next shade step applies it
+                        w.shadow_t[path] = make_float4(transmittance.x, transmittance.y, transmittance.z, 0.0f);
+                    } else {
+                        // the path's radiance is not touched between the
+                        // shade steps, so the light joins it here, in the
+                        // order of the path: after this step's emission and
+                        // before the next one's
+                        const float4 L = shadow_word(w, path, kShadowLight);
+                        PathVars sum;
+                        sum.stored = w.radiance + path;
+                        apply_shadow<false>(k, sum, V(L.x, L.y, L.z),
+                                            bits_of(shadow_word(w, path, kShadowDirection).w), transmittance, no_split,
+                                            no_split);
+                        if (!sum.stored)
+                            w.radiance[path] =
+                                make_float4(sum.radiance.x, sum.radiance.y, sum.radiance.z, sum.transparency);
+                    }
                     active = false;
                 } else {
                     // past a transparent surface: same shadow ray from the next float
@@ -384,10 +420,10 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wf_trace_kernel(SceneView s, K
 // wave diverges less; the order within a class is arbitrary, and no path's
 // result depends on it.  Every thread of the block calls it.
 __device__ __forceinline__ uint32_t sort_block(const SceneView &s, const WavefrontView &w, uint32_t entry,
-                                               uint32_t *slot, uint32_t *counts) {
+                                               bool first, uint32_t *slot, uint32_t *counts) {
     uint32_t key = 0u;
     if (entry != kSkip) {
-        const uint32_t inst = w.hit[entry].x;
+        const uint32_t inst = bits_of(first ? w.first_hit[entry].x : path_word(w, entry, kPathHit).x);
         key = inst < s.instance_count ? s.instances[inst].shade_class : 0u;
         key = key < kShadeKeys ? key : kShadeKeys - 1u;
     }
@@ -435,69 +471,65 @@ __device__ __forceinline__ void shade_launch(const SceneView &s, const KernelPar
     __shared__ uint32_t sort_slot[kShadeBlock];
     __shared__ uint32_t sort_count[kShadeKeys];
     const bool sorted = w.shade_sort != 0u;
+    const bool first = it == 0u;
     // the block steps over the list together (the sort is block-wide)
     for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += stride) {
         const uint32_t i = base + threadIdx.x;
         uint32_t entry = i < count ? list[i] : kSkip;
-        if (sorted) entry = sort_block(s, w, entry, sort_slot, sort_count);
-        bool cont = false, shadow = false;
+        if (sorted) entry = sort_block(s, w, entry, first, sort_slot, sort_count);
+        bool cont = false, shadow = false, live = false;
         uint32_t path = 0u;
         if (entry != kSkip) {
             path = entry;
-            PathVars p = load_path<LIGHTS>(w, path);
+            Hit h;
+            PathVars p = load_path<LIGHTS>(w, path, first, h);
             const bool aov = p.ps.bounce == 0u;
-            if (LP) p.lp = load_lp(w, path);
-            if ((p.bits & PATH_SHADOW_PENDING) != 0u) {
-                const float4 L = w.shadow_l[path];
+            const uint32_t flag = p.ps.flag;
+            if (LP && !first) p.lp = load_lp(w, path);
+            if (LP && (p.bits & PATH_SHADOW_PENDING) != 0u) {
+                const float4 L = shadow_word(w, path, kShadowLight);
                 const float4 tr = w.shadow_t[path];
-                f3 dw = V(0.0f, 0.0f, 0.0f), gw = dw;
-                if (LP) {
-                    const float4 a = w.shadow_split[path], b = w.shadow_split[w.capacity + path];
-                    dw = V(a.x, a.y, a.z);
-                    gw = V(b.x, b.y, b.z);
-                }
-                apply_shadow<LP>(k, p, V(L.x, L.y, L.z), __float_as_uint(w.shadow_d[path].w), V(tr.x, tr.y, tr.z),
-                                 dw, gw);
+                const float4 a = w.shadow_split[path], b = w.shadow_split[w.capacity + path];
+                apply_shadow<LP>(k, p, V(L.x, L.y, L.z), bits_of(shadow_word(w, path, kShadowDirection).w),
+                                 V(tr.x, tr.y, tr.z), V(a.x, a.y, a.z), V(b.x, b.y, b.z));
                 p.bits &= ~PATH_SHADOW_PENDING;
             }
-            if ((p.bits & PATH_FINISHING) != 0u) {
-                p.bits = (p.bits & ~PATH_FINISHING) | PATH_DONE;
-            } else {
-                const uint4 hv = w.hit[path];
-                const float2 uv = w.hit_uv[path];
-                Hit h;
-                h.valid = hv.x != kNone;
-                h.inst = hv.x;
-                h.object = hv.x;
-                h.prim = hv.y;
-                h.cprim = hv.z;
-                h.t = __uint_as_float(hv.w);
-                h.u = uv.x;
-                h.v = uv.y;
+            if (!LP || (p.bits & PATH_FINISHING) == 0u) {
                 ShadowRay sr;
                 cont = path_step<false, LP, LIGHTS>(s, lv, k, sobol, p, h, sr, nullptr);
                 shadow = sr.active;
                 if (shadow) {
-                    w.shadow_o[path] = make_float4(sr.ray.o.x, sr.ray.o.y, sr.ray.o.z, sr.ray.tmax);
-                    w.shadow_d[path] = make_float4(sr.ray.d.x, sr.ray.d.y, sr.ray.d.z, __uint_as_float(sr.depth));
-                    w.shadow_q[path] = make_uint4(sr.q.src_obj, sr.q.src_prim, sr.q.light_obj, sr.q.light_prim);
-                    w.shadow_l[path] = make_float4(sr.L.x, sr.L.y, sr.L.z, __uint_as_float(sr.tdepth));
+                    shadow_word(w, path, kShadowOrigin) = make_float4(sr.ray.o.x, sr.ray.o.y, sr.ray.o.z, sr.ray.tmax);
+                    shadow_word(w, path, kShadowDirection) =
+                        make_float4(sr.ray.d.x, sr.ray.d.y, sr.ray.d.z, __uint_as_float(sr.depth));
+                    shadow_word(w, path, kShadowIdentity) =
+                        bit_words(sr.q.src_obj, sr.q.src_prim, sr.q.light_obj, sr.q.light_prim);
+                    shadow_word(w, path, kShadowLight) =
+                        make_float4(sr.L.x, sr.L.y, sr.L.z, __uint_as_float(sr.tdepth));
                     if (LP) {
                         w.shadow_split[path] = make_float4(sr.dw.x, sr.dw.y, sr.dw.z, 0.0f);
                         w.shadow_split[w.capacity + path] = make_float4(sr.gw.x, sr.gw.y, sr.gw.z, 0.0f);
+                        p.bits |= PATH_SHADOW_PENDING;
                     }
-                    p.bits |= PATH_SHADOW_PENDING;
                 }
-                if (!cont) p.bits |= shadow ? PATH_FINISHING : PATH_DONE;
+                if (LP && !cont) p.bits |= shadow ? PATH_FINISHING : PATH_DONE;
             }
-            store_step<LIGHTS>(w, path, p, aov);
+            // A path that ended leaves its film sums only; what its last
+            // shadow ray brings is added by the trace kernel, except to the
+            // light passes, which the next shade step completes.
+            live = cont || (LP && shadow);
+            if (live) store_step<LIGHTS>(w, path, p);
+            if (!p.stored) w.radiance[path] = make_float4(p.radiance.x, p.radiance.y, p.radiance.z, p.transparency);
+            if (aov) w.albedo[path] = make_float4(p.albedo.x, p.albedo.y, p.albedo.z, 0.0f);
+            if (first || ((flag ^ p.ps.flag) & FLAG_SINGLE_PASS_DONE) != 0u)
+                w.normal[path] = make_float4(p.normal.x, p.normal.y, p.normal.z, 0.0f);
             if (LP) store_lp(w, path, p.lp);
         }
         // the wave's continuation entries, then its shadow entries, into its
         // queue reservation, and its live paths into its list reservation;
         // an append that overflows a reservation continues in a new chunk
-        const unsigned long long cm = __ballot(cont), sm = __ballot(shadow), lm = cm | sm;
-        if (lm != 0ull) {
+        const unsigned long long cm = __ballot(cont), sm = __ballot(shadow), lm = __ballot(live);
+        if ((cm | sm) != 0ull) {
             const uint32_t nc = static_cast<uint32_t>(__popcll(cm)), ns = static_cast<uint32_t>(__popcll(sm));
             const uint32_t nq = nc + ns, nl = static_cast<uint32_t>(__popcll(lm));
             const uint32_t q_old = q_pos, q_avail = q_end - q_pos;
@@ -530,7 +562,7 @@ __device__ __forceinline__ void shade_launch(const SceneView &s, const KernelPar
                 next_queue[r2 < q_avail ? q_old + r2 : q_new + (r2 - q_avail)] = (path << 1) | 1u;
             }
             const uint32_t lr = static_cast<uint32_t>(__popcll(lm & below));
-            if (cont || shadow) next_list[lr < l_avail ? l_old + lr : l_new + (lr - l_avail)] = path;
+            if (live) next_list[lr < l_avail ? l_old + lr : l_new + (lr - l_avail)] = path;
         }
     }
     // the unused ends of this wave's reservations become skip entries
@@ -646,24 +678,17 @@ __global__ __launch_bounds__(kShadeBlock) void generate_batch_kernel(const Batch
     const uint32_t tiles_x = (k.window_width + 7u) >> 3;
     const uint32_t px = (tile % tiles_x) * 8u + (lane & 7u);
     const uint32_t py = (tile / tiles_x) * 8u + (lane >> 3);
-    PathVars p;
     bool live = false;
     if (px < k.window_width && py < k.window_height) {
+        PathVars p;
         init_path(k, it.sobol, it.filter, px + k.window_x, py + k.window_y, sample, p);
         live = (p.bits & PATH_DONE) == 0u;
-    } else {
-        p.bits = PATH_DONE;
-        p.ray.o = p.ray.d = V(0.0f, 0.0f, 0.0f);
-        p.ray.tmin = p.ray.tmax = 0.0f;
-        p.src_obj = p.src_prim = 0xffffffffu;
-        p.throughput = p.radiance = p.normal = p.albedo = p.mis_normal = V(0.0f, 0.0f, 0.0f);
-        p.prev_pdf = p.transparency = 0.0f;
-        p.ps = PathState{0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-        p.sample = sample;
-        p.rng_hash = 0u;
-        p.step = 0u;
+        if (live) {
+            store_camera_path(w, i, p);
+        } else {
+            store_empty_film(w, i);
+        }
     }
-    store_path(w, i, p);
     w.queue[0][i] = live ? (i << 1) : kSkip;
     w.list[0][i] = live ? i : kSkip;
 }
