@@ -471,12 +471,13 @@ typedef struct psx_wavefront_tuning {
                               tile_width x (64 / tile_width) pixels (8)      */
     uint32_t refill_lanes; /* 1..64: idle lanes of a trace wave that make it
                               take new rays from the queue (16)              */
-    uint32_t trace_chunk;  /* 16..4096: queue entries a trace wave reserves
-                              per atomic (128)                               */
-    uint32_t queue_chunk;  /* 128 or 256: next-queue slots a shade wave
+    uint32_t trace_chunk;  /* 16..4096: a trace wave reserves twice as many
+                              queue entries per atomic, fewer where the
+                              queue is short (128)                           */
+    uint32_t queue_chunk;  /* 128 or 256: most next-queue slots a shade wave
                               reserves per atomic (256)                      */
-    uint32_t list_chunk;   /* 64, 128 or 256: shade-list slots a shade wave
-                              reserves per atomic (128)                      */
+    uint32_t list_chunk;   /* 64, 128 or 256: a shade wave reserves up to twice
+                              as many shade-list slots per atomic (128)      */
     uint32_t sort_shading; /* 0 or 1: each shade block takes its 256 paths
                               sorted by closure structure of the hit (0)    */
     uint32_t xcd_segments; /* 1 or 8: trace waves take rays from one queue, or

@@ -433,9 +433,9 @@ struct WavefrontView {
     // launch shape (any values in range give the same film):
     uint32_t tile_shift;    // a wave's 64 paths cover (1 << tile_shift) x (64 >> tile_shift) pixels
     uint32_t refill;        // idle lanes of a trace wave that trigger a refill, 1..64
-    uint32_t trace_chunk;   // queue entries a trace wave reserves per atomic, >= 1
-    uint32_t queue_chunk;   // next-queue slots a shade wave reserves per atomic, 128..kMaxQueueChunk
-    uint32_t list_chunk;    // shade-list slots a shade wave reserves per atomic, 64..kMaxListChunk
+    uint32_t trace_chunk;   // half the queue entries a trace wave reserves per atomic, >= 1
+    uint32_t queue_chunk;   // next-queue slots a shade wave reserves per atomic at most, 128..kMaxQueueChunk
+    uint32_t list_chunk;    // half the shade-list slots a shade wave reserves per atomic at most, 64..kMaxListChunk
     uint32_t shade_sort;    // 1: each shade block takes its 256 paths sorted by shade_class
     uint32_t segments;      // 1, or 8: the trace queue is split in 8 segments, one per XCD
     uint32_t pad1[3];
@@ -443,5 +443,7 @@ struct WavefrontView {
 
 // Largest shade reservations; the queues' headroom is sized for them.
 constexpr uint32_t kMaxQueueChunk = 256u, kMaxListChunk = 256u;
+// List chunks a shade wave reserves at once while many steps lie ahead of it.
+constexpr uint32_t kListScale = 2u;
 
 }  // namespace psx

@@ -42,7 +42,9 @@ uint32_t wavefront_lanes() {
 uint32_t wavefront_queue_headroom() {
     return static_cast<uint32_t>(device_cus()) * kMaxWavesPerCu * kMaxQueueChunk;
 }
-uint32_t wavefront_list_headroom() { return static_cast<uint32_t>(device_cus()) * kMaxWavesPerCu * kMaxListChunk; }
+uint32_t wavefront_list_headroom() {
+    return static_cast<uint32_t>(device_cus()) * kMaxWavesPerCu * kMaxListChunk * kListScale;
+}
 
 // 64 x the tiles of (1 << tile_shift) x (64 >> tile_shift) pixels over the window
 uint32_t wavefront_padded_pixels(const KernelParams &k, uint32_t tile_shift) {

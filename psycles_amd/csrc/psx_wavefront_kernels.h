@@ -241,22 +241,26 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wf_trace_kernel(SceneView s, K
     f3 transmittance = V(1.0f, 1.0f, 1.0f);
     const f3 no_split = V(0.0f, 0.0f, 0.0f);
     // The wave's reservation [res, res_end) of queue entries.  One atomic on
-    // the shared cursor reserves w.trace_chunk entries, which the wave hands to its
+    // the shared cursor reserves `chunk` entries, which the wave hands to its
     // idle lanes over several refills: a returning atomic on one address
     // stalls the whole wave, and claiming per refill made it the largest
     // cost per ray.  `exhausted`: no chunk is left to reserve.
     uint32_t res = 0u, res_end = 0u;
     const uint32_t refill = w.refill;
-    uint32_t chunk = w.trace_chunk;
     // A wave's first reservation is its own by its number, with no atomic:
     // 4096 waves that open with one on the same word take 49 us, the whole
     // time of an iteration with few rays.  A short queue is dealt out evenly
     // in the same way, down to kLeastChunk entries a wave, and then needs no
     // cursor at all.  Neighbouring reservations go to different blocks.
     // Device time of a dispatch: Cornell 256x256x1 1.61 -> 0.60 ms, instanced
-    // 640x400x4 6.2 -> 4.9, Cornell 640x400x16 5.7 -> 4.9.
+    // 640x400x4 6.2 -> 4.9, Cornell 640x400x16 5.7 -> 4.9.  A reservation is
+    // two trace_chunks: the cursor serves one wave in 12 ns, and much larger
+    // ones spread the rays in flight over too much of the scene (device time
+    // at 128, 256 and 1024 entries: instanced frame 86.9, 85.7, 89.5 ms;
+    // Cornell 640x400x16 4.23, 3.89, 3.89).
     const uint32_t waves = gridDim.x * (kTraceBlock / 64u);
     const uint32_t share = (count + waves - 1u) / waves;
+    uint32_t chunk = 2u * w.trace_chunk;
     const uint32_t own = min(chunk, max(share, kLeastChunk));
     const uint32_t dealt = waves * own;
     if (!SEGMENTED) {
@@ -467,7 +471,6 @@ __device__ __forceinline__ void shade_launch(const SceneView &s, const KernelPar
     // in next_list: a returning atomic on the shared counters per step would
     // stall the wave, as it did the trace kernel's refill
     uint32_t q_pos = 0u, q_end = 0u, l_pos = 0u, l_end = 0u;
-    const uint32_t queue_chunk = w.queue_chunk, list_chunk = w.list_chunk;
     __shared__ uint32_t sort_slot[kShadeBlock];
     __shared__ uint32_t sort_count[kShadeKeys];
     const bool sorted = w.shade_sort != 0u;
@@ -532,23 +535,34 @@ __device__ __forceinline__ void shade_launch(const SceneView &s, const KernelPar
         if ((cm | sm) != 0ull) {
             const uint32_t nc = static_cast<uint32_t>(__popcll(cm)), ns = static_cast<uint32_t>(__popcll(sm));
             const uint32_t nq = nc + ns, nl = static_cast<uint32_t>(__popcll(lm));
+            // The next reservation: the entries needed now, and while steps
+            // of the list lie ahead of this wave as many as they may append,
+            // up to a chunk.  A short list then leaves few unused entries for
+            // the next iteration to skip, and a long one takes few turns at
+            // the counters, which serve one wave in 12 ns.  Device time:
+            // Cornell 640x400x16 4.24 -> 3.73 ms, instanced 640x400x4 4.67 ->
+            // 4.24; counting on a quarter of the paths ahead to go on costs
+            // turns (4.22 ms), on twice as many leaves more unused (3.90).
+            const uint32_t ahead = ((count - 1u - base) / stride) * 64u;
             const uint32_t q_old = q_pos, q_avail = q_end - q_pos;
             uint32_t q_new = 0u;
             if (nq > q_avail) {
-                if (lane == 0u) q_new = atomicAdd(&next->trace_count, queue_chunk);
+                const uint32_t size = max(nq - q_avail, min(ahead, w.queue_chunk));
+                if (lane == 0u) q_new = atomicAdd(&next->trace_count, size);
                 q_new = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(q_new)));
                 q_pos = q_new + (nq - q_avail);
-                q_end = q_new + queue_chunk;
+                q_end = q_new + size;
             } else {
                 q_pos += nq;
             }
             const uint32_t l_old = l_pos, l_avail = l_end - l_pos;
             uint32_t l_new = 0u;
             if (nl > l_avail) {
-                if (lane == 0u) l_new = atomicAdd(&next->shade_count, list_chunk);
+                const uint32_t size = max(nl - l_avail, min(ahead, kListScale * w.list_chunk));
+                if (lane == 0u) l_new = atomicAdd(&next->shade_count, size);
                 l_new = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(l_new)));
                 l_pos = l_new + (nl - l_avail);
-                l_end = l_new + list_chunk;
+                l_end = l_new + size;
             } else {
                 l_pos += nl;
             }
