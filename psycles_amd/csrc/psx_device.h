@@ -112,8 +112,10 @@ struct alignas(16) Instance {
     uint32_t override_count;
     float terminator_offset;  // shadow_terminator_geometry_offset
     uint32_t shade_class;     // sort key of the materials it can use, 1..kShadeKeys-1 (0: miss)
-    uint32_t pad[2];
+    uint32_t material;        // of every triangle, or kPerTriangle
+    uint32_t may_smooth;      // 1: some triangles of the mesh can be smooth
 };
+constexpr uint32_t kPerTriangle = 0xfffffffeu;
 
 // Sort keys of shading work: 0 for a miss, then one per closure structure
 // (materials whose closure trees have the same shape run the same code), the
@@ -395,7 +397,7 @@ enum PathWord : uint32_t {
     kPathSource,      // source object, source primitive, flag | visibility << 20 | bits << 25, step
     kPathThroughput,  // xyz, previous BSDF pdf
     kPathIdentity,    // sample, pixel rng hash, bounce | diffuse << 16, glossy | transmission << 16
-    kPathHit,         // instance (kNone = miss), primitive, Cycles primitive, t bits
+    kPathHit,         // instance (kNone = miss), primitive, leaf triangle, t bits
     kPathUv,          // hit u, v, transparent bounces, 0
     kPathMisNormal,   // shading normal of the last non-transparent scatter (scenes with lights)
     kPathWords

@@ -1826,6 +1826,13 @@ int compile(Backend *backend, const psx_scene_desc *d, psx_diag_fn diag, void *d
         g.shade_class = instance_shade_class(src, scene->meshes[mi], slots, material_class);
         overrides.insert(overrides.end(), src.material_overrides, src.material_overrides + src.material_override_count);
         const Mesh &mesh = scene->meshes[mi];
+        g.may_smooth = mesh.smooth_offset != kNone && mesh.normal_offset != kNone ? 1u : 0u;
+        if (mesh.tri_slot_offset != kNone)
+            g.material = kPerTriangle;
+        else if (src.material_override_count > 0u)
+            g.material = src.material_overrides[0];
+        else
+            g.material = mesh.slot_count > 0u ? slots[mesh.slot_offset] : kNone;
         g.applied = users[mi] == 1u ? 1u : 0u;
         float wl[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, wh[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
         bool all_finite = true;

@@ -124,7 +124,8 @@ __device__ __forceinline__ PathVars load_path(const WavefrontView &w, uint32_t i
     h.inst = h.object = bits_of(hv.x);
     h.valid = h.inst != kNone;
     h.prim = bits_of(hv.y);
-    h.cprim = bits_of(hv.z);
+    h.cprim = kNone;  // resolve_surface adds the mesh's offset to `prim`
+    h.tri = bits_of(hv.z);
     h.t = hv.w;
     h.u = uv.x;
     h.v = uv.y;
@@ -379,7 +380,7 @@ __global__ __launch_bounds__(kTraceBlock, 4) void wf_trace_kernel(SceneView s, K
                 float4 *hit = it == 0u ? w.first_hit + path : &path_word(w, path, kPathHit);
                 float2 *uv = it == 0u ? reinterpret_cast<float2 *>(w.albedo + path) + 1
                                       : reinterpret_cast<float2 *>(&path_word(w, path, kPathUv));
-                *hit = bit_words(h.inst, h.prim, h.cprim, __float_as_uint(h.t));
+                *hit = bit_words(h.inst, h.prim, h.tri, __float_as_uint(h.t));
                 *uv = make_float2(h.u, h.v);
                 active = false;
             } else {
