@@ -237,6 +237,24 @@ struct TreeEmitter {
     uint4 identity;  // emitter id, measure flags, 0, 0
 };
 
+// What the importance of a node or emitter depends on, besides the shading
+// point: the terms of its measure that every evaluation repeated (centre, half
+// extent, unit axis, angles compared), computed once per light table with the
+// operations of the evaluation.  A node that is a leaf of one emitter holds
+// that emitter's measure, which is what its importance is.
+constexpr uint32_t kMeasureLive = 1u;     // has an orientation and energy
+constexpr uint32_t kMeasureDistant = 2u;
+constexpr uint32_t kMeasureWide = 4u;     // theta_o + theta_e > pi
+constexpr uint32_t kMeasureNarrow = 8u;   // theta_e < theta_o
+constexpr uint32_t kMeasureLeaf = 16u;
+struct LightMeasure {
+    float4 centre_energy;
+    float4 extent_r2;    // half extent, its square length
+    float4 axis_radius;  // unit cone axis, half the length of the half extent
+    float4 trig;
+    uint4 links;         // kMeasure* bits; inner: left, right; leaf: first, count
+};
+
 // Node of the binary BVH over lamp bounding spheres that the forward-hit
 // search walks: depth-first order, the left child follows its parent, and
 // `miss` is the node after the subtree, so no stack is needed.  `leaf`:
@@ -287,6 +305,8 @@ struct SceneView {
     float light_selection_pdf;        // flat-CDF probability of one lamp
     const TreeNode *tree_nodes;
     const TreeEmitter *tree_emitters;
+    const LightMeasure *node_measures;     // per tree node
+    const LightMeasure *emitter_measures;  // per tree emitter
     const uint2 *tree_mapping;        // emitter id -> (tree emitter, leaf node)
     const uint32_t *emitter_cprim;    // Cycles primitive of each emissive triangle
     uint32_t tree_node_count, tree_emitter_count, tree_root;

@@ -53,6 +53,9 @@ hipError_t launch_sampler(const KernelParams &k, const float4 *sobol, uint32_t s
 hipError_t launch_material_tables(const SceneView &s, float4 *shadow, float4 *emission, uint32_t count,
                                   hipStream_t stream);
 hipError_t launch_instance_opacity(const SceneView &s, uint32_t *flags, uint32_t count, hipStream_t stream);
+hipError_t launch_light_measures(const TreeNode *nodes, uint32_t node_count, const TreeEmitter *emitters,
+                                 uint32_t emitter_count, LightMeasure *node_measures, LightMeasure *emitter_measures,
+                                 hipStream_t stream);
 // psx_query.hip
 uint32_t query_resident_lanes();
 uint32_t query_lanes(uint32_t count, uint32_t max_lanes);
@@ -631,13 +634,15 @@ struct Backend {
 // Light-sampling tables that follow material emission: emitter list, flat
 // CDF, light tree.  Shared by parameter versions whose edits left them valid.
 struct EmitterTables {
-    DeviceBuffer emitters, distribution, tree_nodes, tree_emitters, tree_mapping, emitter_cprim;
+    DeviceBuffer emitters, distribution, tree_nodes, tree_emitters, tree_mapping, emitter_cprim, node_measures,
+        emitter_measures;
     size_t bytes() const {
         return emitters.bytes() + distribution.bytes() + tree_nodes.bytes() + tree_emitters.bytes() +
-               tree_mapping.bytes() + emitter_cprim.bytes();
+               tree_mapping.bytes() + emitter_cprim.bytes() + node_measures.bytes() + emitter_measures.bytes();
     }
     explicit EmitterTables(hipStream_t stream) {
-        for (DeviceBuffer *b : {&emitters, &distribution, &tree_nodes, &tree_emitters, &tree_mapping, &emitter_cprim})
+        for (DeviceBuffer *b : {&emitters, &distribution, &tree_nodes, &tree_emitters, &tree_mapping, &emitter_cprim,
+                                &node_measures, &emitter_measures})
             b->set_stream(stream);
     }
 };
@@ -1030,6 +1035,14 @@ void Scene::rebuild_emitters(ParamTables &t) {
     lt.tree_emitters.upload(tree.emitters);
     lt.tree_mapping.upload(tree.mapping);
     lt.emitter_cprim.upload(cprims);
+    lt.node_measures.allocate(tree.nodes.size() * sizeof(LightMeasure));
+    lt.emitter_measures.allocate(tree.emitters.size() * sizeof(LightMeasure));
+    hip_check(launch_light_measures(lt.tree_nodes.as<TreeNode>(), static_cast<uint32_t>(tree.nodes.size()),
+                                    lt.tree_emitters.as<TreeEmitter>(), static_cast<uint32_t>(tree.emitters.size()),
+                                    lt.node_measures.as<LightMeasure>(), lt.emitter_measures.as<LightMeasure>(),
+                                    table_stream));
+    view.node_measures = lt.node_measures.as<LightMeasure>();
+    view.emitter_measures = lt.emitter_measures.as<LightMeasure>();
     view.tree_nodes = lt.tree_nodes.as<TreeNode>();
     view.tree_emitters = lt.tree_emitters.as<TreeEmitter>();
     view.tree_mapping = lt.tree_mapping.as<uint2>();

@@ -264,6 +264,32 @@ __global__ void material_table_kernel(SceneView s, float4 *shadow, float4 *emiss
 }
 
 
+// the point-independent terms of every light-tree node and emitter
+__global__ void light_measure_kernel(const TreeNode *nodes, uint32_t node_count, const TreeEmitter *emitters,
+                                     uint32_t emitter_count, LightMeasure *node_measures,
+                                     LightMeasure *emitter_measures) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= node_count + emitter_count) return;
+    auto of_emitter = [&](uint32_t e) {
+        const TreeEmitter &t = emitters[e];
+        return light_measure(t.bounds_min_energy, t.bounds_max_theta_o, t.cone_axis_theta_e, t.trig, t.identity.y);
+    };
+    if (i >= node_count) {
+        emitter_measures[i - node_count] = of_emitter(i - node_count);
+        return;
+    }
+    const TreeNode &t = nodes[i];
+    const bool leaf = t.topology.w != kTreeInner;
+    // child_importance (:317-350)
+    LightMeasure m = light_measure(t.bounds_min_energy, t.bounds_max_theta_o, t.cone_axis_theta_e, t.trig, t.emitters.z);
+    if (leaf && t.emitters.y == 1u && t.emitters.x < emitter_count) m = of_emitter(t.emitters.x);
+    if (leaf && t.emitters.y == 0u) m.links.x = 0u;
+    m.links.x |= leaf ? kMeasureLeaf : 0u;
+    m.links.y = leaf ? t.emitters.x : t.topology.y;
+    m.links.z = leaf ? t.emitters.y : t.topology.z;
+    node_measures[i] = m;
+}
+
 // per instance: 1 when every material its triangles can take (the mesh's
 // slot table and the instance's overrides; no slot at all means no material)
 // has no transparent extinction, so any hit on it zeroes a shadow ray
@@ -371,6 +397,16 @@ hipError_t launch_material_tables(const SceneView &s, float4 *shadow, float4 *em
 }
 
 // after launch_material_tables on the same stream (reads s.material_shadow)
+hipError_t launch_light_measures(const TreeNode *nodes, uint32_t node_count, const TreeEmitter *emitters,
+                                 uint32_t emitter_count, LightMeasure *node_measures, LightMeasure *emitter_measures,
+                                 hipStream_t stream) {
+    const uint32_t n = node_count + emitter_count;
+    if (n == 0u) return hipSuccess;
+    hipLaunchKernelGGL(light_measure_kernel, dim3((n + 63u) / 64u), dim3(64), 0, stream, nodes, node_count, emitters,
+                       emitter_count, node_measures, emitter_measures);
+    return hipGetLastError();
+}
+
 hipError_t launch_instance_opacity(const SceneView &s, uint32_t *flags, uint32_t count, hipStream_t stream) {
     if (count == 0u) return hipSuccess;
     hipLaunchKernelGGL(instance_opacity_kernel, dim3((count + 63u) / 64u), dim3(64), 0, stream, s, flags, count);
