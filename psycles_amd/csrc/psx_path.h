@@ -466,13 +466,13 @@ struct Traversal {
     // stack level at which the current instance was entered, 0 in the world,
     // kStale when the stack is back in the world and o and d still an instance's
     int base;
-    // Any-hit traversal (ANYHIT, for shadow queries) ends at the first
+    // Any-hit traversal (ANYHIT and `any`, for shadow queries) ends at the first
     // accepted candidate on an instance whose every material is opaque to
     // shadow rays (`stop` while inside such an instance; `opaque` once
     // ended): the transparent shadow loop's transmittance is then exactly
     // zero whatever else lies on the ray, so the early end changes no result
     // bit.
-    bool stop, opaque;
+    bool any, stop, opaque;
 };
 constexpr int kStale = -1;
 
@@ -643,7 +643,7 @@ __device__ __forceinline__ void traversal_leaf(const SceneView &s, Traversal &t,
     st.set_word(kColdHit + 1u, prim);
     st.set_word(kColdHit + 2u, cprim);
     st.set_word(kColdHit + 3u, first);
-    if (ANYHIT && (world ? s.instance_opaque[inst] != 0u : t.stop)) {
+    if (ANYHIT && t.any && (world ? s.instance_opaque[inst] != 0u : t.stop)) {
         // any opaque candidate in [tmin, tmax] zeroes the shadow
         t.opaque = true;
         traversal_idle(t, st);
@@ -715,13 +715,12 @@ __device__ __forceinline__ void traversal_advance(const SceneView &s, Traversal 
     if (node && !run_change && !run_leaf) traversal_node<COUNT>(s, t, st, node_count);
 }
 
-template <bool COUNT, bool ANYHIT = false>
+template <bool COUNT>
 __device__ Hit closest_hit(const SceneView &s, const Ray &ray, const TraceQuery &q, Stack &st,
-                           uint32_t &node_count, uint32_t &tri_count, bool *opaque = nullptr) {
+                           uint32_t &node_count, uint32_t &tri_count) {
     Traversal t;
     traversal_begin(s, t, st, ray, q);
-    while (traversal_busy(t, st)) traversal_advance<COUNT, ANYHIT>(s, t, st, node_count, tri_count);
-    if (opaque) *opaque = t.opaque;
+    while (traversal_busy(t, st)) traversal_advance<COUNT>(s, t, st, node_count, tri_count);
     return traversal_result(t, st);
 }
 

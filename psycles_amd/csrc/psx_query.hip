@@ -4,8 +4,9 @@
 // with the render path's own traversal: closest hits under the Cycles order
 // and the transparent shadow loop, whose any-hit traversal ends at the first
 // candidate on an instance opaque to shadow rays.  Waves
-// take 64 queries per atomic from a cursor; each lane keeps its stack in an
-// LDS short stack with an HBM spill column, like the trace kernels.
+// take 64 queries at a time and hand them to the lanes that are done; each lane
+// keeps its stack in an LDS short stack with an HBM spill column, like the
+// trace kernels.
 //
 // probe_kernel evaluates one device function per input record, so tests can
 // hold the device code itself against the reference's function fixtures.
@@ -26,70 +27,118 @@ __global__ void clear_words_kernel(uint32_t *p, uint32_t n) {
     if (i < n) p[i] = 0u;
 }
 
-__device__ void run_query(const SceneView &s, const psx_ray_query &q, Stack &st, psx_ray_hit &h) {
-    Ray r;
-    r.o = V(q.origin[0], q.origin[1], q.origin[2]);
-    r.d = V(q.direction[0], q.direction[1], q.direction[2]);
-    r.tmin = q.tmin;
-    r.tmax = q.tmax;
-    TraceQuery tq;
-    tq.visibility = q.visibility;
-    tq.src_obj = q.source_object;
-    tq.src_prim = q.source_primitive;
-    tq.light_obj = q.light_object;
-    tq.light_prim = q.light_primitive;
-    uint32_t nodes = 0u, tris = 0u;
-    h.u = h.v = 0.0f;
-    h.reserved = h.reserved2 = 0u;
-    if (q.kind == PSX_QUERY_SHADOW) {
-        f3 transmittance = V(1.0f, 1.0f, 1.0f);
-        uint32_t tdepth = q.transparent_depth, passes = 0u;
-        for (;;) {
-            bool opaque = false;
-            const Hit b = closest_hit<false, true>(s, r, tq, st, nodes, tris, &opaque);
-            ++passes;
-            if (shadow_hit(s, q.transparent_max, b, r, tdepth, transmittance, opaque)) break;
-        }
-        h.t = q.tmax;
-        h.object = h.primitive = PSX_INVALID_ID;
-        h.hit = (transmittance.x > 0.0f || transmittance.y > 0.0f || transmittance.z > 0.0f) ? 0u : 1u;
-        h.traversals = passes;
-        h.transmittance[0] = transmittance.x;
-        h.transmittance[1] = transmittance.y;
-        h.transmittance[2] = transmittance.z;
-    } else {
-        const Hit b = closest_hit<false>(s, r, tq, st, nodes, tris);
-        h.hit = b.valid ? 1u : 0u;
-        h.t = b.valid ? b.t : q.tmax;
-        h.u = b.valid ? b.u : 0.0f;
-        h.v = b.valid ? b.v : 0.0f;
-        h.object = b.valid ? b.object : PSX_INVALID_ID;
-        h.primitive = b.valid ? b.cprim : PSX_INVALID_ID;
-        h.traversals = 1u;
-        h.transmittance[0] = h.transmittance[1] = h.transmittance[2] = 0.0f;
-    }
-}
+// Queries a wave reserves at a time (32: 16 % slower at 2^21 queries, one
+// atomic each 12 ns; 128: fewer waves at work on 4096, 15 % slower), and its
+// idle lanes that call for new ones (8 and 32 measured the same).
+constexpr uint32_t kQueryChunk = 64u;
+constexpr uint32_t kQueryRefill = 16u;
 
-// `cursor` (one word, zero at launch) hands out 64 queries per wave; `spill`
-// holds kTraversalStackDepth words per lane of the grid.
-__global__ __launch_bounds__(kQueryBlock) void intersect_kernel(SceneView s, const psx_ray_query *queries,
-                                                                uint32_t count, psx_ray_hit *hits, uint32_t *cursor,
-                                                                uint32_t *spill) {
+// `cursor` (one word, zero at launch) hands out the queries beyond each wave's
+// own first ones; `spill` holds kTraversalStackDepth words per lane of the
+// grid.
+//
+// What bounds it is VALU issue, then random fetches.  A lane takes the next
+// query when its own is answered, and closest hits and shadow queries run in
+// one traversal.  When a wave answered 64 queries at a time, first their
+// closest hits and then their shadows, it waited for its longest ray of either
+// kind.  A call with 2^21 random queries, half of them shadows, on the
+// instanced scene (64 spheres of 1.0 M triangles): 5.7 -> 2.2 ms; 30000 from
+// host memory: 360 -> 325 us, 4096: 196 -> 181, 500: 167 -> 153.
+__global__ __launch_bounds__(kQueryBlock, 4) void intersect_kernel(SceneView s, const psx_ray_query *queries,
+                                                                   uint32_t count, psx_ray_hit *hits,
+                                                                   uint32_t *cursor, uint32_t *spill) {
     __shared__ uint32_t lds[kTraversalLds * kQueryBlock];
     Stack st = make_stack(lds, spill, kQueryBlock, threadIdx.x, blockIdx.x * kQueryBlock + threadIdx.x,
                           gridDim.x * kQueryBlock);
     const uint32_t lane = __lane_id();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    uint32_t nodes = 0u, tris = 0u;
+    Traversal t;
+    traversal_idle(t, st);
+    t.any = false;
+    bool active = false, shadow = false;
+    uint32_t at = 0u, tdepth = 0u, transparent_max = 0u, passes = 0u;
+    f3 transmittance = V(1.0f, 1.0f, 1.0f);
+    // the wave's reservation [res, res_end): first its own, by its number, so
+    // that a launch does not open with an atomic of every wave on one word
+    const uint32_t waves = gridDim.x * (kQueryBlock / 64u);
+    const uint32_t dealt = waves * kQueryChunk;
+    const uint32_t first = ((threadIdx.x >> 6) * gridDim.x + blockIdx.x) * kQueryChunk;
+    uint32_t res = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(first < count ? first : count)));
+    uint32_t res_end = count - res > kQueryChunk ? res + kQueryChunk : count;
+    bool exhausted = dealt >= count;
     for (;;) {
-        uint32_t base = 0u;
-        if (lane == 0u) base = atomicAdd(cursor, 64u);
-        base = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(base)));
-        if (base >= count) break;
-        const uint32_t i = base + lane;
-        if (i < count) {
-            const psx_ray_query q = queries[i];
-            psx_ray_hit h;
-            run_query(s, q, st, h);
-            hits[i] = h;
+        if (!exhausted || res < res_end) {
+            const unsigned long long idle = __ballot(!active);
+            const uint32_t want = static_cast<uint32_t>(__popcll(idle));
+            if (res == res_end && !exhausted && want > 0u) {
+                const uint32_t leader = static_cast<uint32_t>(__ffsll(static_cast<long long>(idle)) - 1);
+                uint32_t b = 0u;
+                if (lane == leader) b = dealt + atomicAdd(cursor, kQueryChunk);
+                b = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(b), static_cast<int>(leader)));
+                if (b < count) {
+                    res = b;
+                    res_end = count - b > kQueryChunk ? b + kQueryChunk : count;
+                }
+                exhausted = b >= count || count - b <= kQueryChunk;
+            }
+            const uint32_t avail = res_end - res;
+            const uint32_t rank = static_cast<uint32_t>(__popcll(idle & below));
+            const uint32_t next = res + rank;
+            res += want < avail ? want : avail;
+            if (!active && rank < avail) {
+                at = next;
+                const psx_ray_query q = queries[at];
+                shadow = q.kind == PSX_QUERY_SHADOW;
+                tdepth = q.transparent_depth;
+                transparent_max = q.transparent_max;
+                passes = 0u;
+                transmittance = V(1.0f, 1.0f, 1.0f);
+                traversal_begin(s, t, st,
+                                Ray{V(q.origin[0], q.origin[1], q.origin[2]),
+                                    V(q.direction[0], q.direction[1], q.direction[2]), q.tmin, q.tmax},
+                                TraceQuery{q.visibility, q.source_object, q.source_primitive, q.light_object,
+                                           q.light_primitive});
+                t.any = shadow;
+                active = true;
+            }
+        }
+        const unsigned long long owned = __ballot(active);
+        if (owned == 0ull) {
+            if (exhausted && res == res_end) break;
+            continue;
+        }
+        // with nothing left to take, until half of the owned lanes are done,
+        // so that shadows past a transparent surface go on
+        const uint32_t busy_min = !exhausted || res < res_end ? 64u - kQueryRefill
+                                                              : static_cast<uint32_t>(__popcll(owned)) >> 1u;
+        do {
+            traversal_advance<false, true>(s, t, st, nodes, tris);
+        } while (static_cast<uint32_t>(__popcll(__ballot(traversal_busy(t, st)))) > busy_min);
+        if (active && !traversal_busy(t, st)) {
+            const Hit b = traversal_result(t, st);
+            ++passes;
+            Ray rest;
+            if (shadow && !shadow_hit(s, transparent_max, b, rest, tdepth, transmittance, t.opaque)) {
+                traversal_resume(s, t, st, rest.tmin);
+            } else {
+                const bool found = !shadow && b.valid;
+                const bool lit = transmittance.x > 0.0f || transmittance.y > 0.0f || transmittance.z > 0.0f;
+                psx_ray_hit h;
+                h.t = found ? b.t : st.number(kColdTmax);
+                h.u = found ? b.u : 0.0f;
+                h.v = found ? b.v : 0.0f;
+                h.object = found ? b.object : PSX_INVALID_ID;
+                h.primitive = found ? b.cprim : PSX_INVALID_ID;
+                h.hit = shadow ? !lit : found;
+                h.traversals = passes;
+                h.reserved = h.reserved2 = 0u;
+                h.transmittance[0] = shadow ? transmittance.x : 0.0f;
+                h.transmittance[1] = shadow ? transmittance.y : 0.0f;
+                h.transmittance[2] = shadow ? transmittance.z : 0.0f;
+                hits[at] = h;
+                active = false;
+            }
         }
     }
 }

@@ -6,6 +6,7 @@ others are inside one, single-user meshes in and outside the world tree,
 rays with NaN.  Closest hits identical, shadow
 transmittance bit-identical.
 """
+import ctypes as C
 import sys
 
 import numpy as np
@@ -138,3 +139,38 @@ def test_short_queues(width, height, spp):
         scene.close()
         backend.close()
     assert films[0] == films[1]
+
+
+@pytest.mark.parametrize("n", [1, 65, 4099, 300001])
+@pytest.mark.parametrize("name", sorted(SCENES))
+def test_mixed_queries(name, n):
+    """Closest hits and shadows in one call, from one query to more than the
+    waves of a full launch reserve at first (262144): every word of every hit
+    is the oracle's, also where a lane answers several queries in turn."""
+    print(f"case: mixed queries of {name}, {n} queries", flush=True)
+    make, reach = SCENES[name]
+    snap = make()
+    backend = RendererBackend(0)
+    dev = backend.compile_scene(snap).scene
+    ora = ob.OracleScene(snap)
+    some = [q for pair in zip(queries(300, reach, 5, abi.QUERY_CLOSEST), queries(300, reach, 6, abi.QUERY_SHADOW))
+            for q in pair]
+    rng = np.random.RandomState(n)
+    for q in some:
+        q["transparent_max"] = int(rng.choice([0, 1, 2, 40]))
+        q["transparent_depth"] = int(rng.choice([0, 1]))
+    want = np.frombuffer((abi.RayHit * len(some))(*ora.intersect(some)), np.uint32).reshape(-1, 12)
+    records = np.frombuffer(abi.make_queries(some), np.uint32).reshape(-1, 16)
+    pick = rng.randint(0, len(some), n)
+    sent = np.ascontiguousarray(records[pick])
+    got = np.full((n, 12), 0xABABABAB, np.uint32)
+    lib = backend.lib
+    assert lib.psx_scene_intersect(dev.handle, sent.ctypes.data_as(C.POINTER(abi.RayQuery)), n,
+                                   got.ctypes.data_as(C.POINTER(abi.RayHit))) == 0
+    shadows = records[pick, 13] == abi.QUERY_SHADOW
+    words = [w for w in range(12) if w != 6]  # an early end of a shadow query saves traversals
+    assert np.array_equal(got[:, words], want[pick][:, words])
+    assert np.array_equal(got[~shadows, 6], want[pick][~shadows, 6])
+    assert (got[shadows, 6] >= 1).all() and (got[shadows, 6] <= want[pick][shadows, 6]).all()
+    dev.close()
+    backend.close()
