@@ -1,4 +1,5 @@
-// psx_bvh.cpp - host builder of the two-level BVH4.
+// psx_bvh.cpp - host builder of the BVH4s: the world tree (instances and the
+// triangles of single-user meshes) and one tree per shared mesh.
 //
 // Replaces the acceleration structure the reference obtains from
 // LuisaCompute's Accel (device.create_mesh / accel.emplace_back /

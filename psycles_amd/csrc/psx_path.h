@@ -1,8 +1,8 @@
 // psx_path.h - device code of the MI355X render path shared by the
 // megakernel and the wavefront integrator (gfx950).
 //
-// Camera rays, two-level BVH4 traversal with an LDS short stack and the exact
-// Cycles closest-hit contract, closure-tree shading, emissive-triangle NEE
+// Camera rays, traversal of a world tree and its instances' trees (BVH4) with
+// an LDS short stack and the exact Cycles closest-hit contract, closure-tree shading, emissive-triangle NEE
 // with transparent shadows, Russian roulette and the path step.  Each stage
 // cites the reference file whose behaviour it reproduces.
 //

@@ -5,16 +5,17 @@
 //
 //   trace  persistent waves run closest-hit traversal for continuation rays,
 //          or the whole transparent shadow loop for NEE shadow rays; lanes
-//          whose query finished are refilled from the queue (one atomic per
-//          refill) while the rest of the wave keeps traversing
-//   shade  consumes the hit of each live path: pending shadow result, then one
-//          path step (emission, RR, AOVs, NEE sampling, BSDF sampling); new
-//          rays are appended to the next queue with one atomic per wave
-//          (ballot + prefix count)
+//          whose query finished are refilled from the wave's reservation of
+//          the queue (its first one without an atomic, then one atomic each)
+//          while the rest of the wave keeps traversing
+//   shade  consumes the hit of each live path: one path step (emission, RR,
+//          AOVs, NEE sampling, BSDF sampling); new rays are appended to the
+//          next queue with one atomic per reservation (ballot + prefix count)
 //
-// Shadow results are applied at the start of the next shade, before that
-// step's emission, which is the order in which the megakernel adds them, and a
-// final pass adds each pixel's samples in sample order; the film is therefore
+// The trace kernel adds a shadow ray's light to its path's radiance, between
+// the shade step that sent it and the next one, which is the order in which
+// the megakernel adds it (with light passes the next shade step does, which
+// splits it), and a final pass adds each pixel's samples in sample order; the film is therefore
 // bit-identical to the megakernel's.  Queue counts live in device memory, so
 // the host enqueues all iterations without synchronising; an empty iteration
 // costs two near-empty launches.
