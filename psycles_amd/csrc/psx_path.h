@@ -2331,8 +2331,8 @@ __device__ __forceinline__ TreeImportance lt_importance(const LightMeasure &m, f
         if (!(has_transmission || dot(n, delta) + dot(V(fabsf(n.x), fabsf(n.y), fabsf(n.z)), extent) > 0.0f)) return r;
         const float d2 = dot(delta, delta);
         // distances and sizes for which the short operations hold: all but
-        // degenerate scenes
-        const bool usual = d2 > LT_SAFE && d2 < 0x1p60f && r2 < 0x1p60f && (r2 > 0x1p-40f || r2 == 0.0f);
+        // degenerate scenes (a lamp without extent may be nearer than 2^-30)
+        const bool usual = d2 >= 0x1p-60f && d2 < 0x1p60f && r2 < 0x1p60f && (r2 > 0x1p-40f || r2 == 0.0f);
         float ratio, inverse;
         if (usual) {
             distance = lt_root(d2);

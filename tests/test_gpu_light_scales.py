@@ -61,3 +61,42 @@ def test_light_choice(scale, flat):
     session.close()
     scene.close()
     backend.close()
+
+
+def lamps_over_floor(scale):
+    """A floor under 24 point lamps without extent, the nearest of them at
+    half a scale: their square distances span a factor of 64."""
+    rng = np.random.RandomState(4)
+    p, t = scenes.quad([[-1, 0, -1], [-1, 0, 1], [1, 0, 1], [1, 0, -1]])
+    floor = scenes.MeshData((p * scale).astype(np.float32), t, [0])
+    camera = scenes.CameraData(scenes.look_at((0.0, 2.0 * scale, 2.5 * scale), (0.0, 0.0, 0.0)), math.radians(50.0),
+                               1.0e-3 * scale, 100.0 * scale)
+    snap = scenes.SceneSnapshot([scenes.diffuse_material((0.7, 0.7, 0.7))], [floor],
+                                [scenes.InstanceData(0, scenes.identity())], camera, name="lamps over a floor")
+    snap.lights = [scenes.lamp(abi.LIGHT_POINT, scenes.translation(*(scale * np.array([x, y, z]))), power=3.0, size=0.0)
+                   for x, y, z in rng.uniform((-1, 0.5, -1), (1, 3.0, 1), (24, 3))]
+    return snap
+
+
+# square distances of 2^-60 lie within the second to fourth of these
+@pytest.mark.parametrize("scale", [2.0e-10, 3.0e-10, 6.0e-10, 1.0e-9, 3.0e-9])
+def test_light_choice_at_the_least_distances(scale):
+    print(f"case: light choice over lamps at scale {scale}", flush=True)
+    snap = lamps_over_floor(scale)
+    s = scenes.many_light_settings(72, 48)
+    backend = RendererBackend(0)
+    scene = backend.compile_scene(snap).scene
+    session = backend.create_session(scene, s)
+    oracle = ob.OracleScene(snap)
+    chosen = set()
+    for sample in (0, 5):
+        a = session.trace_events(sample, 16)[:, :, 0]
+        b = oracle.trace_events(s, sample, 16)[:, :, 0]
+        for word in (abi.TRACE_FLAGS, abi.TRACE_OBJECT, abi.TRACE_PRIMITIVE, abi.TRACE_LIGHT):
+            assert np.array_equal(a[..., word] & 31 if word == abi.TRACE_FLAGS else a[..., word],
+                                  b[..., word] & 31 if word == abi.TRACE_FLAGS else b[..., word]), word
+        chosen |= set(np.unique(b[..., abi.TRACE_LIGHT]).tolist())
+    assert len(chosen) > 10
+    session.close()
+    scene.close()
+    backend.close()
