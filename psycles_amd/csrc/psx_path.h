@@ -509,9 +509,9 @@ __device__ __forceinline__ void traversal_start(const SceneView &s, Traversal &t
     t.stop = t.opaque = false;
     traversal_space(t, o, d);
     traversal_idle(t, st);
-    // a NaN anywhere in the ray fails every triangle test: nothing to search
-    const bool nan = __builtin_isunordered(o.x, d.x) || __builtin_isunordered(o.y, d.y) ||
-                     __builtin_isunordered(o.z, d.z) || __builtin_isunordered(tmin, tmax);
+    // a NaN in the origin or the range fails every triangle test: nothing to
+    // search.  In the direction it does not: clamp_bvh_dir makes it finite.
+    const bool nan = __builtin_isunordered(o.x, o.y) || __builtin_isunordered(o.z, tmin) || tmax != tmax;
     if (s.has_tlas && !nan) t.cur = s.tlas_root;
 }
 

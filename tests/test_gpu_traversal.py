@@ -174,3 +174,32 @@ def test_mixed_queries(name, n):
     assert (got[shadows, 6] >= 1).all() and (got[shadows, 6] <= want[pick][shadows, 6]).all()
     dev.close()
     backend.close()
+
+
+@pytest.mark.parametrize("kind", [abi.QUERY_CLOSEST, abi.QUERY_SHADOW])
+def test_directions_with_nan(kind):
+    """A NaN in a direction is the smallest direction of its sign in that
+    component, as the clamp of the reference leaves it: the ray is searched."""
+    print(f"case: NaN directions, kind {kind}", flush=True)
+    snap = heap_scene()
+    rays = queries(600, 1.5, 31, kind)
+    nan = float("nan")
+    for i, q in enumerate(rays):
+        d = [float(c) for c in q["direction"]]
+        for axis in ((0,), (1,), (2,), (0, 2), (0, 1, 2))[i % 5]:
+            d[axis] = nan
+        q["direction"] = d
+        q["tmax"] = 1.0e30 if i % 5 == 4 else 100.0
+        q["tmin"] = 0.0
+        if kind == abi.QUERY_CLOSEST:
+            q["visibility"] = abi.VIS_ALL
+    backend = RendererBackend(0)
+    dev = backend.compile_scene(snap).scene
+    want = ob.OracleScene(snap).intersect(rays)
+    assert 0 < sum(h.hit for h in want)
+    for x, y in zip(dev.intersect(rays), want):
+        assert (x.hit, x.object, x.primitive) == (y.hit, y.object, y.primitive)
+        assert np.float32([x.t, x.u, x.v, *x.transmittance]).tobytes() == \
+            np.float32([y.t, y.u, y.v, *y.transmittance]).tobytes()
+    dev.close()
+    backend.close()
