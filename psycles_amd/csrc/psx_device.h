@@ -310,6 +310,10 @@ struct SceneView {
     const uint2 *tree_mapping;        // emitter id -> (tree emitter, leaf node)
     const uint32_t *emitter_cprim;    // Cycles primitive of each emissive triangle
     uint32_t tree_node_count, tree_emitter_count, tree_root;
+    // Instance boxes allow for the rounding of rays into object space from
+    // origins up to box_reach in every coordinate; beyond it, box tests need
+    // far_slack times the largest coordinate on every side.
+    float box_reach, far_slack;
     uint32_t tlas_root;
     uint32_t instance_count;
     uint32_t material_count;

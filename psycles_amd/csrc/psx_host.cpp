@@ -1807,10 +1807,19 @@ int compile(Backend *backend, const psx_scene_desc *d, psx_diag_fn diag, void *d
         depth = b.depth;
     };
     scene->overrides.resize(d->instance_count);
-    float reach[3];  // largest coordinate that rays of the scene start from or arrive at
-    for (int a = 0; a < 3; ++a) {
-        const float eye = d->camera.transform[12 + a];
-        reach[a] = std::isfinite(eye) ? std::fabs(eye) : 0.0f;
+    // largest coordinate that rays of the scene start from or arrive at: the
+    // camera's, with its near clip and the extent of an orthographic view
+    // plane, and those of the geometry (below)
+    float reach = 0.0f;
+    {
+        const psx_camera &cam = d->camera;
+        const float shift = std::max(std::fabs(cam.lens_shift_x), std::fabs(cam.lens_shift_y));
+        const float plane = cam.projection == 1u ? std::fabs(cam.orthographic_scale) * (1.0f + 2.0f * shift) : 0.0f;
+        for (int a = 0; a < 3; ++a) {
+            const float eye = std::fabs(cam.transform[12 + a]) + std::fabs(cam.near_clip) +
+                              plane * (std::fabs(cam.transform[a]) + std::fabs(cam.transform[4 + a]));
+            if (std::isfinite(eye)) reach = std::max(reach, eye);
+        }
     }
     std::vector<uint8_t> finite(d->instance_count, 0u);  // instances with triangles and finite world positions
     for (uint32_t i = 0; i < d->instance_count; ++i) {
@@ -1886,10 +1895,24 @@ int compile(Backend *backend, const psx_scene_desc *d, psx_diag_fn diag, void *d
         }
         finite[i] = all_finite && mesh.triangle_count > 0u ? 1u : 0u;
         if (finite[i])
-            for (int a = 0; a < 3; ++a) reach[a] = std::max(reach[a], std::max(std::fabs(wl[a]), std::fabs(wh[a])));
+            for (int a = 0; a < 3; ++a) reach = std::max(reach, std::max(std::fabs(wl[a]), std::fabs(wh[a])));
         instances.push_back(g);
         scene->triangles += mesh.triangle_count;
     }
+    // Rounding moves a ray on its way into an instance's object space by up to
+    // 8 ulps of each term, seen in the world (rounding_gain times the largest
+    // coordinate of its origin).  The instance boxes allow for the rays of the
+    // scene, with room for view planes of any usual aspect; query kernels
+    // allow for origins further out (far_margin).
+    const double box_reach = std::min(16.0 * static_cast<double>(reach), static_cast<double>(FLT_MAX));
+    double far_slack = 0.0;
+    auto rounding_gain = [](const float *m, const Affine &w2o, int a) {
+        double gain = 1.0;
+        for (int o = 0; o < 3; ++o)
+            for (int w = 0; w < 3; ++w)
+                gain += std::fabs(static_cast<double>(m[4 * o + a])) * std::fabs(static_cast<double>(w2o.m[3 * w + o]));
+        return gain * 1.0e-6;
+    };
     // World tree: triangles of single-user meshes and one leaf per instance.
     // `merge` = false keeps a tree and an entry per single-user mesh, for
     // scenes whose merged tree would be too deep for the traversal stack.
@@ -1905,6 +1928,7 @@ int compile(Backend *backend, const psx_scene_desc *d, psx_diag_fn diag, void *d
         };
         std::vector<Owner> owners;
         max_blas_depth = 0;
+        far_slack = 0.0;
         for (uint32_t i = 0; i < d->instance_count; ++i) {
             const psx_instance &src = d->instances[i];
             const uint32_t mi = src.mesh, tcount = scene->meshes[mi].triangle_count;
@@ -1928,20 +1952,20 @@ int compile(Backend *backend, const psx_scene_desc *d, psx_diag_fn diag, void *d
             } else {
                 max_blas_depth = std::max(max_blas_depth, shared_depth[mi]);
                 float wl[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, wh[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-                if (finite[i]) {
+                double gain[3];
+                bool tight = finite[i] != 0u;
+                for (int a = 0; a < 3; ++a) {
+                    gain[a] = rounding_gain(src.transform, g.w2o, a);
+                    // not finite for a transform without an inverse
+                    tight &= gain[a] * box_reach < static_cast<double>(FLT_MAX);
+                }
+                if (tight) {
                     double tl[3], th[3];
                     transformed_bounds(nodes, tris, g.blas_root, src.transform, tl, th);
                     for (int a = 0; a < 3; ++a) {
-                        // what rounding can move a ray by on its way into
-                        // object space, seen in the world (8 ulps of each term)
-                        double slack = 0.0;
-                        for (int o = 0; o < 3; ++o)
-                            for (int w = 0; w < 3; ++w)
-                                slack += std::fabs(static_cast<double>(src.transform[4 * o + a])) *
-                                         std::fabs(static_cast<double>(g.w2o.m[3 * w + o])) * reach[w];
-                        slack = (slack + reach[a]) * 1.0e-6;
-                        wl[a] = static_cast<float>(tl[a] - slack);
-                        wh[a] = static_cast<float>(th[a] + slack);
+                        wl[a] = static_cast<float>(tl[a] - gain[a] * box_reach);
+                        wh[a] = static_cast<float>(th[a] + gain[a] * box_reach);
+                        far_slack = std::max(far_slack, gain[a]);
                     }
                 } else {
                     for (int c = 0; c < 8; ++c) {
@@ -2054,6 +2078,8 @@ int compile(Backend *backend, const psx_scene_desc *d, psx_diag_fn diag, void *d
     v.leaves = s.leaves.as<Leaf>();
     v.tlas_root = 0u;
     v.has_tlas = has_tlas ? 1u : 0u;
+    v.box_reach = static_cast<float>(box_reach);
+    v.far_slack = static_cast<float>(std::min(far_slack, static_cast<double>(FLT_MAX)));
     v.instance_count = d->instance_count;
     v.material_count = d->material_count;
     // background lights fold into the constant world radiance

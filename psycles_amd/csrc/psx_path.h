@@ -473,6 +473,7 @@ struct Traversal {
     // zero whatever else lies on the ray, so the early end changes no result
     // bit.
     bool any, stop, opaque;
+    float margin;  // FAR traversals only: what box tests are widened by
 };
 constexpr int kStale = -1;
 
@@ -533,6 +534,13 @@ __device__ __forceinline__ void traversal_resume(const SceneView &s, Traversal &
     traversal_start(s, t, st, st.vec(kColdOrigin), st.vec(kColdDirection), tmin, st.number(kColdTmax));
 }
 
+// Margin of a ray from any origin: none where the boxes allow for its rounding
+// (every ray of a render; most ray queries), else in proportion.
+__device__ __forceinline__ float far_margin(const SceneView &s, f3 o) {
+    const float m = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z));
+    return m > s.box_reach ? m * s.far_slack : 0.0f;
+}
+
 __device__ __forceinline__ bool traversal_busy(const Traversal &t, const Stack &st) {
     return (t.cur & t.leaf) != kEmptySlot || st.sp > 0;
 }
@@ -554,8 +562,8 @@ __device__ __forceinline__ Hit traversal_result(const Traversal &t, const Stack 
 }
 
 // the four child boxes of a node: continue with the nearest hit child, push
-// the others far to near
-template <bool COUNT>
+// the others far to near; FAR widens them by t.margin
+template <bool COUNT, bool FAR>
 __device__ __forceinline__ void traversal_node(const SceneView &s, Traversal &t, Stack &st, uint32_t &node_count) {
     const uint4 *rec = reinterpret_cast<const uint4 *>(s.nodes + (t.cur & ~kKindMask));
     const uint4 head = rec[0], qxy = rec[1], qz = rec[2], refs = rec[3];
@@ -566,6 +574,12 @@ __device__ __forceinline__ void traversal_node(const SceneView &s, Traversal &t,
     const float bx = fmaf(__uint_as_float(head.x), t.inv.x, -t.oi.x);
     const float by = fmaf(__uint_as_float(head.y), t.inv.y, -t.oi.y);
     const float bz = fmaf(__uint_as_float(head.z), t.inv.z, -t.oi.z);
+    f3 b0 = V(bx, by, bz), b1 = b0;
+    if (FAR) {
+        const f3 m = V(t.margin * fabsf(t.inv.x), t.margin * fabsf(t.inv.y), t.margin * fabsf(t.inv.z));
+        b0 = b0 - m;
+        b1 = b1 + m;
+    }
     const uint32_t ref_arr[4] = {refs.x, refs.y, refs.z, refs.w};
     // Per axis, the plane nearer along the ray: the scale has the sign of
     // the inverse direction, lo <= hi, and fma rounds monotonically, so
@@ -583,12 +597,12 @@ __device__ __forceinline__ void traversal_node(const SceneView &s, Traversal &t,
         // magnitude before quantisation, which rounds outward, and the far end
         // is widened by 1e-5, all far above the rounding of these slab terms
         const int sh = 8 * i;
-        const float t0x = fmaf(static_cast<float>((nx >> sh) & 0xffu), sx, bx);
-        const float t1x = fmaf(static_cast<float>((fx >> sh) & 0xffu), sx, bx);
-        const float t0y = fmaf(static_cast<float>((ny >> sh) & 0xffu), sy, by);
-        const float t1y = fmaf(static_cast<float>((fy >> sh) & 0xffu), sy, by);
-        const float t0z = fmaf(static_cast<float>((nz >> sh) & 0xffu), sz, bz);
-        const float t1z = fmaf(static_cast<float>((fz >> sh) & 0xffu), sz, bz);
+        const float t0x = fmaf(static_cast<float>((nx >> sh) & 0xffu), sx, b0.x);
+        const float t1x = fmaf(static_cast<float>((fx >> sh) & 0xffu), sx, b1.x);
+        const float t0y = fmaf(static_cast<float>((ny >> sh) & 0xffu), sy, b0.y);
+        const float t1y = fmaf(static_cast<float>((fy >> sh) & 0xffu), sy, b1.y);
+        const float t0z = fmaf(static_cast<float>((nz >> sh) & 0xffu), sz, b0.z);
+        const float t1z = fmaf(static_cast<float>((fz >> sh) & 0xffu), sz, b1.z);
         const float near = fmaxf(fmaxf(fmaxf(t0x, t0y), t0z), t.lower);
         const float far = fminf(fminf(fminf(t1x, t1y), t1z), t.best_t);
         const uint32_t ref = ref_arr[i];
@@ -685,7 +699,7 @@ __device__ __forceinline__ void traversal_change_space(const SceneView &s, Trave
 // three kinds are three predicated blocks in a row, not branches: as branches
 // the compiler copied the ray's registers around each of them (17 moves a
 // step).
-template <bool COUNT, bool ANYHIT = false>
+template <bool COUNT, bool ANYHIT = false, bool FAR = false>
 __device__ __forceinline__ void traversal_advance(const SceneView &s, Traversal &t, Stack &st, uint32_t &node_count,
                                                   uint32_t &tri_count) {
     // set a leaf aside, then take the next entry from the stack; as signed
@@ -712,7 +726,12 @@ __device__ __forceinline__ void traversal_advance(const SceneView &s, Traversal 
     const bool run_leaf = !run_change && n_leaf >= n_node;
     if (changes && run_change) traversal_change_space<ANYHIT>(s, t, st);
     if (leaf && run_leaf) traversal_leaf<COUNT, ANYHIT>(s, t, st, tri_count);
-    if (node && !run_change && !run_leaf) traversal_node<COUNT>(s, t, st, node_count);
+    if (node && !run_change && !run_leaf) {
+        if (FAR && __builtin_amdgcn_ballot_w64(t.margin > 0.0f) != 0ull)
+            traversal_node<COUNT, true>(s, t, st, node_count);
+        else
+            traversal_node<COUNT, false>(s, t, st, node_count);
+    }
 }
 
 template <bool COUNT>

@@ -56,6 +56,7 @@ __global__ __launch_bounds__(kQueryBlock, 4) void intersect_kernel(SceneView s, 
     Traversal t;
     traversal_idle(t, st);
     t.any = false;
+    t.margin = 0.0f;
     bool active = false, shadow = false;
     uint32_t at = 0u, tdepth = 0u, transparent_max = 0u, passes = 0u;
     f3 transmittance = V(1.0f, 1.0f, 1.0f);
@@ -100,6 +101,7 @@ __global__ __launch_bounds__(kQueryBlock, 4) void intersect_kernel(SceneView s, 
                                 TraceQuery{q.visibility, q.source_object, q.source_primitive, q.light_object,
                                            q.light_primitive});
                 t.any = shadow;
+                t.margin = far_margin(s, V(q.origin[0], q.origin[1], q.origin[2]));
                 active = true;
             }
         }
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(kQueryBlock, 4) void intersect_kernel(SceneView s, 
         // to 50 transparent slabs).
         const uint32_t busy_min = !exhausted || res < res_end ? 64u - kQueryRefill : 0u;
         do {
-            traversal_advance<false, true>(s, t, st, nodes, tris);
+            traversal_advance<false, true, true>(s, t, st, nodes, tris);
         } while (static_cast<uint32_t>(__popcll(__ballot(traversal_busy(t, st)))) > busy_min);
         if (active && !traversal_busy(t, st)) {
             const Hit b = traversal_result(t, st);

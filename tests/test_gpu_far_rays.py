@@ -1,0 +1,75 @@
+"""Ray queries whose origin lies far outside the scene, against the oracle's
+brute-force search.
+
+The object-space ray of an instance is rounded by the magnitude of its world
+origin, so from far away a silhouette moves by more than any margin that is
+fixed at scene compilation.  The rays here run along an axis, where the slab
+test has no lateral margin of its own, past the extreme vertices of rotated
+instances of one flat mesh.
+"""
+import numpy as np
+import pytest
+
+import oracle_binding as ob
+from psycles_amd import abi, scenes
+from psycles_amd.render import RendererBackend
+
+pytestmark = pytest.mark.gpu
+
+
+def turned_cards(count=40, seed=2):
+    rng = np.random.RandomState(seed)
+    p, t = scenes.quad([[-1, 0, -0.4], [-1, 0, 0.4], [1, 0, 0.4], [1, 0, -0.4]])
+    instances = []
+    for _ in range(count):
+        q, r = np.linalg.qr(rng.normal(size=(3, 3)))
+        m = np.eye(4)
+        m[:3, :3] = q * np.sign(np.diag(r)) * rng.uniform(0.3, 1.5)
+        m[:3, 3] = rng.uniform(-6, 6, 3)
+        instances.append(scenes.InstanceData(0, m))
+    return scenes.SceneSnapshot([scenes.diffuse_material((0.5, 0.5, 0.5))], [scenes.MeshData(p, t, [0])], instances,
+                                scenes.CameraData(scenes.translation(0, 0, 9)), name="turned cards")
+
+
+def silhouette_rays(snap, distance, seed):
+    """For each instance, rays along every axis through its extreme vertices,
+    moved in and out by a few float spacings of the distance."""
+    rng = np.random.RandomState(seed)
+    spacing = float(np.spacing(np.float32(distance)))
+    corners = np.asarray(snap.meshes[0].positions, np.float64).reshape(-1, 3)
+    out = []
+    for inst in snap.instances:
+        m = np.asarray(inst.transform, np.float64).reshape(4, 4)
+        world = corners @ m[:3, :3].T + m[:3, 3]
+        for axis in range(3):
+            for side in range(3):
+                if side == axis:
+                    continue
+                for end in (np.argmin, np.argmax):
+                    v = world[end(world[:, side])]
+                    for step in rng.uniform(-4.0, 4.0, 6):
+                        sign = float(rng.choice([-1.0, 1.0]))
+                        o, d = v.copy(), np.zeros(3)
+                        o[side] += step * spacing
+                        o[axis] = -sign * distance
+                        d[axis] = sign
+                        out.append({"origin": o, "direction": d, "tmin": 0.0, "tmax": 4.0 * distance,
+                                    "visibility": abi.VIS_ALL, "kind": abi.QUERY_CLOSEST})
+    return out
+
+
+@pytest.mark.parametrize("distance", [1.0e1, 1.0e3, 1.0e4, 1.0e5, 1.0e6, 1.0e7])
+def test_silhouettes_from_far(distance):
+    print(f"case: silhouettes from {distance:g}", flush=True)
+    snap = turned_cards()
+    backend = RendererBackend(0)
+    scene = backend.compile_scene(snap).scene
+    oracle = ob.OracleScene(snap, brute_force=True)
+    rays = silhouette_rays(snap, distance, 3)
+    got = [(h.hit, h.object, h.primitive, np.float32(h.t).tobytes()) for h in scene.intersect(rays)]
+    want = [(h.hit, h.object, h.primitive, np.float32(h.t).tobytes()) for h in oracle.intersect(rays)]
+    wrong = sum(a != b for a, b in zip(got, want))
+    print(f"{wrong} of {len(rays)} rays differ, {sum(w[0] for w in want)} hit", flush=True)
+    assert wrong == 0
+    scene.close()
+    backend.close()
