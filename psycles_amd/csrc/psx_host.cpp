@@ -1309,6 +1309,7 @@ void initialize_session(Session &s, const psx_render_settings &rs) {
         s.light.reset();
     }
     if (!s.filter.bytes() || s.filter_kind != rs.pixel_filter || s.filter_width != rs.filter_width) {
+        s.filter_kind = kNone;  // no table until the new one is uploaded
         s.filter.upload(pixel_filter_table(rs.pixel_filter, rs.filter_width));
         s.filter_kind = rs.pixel_filter;
         s.filter_width = rs.filter_width;
@@ -1322,6 +1323,7 @@ void initialize_session(Session &s, const psx_render_settings &rs) {
 void prepare_sobol(Session &s, uint32_t total) {
     const uint32_t size = sequence_size_for(total);
     if (size != s.sobol_size) {
+        s.sobol_size = 0u;  // no table until the new one is made, which can fail
         s.sobol.allocate(static_cast<size_t>(size) * kSobolPatterns * sizeof(float4));
         hip_check(launch_sobol_table(s.sobol.as<float4>(), size, s.stream));
         s.sobol_size = size;
@@ -3220,11 +3222,8 @@ float time_shape(Session &s, const psx_wavefront_tuning &t, const FilmView &film
 int autotune(Session &s, uint32_t probe, psx_tuning_report *report) {
     const psx_backend_options &opt = s.scene->backend->options;
     if (opt.integrator != PSX_INTEGRATOR_WAVEFRONT && !s.light_passes) return PSX_ERROR_UNSUPPORTED;
-    if (s.total_aa != 0u) {
-        probe = std::min(probe, s.total_aa);
-    } else {
-        prepare_sobol(s, probe);
-    }
+    if (s.total_aa != 0u) probe = std::min(probe, s.total_aa);
+    prepare_sobol(s, s.total_aa != 0u ? s.total_aa : probe);
     // scratch film: the probes never touch the session's
     const size_t pixels = static_cast<size_t>(s.window_w) * s.window_h;
     DeviceBuffer combined, normal, albedo, count, light;

@@ -1,0 +1,357 @@
+// memory_failure_driver.cpp - libpsx.so on a device that is only pretended:
+// this program defines the HIP runtime's functions itself, so the library's
+// host code runs without a GPU and allocations can be made to fail.
+//
+// "Device" memory is host memory, kernels do nothing but check that the
+// tables, films and path state they are given are live and large enough, and
+// the render and pass kernels move just enough data to follow pixels from the
+// film to a sink.  Usage: memory_failure_driver <scenario>; prints "ok".
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "psx.h"
+#include "psx_device.h"
+
+namespace {
+
+struct Fake {
+    std::map<const void *, std::string> kernels;  // host stub -> device name
+    std::map<const char *, size_t> live;
+    size_t refuse_bytes = ~static_cast<size_t>(0);  // device allocations of at least this fail
+    long fail_in = -1;                              // the allocation after this many fails
+    int launches = 0;
+    std::vector<std::string> faults;
+};
+// first used by the library's static constructors, before this program's own
+Fake &fake() {
+    static Fake *f = new Fake;
+    return *f;
+}
+
+void fault(const std::string &what) {
+    if (fake().faults.size() < 8u) fake().faults.push_back(what);
+}
+
+void need(const char *kernel, const char *what, const void *p, size_t bytes) {
+    const auto &live = fake().live;
+    auto it = live.upper_bound(static_cast<const char *>(p));
+    if (p && it != live.begin()) {
+        --it;
+        if (static_cast<const char *>(p) + bytes <= it->first + it->second) return;
+    }
+    fault(std::string(kernel) + ": " + what);
+}
+
+template <typename T>
+const T &arg(void **args, int i) {
+    return *static_cast<const T *>(args[i]);
+}
+
+void need_tables(const char *kernel, const psx::KernelParams &k, const float4 *sobol, const float *filter) {
+    need(kernel, "sampler table", sobol, static_cast<size_t>(k.sequence_size) * 256u * 16u);
+    need(kernel, "filter table", filter, 1024u * 4u);
+}
+
+void need_film(const char *kernel, const psx::FilmView &f, size_t n) {
+    need(kernel, "combined", f.combined, n * 16u);
+    need(kernel, "normal", f.normal, n * 16u);
+    need(kernel, "albedo", f.albedo, n * 16u);
+    need(kernel, "sample count", f.sample_count, n * 4u);
+    if (f.light) need(kernel, "light", f.light, n * psx::kLightPasses * 16u);
+}
+
+void need_paths(const char *kernel, const psx::WavefrontView &w) {
+    const size_t n = w.capacity;
+    need(kernel, "path", w.path, n * psx::kPathWords * 16u);
+    need(kernel, "shadow", w.shadow, n * psx::kShadowWords * 16u);
+    need(kernel, "radiance", w.radiance, n * 16u);
+    need(kernel, "normal", w.normal, n * 16u);
+    need(kernel, "albedo", w.albedo, n * 16u);
+    need(kernel, "first hit", w.first_hit, n * 16u);
+    for (int i = 0; i < 2; ++i) {
+        need(kernel, "queue", w.queue[i], n * 8u);
+        need(kernel, "list", w.list[i], n * 4u);
+    }
+    need(kernel, "counters", w.counters, sizeof(psx::WavefrontCounters));
+    if (w.lp) {
+        need(kernel, "light sums", w.lp, n * 160u);
+        need(kernel, "shadow split", w.shadow_split, n * 32u);
+        need(kernel, "shadow transmittance", w.shadow_t, n * 16u);
+    }
+}
+
+// a film whose float number i holds i (in 24 bits) and whose counts are right
+void fill_film(const psx::FilmView &f, size_t pixels, uint32_t samples) {
+    for (size_t i = 0; i < 4u * pixels; ++i) {
+        const float v = static_cast<float>(i & 0xffffffu);
+        f.combined[i] = f.normal[i] = f.albedo[i] = v;
+    }
+    for (size_t i = 0; i < pixels; ++i) f.sample_count[i] += samples;
+}
+
+void run(const std::string &name, void **args) {
+    const char *k = name.c_str();
+    auto is = [&](const char *part) { return name.find(part) != std::string::npos; };
+    if (is("render_kernel")) {
+        const auto &p = arg<psx::KernelParams>(args, 1);
+        const auto &film = arg<psx::FilmView>(args, 4);
+        const size_t n = static_cast<size_t>(p.window_width) * p.window_height;
+        need_tables(k, p, arg<const float4 *>(args, 2), arg<const float *>(args, 3));
+        need_film(k, film, n);
+        if (fake().faults.empty()) fill_film(film, n, arg<uint32_t>(args, 6));
+    } else if (is("generate_kernel")) {
+        need_tables(k, arg<psx::KernelParams>(args, 0), arg<const float4 *>(args, 1), arg<const float *>(args, 2));
+        need_paths(k, arg<psx::WavefrontView>(args, 3));
+    } else if (is("wf_trace_kernel")) {
+        need_paths(k, arg<psx::WavefrontView>(args, 2));
+    } else if (is("wf_shade_kernel")) {
+        need_paths(k, arg<psx::WavefrontView>(args, 3));
+    } else if (is("accumulate_kernel")) {
+        const auto &p = arg<psx::KernelParams>(args, 0);
+        const auto &film = arg<psx::FilmView>(args, 2);
+        const size_t n = static_cast<size_t>(p.window_width) * p.window_height;
+        need_paths(k, arg<psx::WavefrontView>(args, 1));
+        need_film(k, film, n);
+        if (fake().faults.empty()) fill_film(film, n, arg<uint32_t>(args, 3));
+    } else if (is("sobol_kernel")) {
+        need(k, "table", arg<float4 *>(args, 0), static_cast<size_t>(arg<uint32_t>(args, 1)) * 256u * 16u);
+    } else if (is("sampler_kernel")) {
+        need(k, "sampler table", arg<const float4 *>(args, 1),
+             static_cast<size_t>(arg<psx::KernelParams>(args, 0).sequence_size) * 256u * 16u);
+    }
+}
+
+hipError_t take(void **p, size_t bytes, bool device) {
+    Fake &f = fake();
+    *p = nullptr;
+    if (device && (bytes >= f.refuse_bytes || (f.fail_in >= 0 && f.fail_in-- == 0))) return hipErrorOutOfMemory;
+    *p = std::calloc(bytes, 1u);
+    if (!*p) return hipErrorOutOfMemory;
+    f.live[static_cast<char *>(*p)] = bytes;
+    return hipSuccess;
+}
+hipError_t give(void *p) {
+    if (p && fake().live.erase(static_cast<char *>(p)) == 0u) fault("freed twice");
+    std::free(p);
+    return hipSuccess;
+}
+template <typename H>
+hipError_t handle(H *h) {
+    *h = reinterpret_cast<H>(std::malloc(1u));
+    return hipSuccess;
+}
+
+}  // namespace
+
+// ---- the HIP runtime ---------------------------------------------------------
+extern "C" {
+void **__hipRegisterFatBinary(const void *) {
+    static void *module = nullptr;
+    return &module;
+}
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *stub, char *, const char *name, unsigned, void *, void *, void *, void *,
+                           int *) {
+    fake().kernels[stub] = name;
+}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+namespace {
+struct Config {
+    dim3 grid, block;
+    size_t shared;
+    hipStream_t stream;
+} config;
+}  // namespace
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t shared, hipStream_t stream) {
+    config = Config{grid, block, shared, stream};
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hipStream_t *stream) {
+    *grid = config.grid;
+    *block = config.block;
+    *shared = config.shared;
+    *stream = config.stream;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *stub, dim3, dim3, void **args, size_t, hipStream_t) {
+    ++fake().launches;
+    run(fake().kernels[stub], args);
+    return hipSuccess;
+}
+hipError_t hipMalloc(void **p, size_t bytes) { return take(p, bytes, true); }
+hipError_t hipMallocAsync(void **p, size_t bytes, hipStream_t) { return take(p, bytes, true); }
+hipError_t hipFree(void *p) { return give(p); }
+hipError_t hipFreeAsync(void *p, hipStream_t) { return give(p); }
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return take(p, bytes, false); }
+hipError_t hipHostFree(void *p) { return give(p); }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) {
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemset(void *p, int v, size_t n) {
+    need("hipMemset", "target", p, n);
+    if (fake().faults.empty()) std::memset(p, v, n);
+    return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t) { return hipMemset(p, v, n); }
+hipError_t hipGetDeviceCount(int *n) {
+    *n = 1;
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int *d) {
+    *d = 0;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) {
+    *v = 256;
+    return hipSuccess;
+}
+hipError_t hipFuncGetAttributes(hipFuncAttributes *a, const void *) {
+    std::memset(a, 0, sizeof(*a));
+    a->numRegs = 128;
+    return hipSuccess;
+}
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) {
+    *n = 4;
+    return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void **p, const void *) {
+    static char word[16];
+    *p = word;
+    return hipSuccess;
+}
+const char *hipGetErrorName(hipError_t) { return "pretended"; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t *s) { return handle(s); }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return handle(s); }
+hipError_t hipStreamDestroy(hipStream_t s) {
+    std::free(s);
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { return handle(e); }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return handle(e); }
+hipError_t hipEventDestroy(hipEvent_t e) {
+    std::free(e);
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
+    *ms = 1.0f;
+    return hipSuccess;
+}
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *) { return hipSuccess; }
+}  // extern "C"
+
+// ---- scenarios -----------------------------------------------------------------
+namespace {
+
+bool expect(bool ok, const char *what) {
+    if (!ok) std::printf("failed: %s\n", what);
+    return ok;
+}
+#define EXPECT(x) \
+    if (!expect((x), #x)) return 1
+
+struct World {
+    psx_backend *backend = nullptr;
+    psx_scene *scene = nullptr;
+    psx_session *session = nullptr;
+    psx_render_settings settings{};
+    std::vector<uint32_t> passes, channels;
+
+    psx_render_settings sized(uint32_t width, uint32_t height) {
+        psx_render_settings s = settings;
+        s.width = width;
+        s.height = height;
+        return s;
+    }
+    bool make(uint32_t integrator, std::vector<uint32_t> kinds) {
+        psx_backend_options o{1u, 1u, integrator, PSX_BACKEND_NO_GRAPHS};
+        if (psx_backend_create(0, &o, &backend) != PSX_OK) return false;
+        static const float positions[9] = {0, 0, 0, 1, 0, 0, 0, 1, 0};
+        static const uint32_t triangle[3] = {0, 1, 2}, slot[1] = {0};
+        static const float parameters[4] = {0.5f, 0.5f, 0.5f, 0.0f};
+        psx_closure_instr diffuse{};
+        diffuse.op = PSX_CLOSURE_DIFFUSE;
+        diffuse.roughness = 3u;
+        psx_material material{&diffuse, 1u, 0u, parameters, 4u, PSX_EMISSION_SAMPLING_NONE};
+        psx_mesh mesh{positions, 3u, triangle, 1u, nullptr, nullptr, slot, 1u, nullptr};
+        psx_instance instance{};
+        instance.visibility_mask = PSX_VISIBILITY_ALL;
+        psx_scene_desc d{};
+        d.abi_version = PSX_ABI_VERSION;
+        for (int i = 0; i < 4; ++i) instance.transform[5 * i] = d.camera.transform[5 * i] = 1.0f;
+        d.materials = &material;
+        d.material_count = 1u;
+        d.meshes = &mesh;
+        d.mesh_count = 1u;
+        d.instances = &instance;
+        d.instance_count = 1u;
+        d.camera.field_of_view = d.camera.horizontal_field_of_view = 0.8f;
+        d.camera.near_clip = 1.0e-3f;
+        d.camera.far_clip = 100.0f;
+        if (psx_scene_compile(backend, &d, nullptr, nullptr, &scene) != PSX_OK) return false;
+        psx_render_settings_default(&settings);
+        passes = std::move(kinds);
+        channels.assign(passes.size(), 4u);
+        settings.passes = passes.data();
+        settings.pass_channels = channels.data();
+        settings.pass_count = static_cast<uint32_t>(passes.size());
+        const psx_render_settings s = sized(64, 48);
+        return psx_session_create(scene, &s, &session) == PSX_OK;
+    }
+    ~World() {
+        if (session) psx_session_destroy(session);
+        if (scene) psx_scene_destroy(scene);
+        if (backend) psx_backend_destroy(backend);
+    }
+};
+
+// a larger sampler table that cannot be had, then the first one again
+int table(uint32_t integrator) {
+    World w;
+    EXPECT(w.make(integrator, {PSX_PASS_COMBINED}));
+    const psx_render_settings s = w.sized(64, 48);
+    EXPECT(psx_session_render_device(w.session, 0, 1, 16) == PSX_OK);
+    EXPECT(psx_session_reset(w.session, &s) == PSX_OK);
+    fake().refuse_bytes = 8192u * 256u * 16u;
+    EXPECT(psx_session_render_device(w.session, 0, 1, 8192) == PSX_ERROR_OUT_OF_MEMORY);
+    psx_tuning_report report;
+    if (integrator == PSX_INTEGRATOR_WAVEFRONT)
+        EXPECT(psx_session_autotune(w.session, 1u, &report) == PSX_ERROR_OUT_OF_MEMORY);
+    EXPECT(psx_session_reset(w.session, &s) == PSX_OK);
+    EXPECT(psx_session_render_device(w.session, 0, 1, 16) == PSX_OK);
+    fake().refuse_bytes = ~static_cast<size_t>(0);
+    EXPECT(psx_session_reset(w.session, &s) == PSX_OK);
+    EXPECT(psx_session_render_device(w.session, 0, 1, 8192) == PSX_OK);
+    return 0;
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+    if (argc != 2) return 2;
+    const std::string scenario = argv[1];
+    int rc = 2;
+    if (scenario == "table") rc = table(PSX_INTEGRATOR_MEGAKERNEL) || table(PSX_INTEGRATOR_WAVEFRONT);
+    for (const std::string &f : fake().faults) std::printf("fault: %s\n", f.c_str());
+    if (rc != 0 || !fake().faults.empty() || fake().launches == 0) return 1;
+    std::printf("ok\n");
+    return 0;
+}
