@@ -1077,6 +1077,9 @@ struct WavefrontState {
 
     void allocate(uint32_t capacity, uint32_t padded_pixels, uint32_t iterations, bool light_passes) {
         const size_t n = capacity;
+        // no path state until every array is there: one that fails leaves the
+        // others freed
+        view = WavefrontView{};
         light = light_passes;
         if (light_passes) {
             lp.allocate(n * 10u * 16u);

@@ -274,6 +274,7 @@ struct World {
     psx_session *session = nullptr;
     psx_render_settings settings{};
     std::vector<uint32_t> passes, channels;
+    uint32_t samples_per_dispatch = 1u;
 
     psx_render_settings sized(uint32_t width, uint32_t height) {
         psx_render_settings s = settings;
@@ -282,7 +283,7 @@ struct World {
         return s;
     }
     bool make(uint32_t integrator, std::vector<uint32_t> kinds) {
-        psx_backend_options o{1u, 1u, integrator, PSX_BACKEND_NO_GRAPHS};
+        psx_backend_options o{1u, samples_per_dispatch, integrator, PSX_BACKEND_NO_GRAPHS};
         if (psx_backend_create(0, &o, &backend) != PSX_OK) return false;
         static const float positions[9] = {0, 0, 0, 1, 0, 0, 0, 1, 0};
         static const uint32_t triangle[3] = {0, 1, 2}, slot[1] = {0};
@@ -343,6 +344,27 @@ int table(uint32_t integrator) {
     return 0;
 }
 
+// more samples a dispatch than fit, any of the arrays failing, then as many
+// as before; with light passes or without
+int path_state(std::vector<uint32_t> kinds) {
+    for (long nth = 0; nth < 64; ++nth) {
+        World w;
+        w.samples_per_dispatch = 4u;
+        EXPECT(w.make(PSX_INTEGRATOR_WAVEFRONT, kinds));
+        EXPECT(psx_session_render_device(w.session, 0, 2, 64) == PSX_OK);
+        fake().fail_in = nth;
+        const int rc = psx_session_render_device(w.session, 2, 4, 64);
+        const bool all_tried = fake().fail_in >= 0;
+        fake().fail_in = -1;
+        EXPECT(rc == (all_tried ? PSX_OK : PSX_ERROR_OUT_OF_MEMORY));
+        const uint32_t first = all_tried ? 6u : 2u;
+        EXPECT(psx_session_render_device(w.session, first, 1, 64) == PSX_OK);
+        EXPECT(psx_session_render_device(w.session, first + 1u, 4, 64) == PSX_OK);
+        if (all_tried) return 0;
+    }
+    return 1;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -350,6 +372,8 @@ int main(int argc, char **argv) {
     const std::string scenario = argv[1];
     int rc = 2;
     if (scenario == "table") rc = table(PSX_INTEGRATOR_MEGAKERNEL) || table(PSX_INTEGRATOR_WAVEFRONT);
+    if (scenario == "path-state")
+        rc = path_state({PSX_PASS_COMBINED}) || path_state({PSX_PASS_COMBINED, PSX_PASS_DIFFUSE_DIRECT});
     for (const std::string &f : fake().faults) std::printf("fault: %s\n", f.c_str());
     if (rc != 0 || !fake().faults.empty() || fake().launches == 0) return 1;
     std::printf("ok\n");
