@@ -51,7 +51,8 @@ enum {
     PSX_ERROR_OUT_OF_MEMORY = -3,
     PSX_ERROR_CANCELLED = -4,     /* render_samples returned false: cancel   */
     PSX_ERROR_RANGE = -5,         /* render_samples returned false: range    */
-    PSX_ERROR_INCOMPLETE = -6,    /* sample_count readback mismatch         */
+    PSX_ERROR_INCOMPLETE = -6,    /* sample_count readback mismatch, or a
+                                     session whose reset failed             */
     PSX_ERROR_UNSUPPORTED = -7,
     PSX_ERROR_NO_DEVICE = -8
 };
@@ -425,6 +426,8 @@ int psx_scene_update_parameters(psx_scene *scene, uint32_t material,
 int psx_session_create(psx_scene *scene, const psx_render_settings *settings,
                        psx_session **out_session);
 void psx_session_destroy(psx_session *session);
+/* A reset that runs out of memory leaves the session without a film: its
+ * calls return PSX_ERROR_INCOMPLETE until a reset succeeds. */
 int psx_session_reset(psx_session *session,
                       const psx_render_settings *settings);
 /* SampleRange{first, count, offset, total}.  Returns PSX_OK when the sink

@@ -1167,6 +1167,7 @@ struct Session {
     std::vector<uint32_t> passes, pass_channels;
     KernelParams params{};
     uint32_t window_w = 0, window_h = 0;
+    bool ready = false;  // the last reset got its film; until one does, nothing renders or is read
     DeviceBuffer combined, normal, albedo, sample_count, sobol, filter, counters, spill, tile_cursor;
     DeviceBuffer light;        // light-pass sums (kLightPasses float4 per pixel) when requested
     bool light_passes = false;
@@ -1287,18 +1288,20 @@ void keep_settings(Session &s, const psx_render_settings &rs) {
 
 // LuisaRenderSession::initialize (src/luisa/path_tracer_kernel.cpp:44-439)
 void initialize_session(Session &s, const psx_render_settings &rs) {
+    s.ready = false;
     keep_settings(s, rs);
     s.params = kernel_params(*s.scene, s.scene->view, rs);
     const KernelParams &k = s.params;
     s.window_w = k.window_width;
     s.window_h = k.window_height;
     const size_t pixels = static_cast<size_t>(s.window_w) * s.window_h;
-    if (s.sample_count.bytes() != std::max<size_t>(pixels * 4u, 16u)) {
-        s.combined.allocate(pixels * 16u);
-        s.normal.allocate(pixels * 16u);
-        s.albedo.allocate(pixels * 16u);
-        s.sample_count.allocate(pixels * 4u);
-    }
+    auto fit = [](DeviceBuffer &b, size_t bytes) {
+        if (b.bytes() != std::max<size_t>(bytes, 16u)) b.allocate(bytes);
+    };
+    fit(s.combined, pixels * 16u);
+    fit(s.normal, pixels * 16u);
+    fit(s.albedo, pixels * 16u);
+    fit(s.sample_count, pixels * 4u);
     hip_check(hipMemset(s.combined.as<void>(), 0, pixels * 16u));
     hip_check(hipMemset(s.normal.as<void>(), 0, pixels * 16u));
     hip_check(hipMemset(s.albedo.as<void>(), 0, pixels * 16u));
@@ -1306,7 +1309,7 @@ void initialize_session(Session &s, const psx_render_settings &rs) {
     s.light_passes = false;
     for (uint32_t kind : s.passes) s.light_passes |= light_pass_slot(kind) >= 0;
     if (s.light_passes) {
-        if (s.light.bytes() != pixels * kLightPasses * 16u) s.light.allocate(pixels * kLightPasses * 16u);
+        fit(s.light, pixels * kLightPasses * 16u);
         hip_check(hipMemset(s.light.as<void>(), 0, pixels * kLightPasses * 16u));
     } else {
         s.light.reset();
@@ -1320,6 +1323,7 @@ void initialize_session(Session &s, const psx_render_settings &rs) {
     if (!s.counters.bytes()) s.counters.allocate(sizeof(Counters));
     s.total_aa = 0;
     s.rendered = 0;
+    s.ready = true;
 }
 
 // prepare_sobol_table (src/luisa/path_tracer_session.cpp:41-69)
@@ -3066,6 +3070,7 @@ int psx_session_reset(psx_session *handle, const psx_render_settings *rs) {
 
 namespace {
 int check_range(Session *s, uint32_t first, uint32_t count, uint32_t offset, uint32_t total) {
+    if (!s->ready) return PSX_ERROR_INCOMPLETE;
     if (s->cancelled.load()) return PSX_ERROR_CANCELLED;
     if (count == 0u) return PSX_ERROR_RANGE;
     const uint64_t end = static_cast<uint64_t>(first) + offset + count;
@@ -3340,6 +3345,7 @@ int psx_session_autotune(psx_session *handle, uint32_t probe_samples, psx_tuning
     Session *s = reinterpret_cast<Session *>(handle);
     if (!s || probe_samples == 0u || probe_samples > 64u) return PSX_ERROR_INVALID_ARGUMENT;
     return guarded([&] {
+        if (!s->ready) return static_cast<int>(PSX_ERROR_INCOMPLETE);
         hip_check(hipSetDevice(s->scene->backend->device));
         return autotune(*s, probe_samples, report);
     });
@@ -3349,6 +3355,7 @@ int psx_session_read_film(psx_session *handle, float *combined, float *normal, f
     Session *s = reinterpret_cast<Session *>(handle);
     if (!s) return PSX_ERROR_INVALID_ARGUMENT;
     return guarded([&] {
+        if (!s->ready) return static_cast<int>(PSX_ERROR_INCOMPLETE);
         hip_check(hipSetDevice(s->scene->backend->device));
         const size_t n = static_cast<size_t>(s->window_w) * s->window_h;
         if (combined) hip_check(hipMemcpy(combined, s->combined.as<void>(), n * 16u, hipMemcpyDeviceToHost));
@@ -3364,6 +3371,7 @@ int psx_session_read_light_passes(psx_session *handle, float *out) {
     if (!s || !out) return PSX_ERROR_INVALID_ARGUMENT;
     if (!s->light_passes) return PSX_ERROR_UNSUPPORTED;
     return guarded([&] {
+        if (!s->ready) return static_cast<int>(PSX_ERROR_INCOMPLETE);
         hip_check(hipSetDevice(s->scene->backend->device));
         const size_t n = static_cast<size_t>(s->window_w) * s->window_h;
         hip_check(hipMemcpy(out, s->light.as<void>(), n * kLightPasses * 16u, hipMemcpyDeviceToHost));
@@ -3375,6 +3383,7 @@ int psx_session_primary_hits(psx_session *handle, uint32_t sample, uint32_t tota
     Session *s = reinterpret_cast<Session *>(handle);
     if (!s || !out || total == 0u || sample >= total) return PSX_ERROR_INVALID_ARGUMENT;
     return guarded([&] {
+        if (!s->ready) return static_cast<int>(PSX_ERROR_INCOMPLETE);
         hip_check(hipSetDevice(s->scene->backend->device));
         prepare_sobol(*s, total);
         const size_t n = static_cast<size_t>(s->window_w) * s->window_h;
@@ -3392,6 +3401,7 @@ int psx_session_trace_events(psx_session *handle, uint32_t sample, uint32_t tota
     Session *s = reinterpret_cast<Session *>(handle);
     if (!s || !out || total == 0u || sample >= total) return PSX_ERROR_INVALID_ARGUMENT;
     return guarded([&] {
+        if (!s->ready) return static_cast<int>(PSX_ERROR_INCOMPLETE);
         hip_check(hipSetDevice(s->scene->backend->device));
         prepare_sobol(*s, total);
         const size_t n = static_cast<size_t>(s->window_w) * s->window_h;
@@ -3418,6 +3428,7 @@ int psx_session_path_trace(psx_session *handle, uint32_t pixel_x, uint32_t pixel
     const uint32_t x = pixel_x - k.window_x, y = fy - k.window_y;
     if (x >= s->window_w || y >= s->window_h) return PSX_ERROR_INVALID_ARGUMENT;
     return guarded([&] {
+        if (!s->ready) return static_cast<int>(PSX_ERROR_INCOMPLETE);
         hip_check(hipSetDevice(s->scene->backend->device));
         prepare_sobol(*s, total);
         DeviceBuffer slots, rec;
@@ -3452,6 +3463,7 @@ int psx_session_sampler_probe(psx_session *handle, uint32_t sample, uint32_t tot
     Session *s = reinterpret_cast<Session *>(handle);
     if (!s || !out || total == 0u || dim_count == 0u || dim_count > 64u) return PSX_ERROR_INVALID_ARGUMENT;
     return guarded([&] {
+        if (!s->ready) return static_cast<int>(PSX_ERROR_INCOMPLETE);
         hip_check(hipSetDevice(s->scene->backend->device));
         prepare_sobol(*s, total);
         const size_t n = static_cast<size_t>(s->window_w) * s->window_h;

@@ -365,6 +365,41 @@ int path_state(std::vector<uint32_t> kinds) {
     return 1;
 }
 
+// a reset to a larger window, any of the film's arrays failing: the session
+// renders nothing until a reset has succeeded
+int film(std::vector<uint32_t> kinds) {
+    for (long nth = 0; nth < 16; ++nth) {
+        World w;
+        EXPECT(w.make(PSX_INTEGRATOR_MEGAKERNEL, kinds));
+        const psx_render_settings small = w.sized(64, 48), large = w.sized(96, 64);
+        EXPECT(psx_session_render_device(w.session, 0, 1, 16) == PSX_OK);
+        fake().fail_in = nth;
+        const int rc = psx_session_reset(w.session, &large);
+        const bool all_tried = fake().fail_in >= 0;
+        fake().fail_in = -1;
+        EXPECT(rc == (all_tried ? PSX_OK : PSX_ERROR_OUT_OF_MEMORY));
+        if (!all_tried) {
+            std::vector<float> out(96u * 64u * 64u * 12u);
+            std::vector<uint32_t> words(96u * 64u * PSX_TRACE_EVENTS * PSX_TRACE_WORDS);
+            EXPECT(psx_session_render_device(w.session, 0, 1, 16) == PSX_ERROR_INCOMPLETE);
+            EXPECT(psx_session_render(w.session, 0, 1, 0, 16, nullptr) == PSX_ERROR_INCOMPLETE);
+            EXPECT(psx_session_read_film(w.session, out.data(), nullptr, nullptr, nullptr) == PSX_ERROR_INCOMPLETE);
+            EXPECT(psx_session_primary_hits(w.session, 0, 16, words.data()) == PSX_ERROR_INCOMPLETE);
+            EXPECT(psx_session_trace_events(w.session, 0, 16, words.data()) == PSX_ERROR_INCOMPLETE);
+            EXPECT(psx_session_path_trace(w.session, 1, 1, 0, 16, out.data(), nullptr) == PSX_ERROR_INCOMPLETE);
+            EXPECT(psx_session_sampler_probe(w.session, 0, 16, 0, 4, words.data()) == PSX_ERROR_INCOMPLETE);
+            psx_tuning_report report;
+            EXPECT(psx_session_autotune(w.session, 1, &report) == PSX_ERROR_INCOMPLETE);
+        }
+        EXPECT(psx_session_reset(w.session, &small) == PSX_OK);
+        EXPECT(psx_session_render_device(w.session, 0, 1, 16) == PSX_OK);
+        EXPECT(psx_session_reset(w.session, &large) == PSX_OK);
+        EXPECT(psx_session_render_device(w.session, 0, 1, 16) == PSX_OK);
+        if (all_tried) return 0;
+    }
+    return 1;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -374,6 +409,7 @@ int main(int argc, char **argv) {
     if (scenario == "table") rc = table(PSX_INTEGRATOR_MEGAKERNEL) || table(PSX_INTEGRATOR_WAVEFRONT);
     if (scenario == "path-state")
         rc = path_state({PSX_PASS_COMBINED}) || path_state({PSX_PASS_COMBINED, PSX_PASS_DIFFUSE_DIRECT});
+    if (scenario == "film") rc = film({PSX_PASS_COMBINED}) || film({PSX_PASS_COMBINED, PSX_PASS_DIFFUSE_DIRECT});
     for (const std::string &f : fake().faults) std::printf("fault: %s\n", f.c_str());
     if (rc != 0 || !fake().faults.empty() || fake().launches == 0) return 1;
     std::printf("ok\n");
