@@ -818,7 +818,9 @@ typedef struct psx_server_options {
     uint32_t path_capacity;        /* paths per batch (0: 8,388,608)        */
     uint32_t streams;              /* concurrent batches, 2..8 (0: 6); the  */
                                    /* upper half take viewport batches only */
-    uint64_t hbm_budget;           /* bytes for films + batch state (0: 200 GB) */
+    uint64_t hbm_budget;           /* bytes for films + batch state (0: 200 GB); */
+                                   /* a call that writes passes takes up to */
+                                   /* 32 MiB more, or none on a full card   */
     uint32_t viewport_max_pixels;  /* (0: 256,000)                          */
     uint32_t viewport_max_samples; /* (0: 4)                                */
     uint32_t target_batch_ms;      /* final-frame batch length the server   */

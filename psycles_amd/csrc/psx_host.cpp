@@ -126,6 +126,17 @@ class DeviceBuffer {
             hip_check(hipMalloc(&ptr_, bytes));
         bytes_ = bytes;
     }
+    // allocate() for memory that can be done without
+    bool try_allocate(size_t bytes) {
+        reset();
+        if (hipMalloc(&ptr_, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            ptr_ = nullptr;
+            return false;
+        }
+        bytes_ = bytes;
+        return true;
+    }
     // Stream-ordered allocation and release on `stream` from now on: no
     // device-wide synchronisation when the buffer is freed while other
     // streams run.  The stream must outlive the buffer's allocation.
@@ -546,12 +557,21 @@ uint64_t structure_signature(const HostMaterial &m) {
 // ---------------------------------------------------------------------------
 // handles
 // ---------------------------------------------------------------------------
-// What a pass download needs: a stream, device memory for the pass pixels and
-// pinned host memory that the sink reads.
+// Stagings between downloads: pinning 90 MB takes longer than filling it, so
+// a backend keeps up to two of at most kStagingBytes each; concurrent
+// downloads beyond that make their own and free them.
+constexpr size_t kStagingBytes = 256u << 20;
+// Device memory that a download works through a tile at a time, one pass of
+// 1920 x 1080 pixels.
+constexpr size_t kTileBytes = 32u << 20;
+
+// What a pass download needs: a stream, a device tile for the pass pixels and
+// pinned host memory that the sink reads.  A full card has no tile left: the
+// pass kernels then write into the pinned memory themselves.
 struct PassStaging {
     hipStream_t stream = nullptr;
     std::vector<hipEvent_t> events;
-    DeviceBuffer device;
+    DeviceBuffer tile;
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
 
@@ -571,21 +591,18 @@ struct PassStaging {
             hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming));
             events.push_back(e);
         }
-        if (device.bytes() < bytes) device.allocate(bytes);
+        const size_t tile_bytes = std::min(bytes, kTileBytes);
+        if (tile.bytes() < tile_bytes) (void)tile.try_allocate(tile_bytes);
         if (pinned_bytes < bytes) {
             if (pinned) (void)hipHostFree(pinned);
             pinned = nullptr;
             pinned_bytes = 0;
-            hip_check(hipHostMalloc(&pinned, bytes, hipHostMallocDefault));
+            hip_check(hipHostMalloc(&pinned, bytes, hipHostMallocCoherent));
             pinned_bytes = bytes;
         }
     }
 };
 
-// Stagings between downloads: pinning 90 MB takes longer than filling it, so
-// a backend keeps up to two of at most kStagingBytes each; concurrent
-// downloads beyond that make their own and free them.
-constexpr size_t kStagingBytes = 256u << 20;
 struct StagingPool {
     std::mutex mutex;
     std::vector<std::unique_ptr<PassStaging>> idle;
@@ -1571,61 +1588,92 @@ PassRule pass_rule(uint32_t kind, bool light, uint32_t &slot) {
 // write_passes (src/luisa/path_tracer_session.cpp:71-254).  Kernels make the
 // pass pixels, and copies into pinned memory run ahead of the sink's calls.
 // The film of a finished render does not change, so the work goes on the
-// staging's own stream.
+// staging's own stream.  The sink gets each pass in one call.
 int write_passes(Backend &backend, Session &s, const psx_sink *sink) {
     const size_t n = static_cast<size_t>(s.window_w) * s.window_h;
-    const FilmView film{s.combined.as<float>(), s.normal.as<float>(), s.albedo.as<float>(),
-                        s.sample_count.as<uint32_t>(), s.light_passes ? s.light.as<float>() : nullptr};
     const float exposure = s.settings.integrator.film_exposure;
     const bool write = sink && sink->write;
     StagingLease lease(backend.staging);
     PassStaging &stage = *lease;
     constexpr size_t kHead = 256u;  // the count check's word
-    auto pass_bytes = [&](size_t p) {
-        return n * std::max(1u, std::min(s.pass_channels[p], 4u)) * sizeof(float);
+    auto channels = [&](size_t p) { return std::max(1u, std::min(s.pass_channels[p], 4u)); };
+    auto pass_bytes = [&](size_t p) { return n * channels(p) * sizeof(float); };
+    auto film = [&](size_t first) {
+        return FilmView{s.combined.as<float>() + 4u * first, s.normal.as<float>() + 4u * first,
+                        s.albedo.as<float>() + 4u * first, s.sample_count.as<uint32_t>() + first,
+                        s.light_passes ? s.light.as<float>() + 4u * kLightPasses * first : nullptr};
     };
+    // queues `count` pixels of pass p from `first` into pinned memory, then `ready`
+    auto queue = [&](size_t p, size_t first, size_t count, char *pinned, hipEvent_t ready) {
+        uint32_t slot;
+        const PassRule rule = pass_rule(s.passes[p], s.light_passes, slot);
+        const size_t pixel = channels(p) * sizeof(float);
+        const size_t step = stage.tile.bytes() ? stage.tile.bytes() / pixel : count;
+        for (size_t at = 0; at < count; at += step) {
+            const size_t m = std::min(step, count - at);
+            char *host = pinned + at * pixel;
+            char *out = stage.tile.bytes() ? stage.tile.as<char>() : host;
+            hip_check(launch_pass(film(first + at), m, rule, slot, channels(p), exposure,
+                                  reinterpret_cast<float *>(out), stage.stream));
+            if (out != host) hip_check(hipMemcpyAsync(host, out, m * pixel, hipMemcpyDeviceToHost, stage.stream));
+        }
+        hip_check(hipEventRecord(ready, stage.stream));
+    };
+    auto give = [&](size_t p, const char *pixels) {
+        sink->write(sink->user, s.passes[p], channels(p), s.settings.window_x, s.settings.window_y, s.window_w,
+                    s.window_h, s.settings.width, s.settings.height, reinterpret_cast<const float *>(pixels));
+    };
+    bool begun = false;
     size_t done = 0u;
-    bool checked = false;
     do {
-        // as many passes as the staging holds, at least one
+        // as many passes as the staging holds; none of them when the next
+        // one alone is larger
         size_t end = done, bytes = kHead;
-        while (write && end < s.passes.size() && (end == done || bytes + pass_bytes(end) <= kStagingBytes))
+        while (write && end < s.passes.size() && bytes + pass_bytes(end) <= kStagingBytes)
             bytes += pass_bytes(end++);
-        stage.reserve(bytes, end - done + 1u);
-        if (!checked) {
-            hip_check(launch_count_check(film.sample_count, n, s.rendered, stage.device.as<uint32_t>(), stage.stream));
-            hip_check(hipMemcpyAsync(stage.pinned, stage.device.as<void>(), sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                     stage.stream));
+        const bool larger = write && end == done && done < s.passes.size();
+        stage.reserve(larger ? kStagingBytes : bytes, 1u + std::max<size_t>(end - done, 2u));
+        char *const pinned = static_cast<char *>(stage.pinned);
+        if (!begun) {
+            auto *wrong = reinterpret_cast<uint32_t *>(pinned);
+            *wrong = 0u;
+            hip_check(launch_count_check(film(0u).sample_count, n, s.rendered, wrong, stage.stream));
             hip_check(hipEventRecord(stage.events[0], stage.stream));
         }
         size_t at = kHead;
-        for (size_t p = done; p < end; ++p) {
-            uint32_t slot;
-            const PassRule rule = pass_rule(s.passes[p], s.light_passes, slot);
-            char *out = stage.device.as<char>() + at;
-            hip_check(launch_pass(film, n, rule, slot, std::max(1u, std::min(s.pass_channels[p], 4u)), exposure,
-                                  reinterpret_cast<float *>(out), stage.stream));
-            hip_check(hipMemcpyAsync(static_cast<char *>(stage.pinned) + at, out, pass_bytes(p),
-                                     hipMemcpyDeviceToHost, stage.stream));
-            hip_check(hipEventRecord(stage.events[p - done + 1u], stage.stream));
-            at += pass_bytes(p);
-        }
-        if (!checked) {
+        for (size_t p = done; p < end; at += pass_bytes(p++))
+            queue(p, 0u, n, pinned + at, stage.events[p - done + 1u]);
+        if (!begun) {
             hip_check(hipEventSynchronize(stage.events[0]));
-            checked = true;
-            if (*static_cast<const uint32_t *>(stage.pinned) != 0u) {
+            if (*reinterpret_cast<const volatile uint32_t *>(pinned) != 0u) {
                 hip_check(hipStreamSynchronize(stage.stream));
                 return PSX_ERROR_INCOMPLETE;
             }
+            begun = true;
             if (sink && sink->begin) sink->begin(sink->user, &s.settings);
         }
         at = kHead;
-        for (size_t p = done; p < end; ++p) {
+        for (size_t p = done; p < end; at += pass_bytes(p++)) {
             hip_check(hipEventSynchronize(stage.events[p - done + 1u]));
-            sink->write(sink->user, s.passes[p], std::max(1u, std::min(s.pass_channels[p], 4u)), s.settings.window_x,
-                        s.settings.window_y, s.window_w, s.window_h, s.settings.width, s.settings.height,
-                        reinterpret_cast<const float *>(static_cast<const char *>(stage.pinned) + at));
-            at += pass_bytes(p);
+            give(p, pinned + at);
+        }
+        if (larger) {
+            // through the two halves of the staging into memory of its own
+            const size_t pixel = channels(done) * sizeof(float);
+            const size_t part = (kStagingBytes - kHead) / 2u / pixel, parts = (n + part - 1u) / part;
+            std::unique_ptr<char[]> whole(new char[pass_bytes(done)]);
+            auto half = [&](size_t i) { return pinned + kHead + (i & 1u) * part * pixel; };
+            auto count = [&](size_t i) { return std::min(part, n - i * part); };
+            for (size_t i = 0; i < std::min<size_t>(parts, 2u); ++i)
+                queue(done, i * part, count(i), half(i), stage.events[1u + i]);
+            for (size_t i = 0; i < parts; ++i) {
+                hip_check(hipEventSynchronize(stage.events[1u + (i & 1u)]));
+                std::memcpy(whole.get() + i * part * pixel, half(i), count(i) * pixel);
+                if (i + 2u < parts)
+                    queue(done, (i + 2u) * part, count(i + 2u), half(i), stage.events[1u + (i & 1u)]);
+            }
+            give(done, whole.get());
+            ++end;
         }
         done = end;
     } while (write && done < s.passes.size());

@@ -110,11 +110,7 @@ __global__ __launch_bounds__(kPassBlock) void pass_kernel(FilmView film, uint64_
     if (CHANNELS > 3u) o[3] = v.w;
 }
 
-__global__ void clear_word_kernel(uint32_t *word) {
-    if (threadIdx.x == 0u) *word = 0u;
-}
-
-// sets `wrong` when a pixel's count differs from `expected`
+// sets `wrong`, a word of host memory, when a pixel's count differs from `expected`
 __global__ __launch_bounds__(kPassBlock) void count_check_kernel(const uint32_t *counts, uint64_t pixels,
                                                                  uint32_t expected, uint32_t *wrong) {
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kPassBlock + threadIdx.x;
@@ -153,7 +149,6 @@ hipError_t launch_sobol_table(float4 *table, uint32_t size, hipStream_t stream) 
 
 hipError_t launch_count_check(const uint32_t *counts, uint64_t pixels, uint32_t expected, uint32_t *wrong,
                               hipStream_t stream) {
-    hipLaunchKernelGGL(clear_word_kernel, dim3(1), dim3(64), 0, stream, wrong);
     hipLaunchKernelGGL(count_check_kernel, dim3(static_cast<uint32_t>((pixels + kPassBlock - 1u) / kPassBlock)),
                        dim3(kPassBlock), 0, stream, counts, pixels, expected, wrong);
     return hipGetLastError();

@@ -119,6 +119,20 @@ void run(const std::string &name, void **args) {
         need_paths(k, arg<psx::WavefrontView>(args, 1));
         need_film(k, film, n);
         if (fake().faults.empty()) fill_film(film, n, arg<uint32_t>(args, 3));
+    } else if (is("count_check_kernel")) {
+        const auto *counts = arg<const uint32_t *>(args, 0);
+        for (uint64_t i = 0; i < arg<uint64_t>(args, 1); ++i)
+            if (counts[i] != arg<uint32_t>(args, 2)) *arg<uint32_t *>(args, 3) = 1u;
+    } else if (is("pass_kernel")) {
+        const auto &film = arg<psx::FilmView>(args, 0);
+        const uint64_t n = arg<uint64_t>(args, 1);
+        const uint32_t channels = static_cast<uint32_t>(k[name.find("pass_kernelILj") + 14u] - '0');
+        const float *from = arg<psx::PassRule>(args, 2) == psx::PassRule::kCombined ? film.combined : film.normal;
+        auto *out = arg<float *>(args, 5);
+        need(k, "film", from, n * 16u);
+        need(k, "pixels", out, n * channels * 4u);
+        for (uint64_t i = 0; fake().faults.empty() && i < n; ++i)
+            for (uint32_t c = 0; c < channels; ++c) out[i * channels + c] = from[4u * i + c];
     } else if (is("sobol_kernel")) {
         need(k, "table", arg<float4 *>(args, 0), static_cast<size_t>(arg<uint32_t>(args, 1)) * 256u * 16u);
     } else if (is("sampler_kernel")) {
@@ -400,6 +414,51 @@ int film(std::vector<uint32_t> kinds) {
     return 1;
 }
 
+struct Collected {
+    int begun = 0, ended = 0, cancelled = 0;
+    std::vector<uint32_t> kinds;
+    bool right = true;
+};
+psx_sink collect(Collected &c) {
+    psx_sink sink{};
+    sink.user = &c;
+    sink.begin = [](void *u, const psx_render_settings *) { static_cast<Collected *>(u)->begun++; };
+    sink.write = [](void *u, uint32_t kind, uint32_t channels, uint32_t, uint32_t, uint32_t w, uint32_t h, uint32_t,
+                    uint32_t, const float *p) {
+        auto &c = *static_cast<Collected *>(u);
+        c.kinds.push_back(kind);
+        for (size_t i = 0; i < static_cast<size_t>(w) * h; ++i)
+            for (uint32_t k = 0; k < channels; ++k)
+                c.right &= p[i * channels + k] == static_cast<float>((4u * i + k) & 0xffffffu);
+    };
+    sink.end = [](void *u, int cancelled) {
+        static_cast<Collected *>(u)->ended++;
+        static_cast<Collected *>(u)->cancelled = cancelled;
+    };
+    return sink;
+}
+
+// every pass reaches the sink whole, with device memory left or without
+int passes(uint32_t width, uint32_t height, std::vector<uint32_t> channels) {
+    for (bool full : {false, true}) {
+        World w;
+        EXPECT(w.make(PSX_INTEGRATOR_MEGAKERNEL,
+                      std::vector<uint32_t>(channels.size(), static_cast<uint32_t>(PSX_PASS_COMBINED))));
+        w.channels = channels;
+        w.settings.pass_channels = w.channels.data();
+        const psx_render_settings s = w.sized(width, height);
+        EXPECT(psx_session_reset(w.session, &s) == PSX_OK);
+        EXPECT(psx_session_render_device(w.session, 0, 1, 16) == PSX_OK);
+        if (full) fake().refuse_bytes = 0u;
+        Collected c;
+        const psx_sink sink = collect(c);
+        EXPECT(psx_session_render(w.session, 1, 1, 0, 16, &sink) == PSX_OK);
+        fake().refuse_bytes = ~static_cast<size_t>(0);
+        EXPECT(c.begun == 1 && c.ended == 1 && c.cancelled == 0 && c.right && c.kinds.size() == channels.size());
+    }
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -410,6 +469,8 @@ int main(int argc, char **argv) {
     if (scenario == "path-state")
         rc = path_state({PSX_PASS_COMBINED}) || path_state({PSX_PASS_COMBINED, PSX_PASS_DIFFUSE_DIRECT});
     if (scenario == "film") rc = film({PSX_PASS_COMBINED}) || film({PSX_PASS_COMBINED, PSX_PASS_DIFFUSE_DIRECT});
+    if (scenario == "passes")
+        rc = passes(64, 48, {4u, 1u, 3u, 9u}) || passes(1920, 1090, {4u, 2u, 4u}) || passes(4352, 4000, {1u, 4u, 4u, 2u});
     for (const std::string &f : fake().faults) std::printf("fault: %s\n", f.c_str());
     if (rc != 0 || !fake().faults.empty() || fake().launches == 0) return 1;
     std::printf("ok\n");
