@@ -316,6 +316,7 @@ typedef struct psx_sink {
                   uint32_t window_width, uint32_t window_height,
                   uint32_t full_width, uint32_t full_height,
                   const float *pixels);
+    /* follows every begin; cancelled also when the device fails between */
     void (*end)(void *user, int cancelled);
 } psx_sink;
 

@@ -1588,7 +1588,8 @@ PassRule pass_rule(uint32_t kind, bool light, uint32_t &slot) {
 // write_passes (src/luisa/path_tracer_session.cpp:71-254).  Kernels make the
 // pass pixels, and copies into pinned memory run ahead of the sink's calls.
 // The film of a finished render does not change, so the work goes on the
-// staging's own stream.  The sink gets each pass in one call.
+// staging's own stream.  The sink gets each pass in one call, and once it has
+// begun it is ended, as cancelled if the device fails on the way.
 int write_passes(Backend &backend, Session &s, const psx_sink *sink) {
     const size_t n = static_cast<size_t>(s.window_w) * s.window_h;
     const float exposure = s.settings.integrator.film_exposure;
@@ -1624,60 +1625,71 @@ int write_passes(Backend &backend, Session &s, const psx_sink *sink) {
                     s.window_h, s.settings.width, s.settings.height, reinterpret_cast<const float *>(pixels));
     };
     bool begun = false;
-    size_t done = 0u;
-    do {
-        // as many passes as the staging holds; none of them when the next
-        // one alone is larger
-        size_t end = done, bytes = kHead;
-        while (write && end < s.passes.size() && bytes + pass_bytes(end) <= kStagingBytes)
-            bytes += pass_bytes(end++);
-        const bool larger = write && end == done && done < s.passes.size();
-        stage.reserve(larger ? kStagingBytes : bytes, 1u + std::max<size_t>(end - done, 2u));
-        char *const pinned = static_cast<char *>(stage.pinned);
-        if (!begun) {
-            auto *wrong = reinterpret_cast<uint32_t *>(pinned);
-            *wrong = 0u;
-            hip_check(launch_count_check(film(0u).sample_count, n, s.rendered, wrong, stage.stream));
-            hip_check(hipEventRecord(stage.events[0], stage.stream));
-        }
-        size_t at = kHead;
-        for (size_t p = done; p < end; at += pass_bytes(p++))
-            queue(p, 0u, n, pinned + at, stage.events[p - done + 1u]);
-        if (!begun) {
-            hip_check(hipEventSynchronize(stage.events[0]));
-            if (*reinterpret_cast<const volatile uint32_t *>(pinned) != 0u) {
-                hip_check(hipStreamSynchronize(stage.stream));
-                return PSX_ERROR_INCOMPLETE;
+    auto ended = [&](bool cancelled) {
+        if (begun && sink && sink->end) sink->end(sink->user, cancelled ? 1 : 0);
+    };
+    try {
+        size_t done = 0u;
+        do {
+            // as many passes as the staging holds; none of them when the next
+            // one alone is larger
+            size_t end = done, bytes = kHead;
+            while (write && end < s.passes.size() && bytes + pass_bytes(end) <= kStagingBytes)
+                bytes += pass_bytes(end++);
+            const bool larger = write && end == done && done < s.passes.size();
+            stage.reserve(larger ? kStagingBytes : bytes, 1u + std::max<size_t>(end - done, 2u));
+            char *const pinned = static_cast<char *>(stage.pinned);
+            if (!begun) {
+                auto *wrong = reinterpret_cast<uint32_t *>(pinned);
+                *wrong = 0u;
+                hip_check(launch_count_check(film(0u).sample_count, n, s.rendered, wrong, stage.stream));
+                hip_check(hipEventRecord(stage.events[0], stage.stream));
             }
-            begun = true;
-            if (sink && sink->begin) sink->begin(sink->user, &s.settings);
-        }
-        at = kHead;
-        for (size_t p = done; p < end; at += pass_bytes(p++)) {
-            hip_check(hipEventSynchronize(stage.events[p - done + 1u]));
-            give(p, pinned + at);
-        }
-        if (larger) {
-            // through the two halves of the staging into memory of its own
-            const size_t pixel = channels(done) * sizeof(float);
-            const size_t part = (kStagingBytes - kHead) / 2u / pixel, parts = (n + part - 1u) / part;
-            std::unique_ptr<char[]> whole(new char[pass_bytes(done)]);
-            auto half = [&](size_t i) { return pinned + kHead + (i & 1u) * part * pixel; };
-            auto count = [&](size_t i) { return std::min(part, n - i * part); };
-            for (size_t i = 0; i < std::min<size_t>(parts, 2u); ++i)
-                queue(done, i * part, count(i), half(i), stage.events[1u + i]);
-            for (size_t i = 0; i < parts; ++i) {
-                hip_check(hipEventSynchronize(stage.events[1u + (i & 1u)]));
-                std::memcpy(whole.get() + i * part * pixel, half(i), count(i) * pixel);
-                if (i + 2u < parts)
-                    queue(done, (i + 2u) * part, count(i + 2u), half(i), stage.events[1u + (i & 1u)]);
+            size_t at = kHead;
+            for (size_t p = done; p < end; at += pass_bytes(p++))
+                queue(p, 0u, n, pinned + at, stage.events[p - done + 1u]);
+            if (!begun) {
+                hip_check(hipEventSynchronize(stage.events[0]));
+                if (*reinterpret_cast<const volatile uint32_t *>(pinned) != 0u) {
+                    hip_check(hipStreamSynchronize(stage.stream));
+                    return PSX_ERROR_INCOMPLETE;
+                }
+                begun = true;
+                if (sink && sink->begin) sink->begin(sink->user, &s.settings);
             }
-            give(done, whole.get());
-            ++end;
-        }
-        done = end;
-    } while (write && done < s.passes.size());
-    if (sink && sink->end) sink->end(sink->user, s.cancelled.load() ? 1 : 0);
+            at = kHead;
+            for (size_t p = done; p < end; at += pass_bytes(p++)) {
+                hip_check(hipEventSynchronize(stage.events[p - done + 1u]));
+                give(p, pinned + at);
+            }
+            if (larger) {
+                // through the two halves of the staging into memory of its own
+                const size_t pixel = channels(done) * sizeof(float);
+                const size_t part = (kStagingBytes - kHead) / 2u / pixel, parts = (n + part - 1u) / part;
+                std::unique_ptr<char[]> whole(new char[pass_bytes(done)]);
+                auto half = [&](size_t i) { return pinned + kHead + (i & 1u) * part * pixel; };
+                auto count = [&](size_t i) { return std::min(part, n - i * part); };
+                for (size_t i = 0; i < std::min<size_t>(parts, 2u); ++i)
+                    queue(done, i * part, count(i), half(i), stage.events[1u + i]);
+                for (size_t i = 0; i < parts; ++i) {
+                    hip_check(hipEventSynchronize(stage.events[1u + (i & 1u)]));
+                    std::memcpy(whole.get() + i * part * pixel, half(i), count(i) * pixel);
+                    if (i + 2u < parts)
+                        queue(done, (i + 2u) * part, count(i + 2u), half(i), stage.events[1u + (i & 1u)]);
+                }
+                give(done, whole.get());
+                ++end;
+            }
+            done = end;
+        } while (write && done < s.passes.size());
+    } catch (const DeviceError &) {
+        ended(true);
+        throw;
+    } catch (const std::bad_alloc &) {
+        ended(true);
+        throw;
+    }
+    ended(s.cancelled.load());
     return PSX_OK;
 }
 

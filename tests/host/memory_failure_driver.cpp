@@ -25,6 +25,7 @@ struct Fake {
     std::map<const char *, size_t> live;
     size_t refuse_bytes = ~static_cast<size_t>(0);  // device allocations of at least this fail
     long fail_in = -1;                              // the allocation after this many fails
+    long break_in = -1;                             // the wait for an event after this many fails
     int launches = 0;
     std::vector<std::string> faults;
 };
@@ -264,7 +265,10 @@ hipError_t hipEventDestroy(hipEvent_t e) {
 }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) {
+    Fake &f = fake();
+    return f.break_in >= 0 && f.break_in-- == 0 ? hipErrorUnknown : hipSuccess;
+}
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
     *ms = 1.0f;
     return hipSuccess;
@@ -459,6 +463,26 @@ int passes(uint32_t width, uint32_t height, std::vector<uint32_t> channels) {
     return 0;
 }
 
+// a device that fails between a sink's begin and its end
+int broken(uint32_t width, uint32_t height) {
+    World w;
+    EXPECT(w.make(PSX_INTEGRATOR_MEGAKERNEL, {PSX_PASS_COMBINED, PSX_PASS_NORMAL, PSX_PASS_ALBEDO}));
+    const psx_render_settings s = w.sized(width, height);
+    for (long nth = 0;; ++nth) {
+        EXPECT(nth < 32);
+        EXPECT(psx_session_reset(w.session, &s) == PSX_OK);
+        Collected c;
+        const psx_sink sink = collect(c);
+        fake().break_in = nth;
+        const int rc = psx_session_render(w.session, 0, 1, 0, 16, &sink);
+        const bool whole = fake().break_in >= 0;
+        fake().break_in = -1;
+        EXPECT(rc == (whole ? PSX_OK : PSX_ERROR_DEVICE));
+        EXPECT(c.begun == (nth > 0) && c.ended == c.begun && c.cancelled == (nth > 0 && !whole) && c.right);
+        if (whole) return 0;
+    }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -471,6 +495,7 @@ int main(int argc, char **argv) {
     if (scenario == "film") rc = film({PSX_PASS_COMBINED}) || film({PSX_PASS_COMBINED, PSX_PASS_DIFFUSE_DIRECT});
     if (scenario == "passes")
         rc = passes(64, 48, {4u, 1u, 3u, 9u}) || passes(1920, 1090, {4u, 2u, 4u}) || passes(4352, 4000, {1u, 4u, 4u, 2u});
+    if (scenario == "broken") rc = broken(64, 48) || broken(4352, 4000);
     for (const std::string &f : fake().faults) std::printf("fault: %s\n", f.c_str());
     if (rc != 0 || !fake().faults.empty() || fake().launches == 0) return 1;
     std::printf("ok\n");
