@@ -106,5 +106,15 @@ def build_contract_driver() -> Path:
     return out
 
 
+def build_short_operations() -> Path:
+    """Compile tests/short_operations.hip (a device check of three functions
+    of psx_path.h) into _build/, with the library's flags."""
+    hipcc = shutil.which("hipcc") or str(ROCM / "bin" / "hipcc")
+    BUILD.mkdir(exist_ok=True)
+    out = BUILD / "short_operations"
+    _run([hipcc, *HIP_FLAGS, f"-I{CSRC}", str(PKG.parent / "tests" / "short_operations.hip"), "-o", str(out)])
+    return out
+
+
 if __name__ == "__main__":
     print(build_library(verbose=True))

@@ -2269,15 +2269,18 @@ struct TreeImportance {
 };
 
 // Correctly rounded 1 / x, a / x and sqrt(x) in 3, 6 and 6 instructions, where
-// the compiler's, which scale and fix up operands of any size, take 10 to 16.
-// Checked on gfx950 against those: 1 / x and sqrt(x) for every x from 2^-100 to
-// 2^100, a / x for two random a of 2^-20 to 2^20 times the size of each x.
-// lt_quotient takes `y` = lt_reciprocal(x) and any such a and x, or a = 0;
-// lt_root takes 0 or 2^-60 to 2^100 (Markstein, "Computation of elementary
-// functions on the IBM RISC System/6000 processor", 1990).  The descents of the
-// light tree are bound by issue, with 16 of 64 lanes: 1280 x 720 at 32 samples
-// under 4096 lights went from 242.6 to 237.9 ms of kernels, 8 samples at
-// 640 x 360 from 13.2 to 12.9.
+// the compiler's, which scale and fix up operands of any size, take 10 to 16
+// (Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", 1990).  From any approximation within a unit in the last place
+// reciprocal and root are exact but for one mantissa each, and the quotient,
+// which takes `y` = lt_reciprocal(x), is exact short of under- and overflow:
+// tests/host/path_header_driver.cpp tries every mantissa and every pair that
+// could round wrongly.  The device's approximations leave no wrong one: every
+// 1 / x from 2^-100 to 2^100 and every sqrt(x) of 0 and 2^-60 to 2^100, which
+// are the ranges that the functions take (tests/short_operations.hip).  The
+// descents of the light tree are bound by issue, with 16 of 64 lanes: under
+// 10000 emissive triangles and 321 lamps, kernels of 1920 x 1080 at 32 samples
+// went from 242.6 to 237.9 ms, of 256 x 256 at one from 13.2 to 12.9.
 __device__ __forceinline__ float lt_reciprocal(float x) {
     const float y = __builtin_amdgcn_rcpf(x);
     return fmaf(fmaf(-x, y, 1.0f), y, y);
