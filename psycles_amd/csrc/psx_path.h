@@ -306,7 +306,8 @@ typedef __attribute__((address_space(3))) uint32_t LdsWord;
 // Per-lane traversal stack: the top kShortStack entries live in LDS laid out
 // [entry][lane] (bank-conflict free), older entries move to a per-lane column
 // of an HBM spill buffer laid out [entry][lane of the grid].  Scene
-// compilation bounds the depth by kTraversalStackDepth.
+// compilation bounds the depth by kTraversalStackDepth; a stack beyond it would
+// lose entries but touch no word outside its column.
 struct Stack {
     LdsWord *lds;     // this lane's column of the LDS ring; the cold words follow
     uint32_t *spill;  // this lane's spill column
@@ -334,7 +335,7 @@ struct Stack {
         uint32_t e = lds[(sp & (kShortStack - 1u)) * lanes];
         if (sp < bottom) {
             bottom = sp;
-            e = spill[static_cast<size_t>(sp) * stride];
+            e = spill[static_cast<size_t>(sp < kStackDepth ? sp : kStackDepth - 1) * stride];
         }
         return e;
     }

@@ -158,6 +158,45 @@ int quotient() {
     return bad != 0 || all < 90000000 || psx::lt_quotient(0.0f, 3.0f, 1.0f / 3.0f) != 0.0f;
 }
 
+// Pushes in threes and pops as the traversal makes them.  Down to the depth
+// that scene compilation allows, every entry comes back; whatever the depth,
+// only this lane's kTraversalStackDepth spill words are touched.
+int stack() {
+    constexpr uint32_t kLanes = 4u, kLane = 2u, kGuard = 400u, kForeign = 0xdeadbeefu;
+    const uint32_t depth = psx::kTraversalStackDepth, rows = depth + 2u * kGuard;
+    for (uint32_t deepest : {3u, 16u, 17u, 40u, depth - 2u, depth, depth + 1u, depth + 20u, depth + 300u}) {
+        std::vector<uint32_t> lds(psx::kTraversalLds * kLanes, kForeign), spill(rows * kLanes, kForeign);
+        psx::Stack st = psx::make_stack(lds.data(), spill.data() + kGuard * kLanes, kLanes, kLane, kLane, kLanes);
+        std::vector<uint32_t> model;
+        uint32_t seed = deepest, next = 1u;
+        auto random = [&] { return (seed = seed * 1664525u + 1013904223u) >> 16; };
+        for (int step = 0; step < 20000; ++step) {
+            const bool grow = (step / 500) % 2 == 0;
+            if (model.size() + 3u <= deepest && random() % 4u < (grow ? 3u : 1u)) {
+                st.reserve3();
+                for (int i = 0; i < 3; ++i) {
+                    const bool keep = random() % 4u != 0u;
+                    st.push_if(next, keep);
+                    if (keep) model.push_back(next);
+                    ++next;
+                }
+            } else if (!model.empty()) {
+                const uint32_t e = st.pop();
+                if (e == kForeign || (deepest <= depth && e != model.back())) return 1;
+                model.pop_back();
+            }
+            if (st.sp != static_cast<int>(model.size())) return 1;
+        }
+        for (uint32_t i = 0; i < spill.size(); ++i) {
+            const bool own = i % kLanes == kLane && i / kLanes >= kGuard && i / kLanes < kGuard + depth;
+            if (!own && spill[i] != kForeign) return 1;
+        }
+        for (uint32_t i = 0; i < lds.size(); ++i)
+            if ((i % kLanes != kLane || i / kLanes >= psx::kShortStack) && lds[i] != kForeign) return 1;
+    }
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -166,6 +205,7 @@ int main(int argc, char **argv) {
     if (what == "reciprocal") rc = reciprocal();
     if (what == "root") rc = root();
     if (what == "quotient") rc = quotient();
+    if (what == "stack") rc = stack();
     if (rc != 0) return 1;
     std::printf("ok\n");
     return 0;

@@ -1,6 +1,8 @@
-"""The short reciprocal, root and quotient of the light importance
-(psx_path.h): on the host for every approximation that the hardware may give,
-on the device for those it gives."""
+"""Parts of the device header psx_path.h by themselves.
+
+The short reciprocal, root and quotient of the light importance: on the host
+for every approximation that the hardware may give, on the device for those it
+gives.  The traversal stack's bookkeeping, on the host."""
 import shutil
 import subprocess
 
@@ -23,14 +25,14 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("operation", ["reciprocal", "root", "quotient"])
-def test_on_the_host(driver, operation):
-    r = subprocess.run([str(driver), operation], capture_output=True, text=True, timeout=120)
+@pytest.mark.parametrize("part", ["reciprocal", "root", "quotient", "stack"])
+def test_on_the_host(driver, part):
+    r = subprocess.run([str(driver), part], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
 
 
 @pytest.mark.gpu
-def test_on_the_device():
+def test_short_operations_on_the_device():
     exe = build.BUILD / "short_operations"
     if not exe.exists():
         exe = build.build_short_operations()
