@@ -1693,8 +1693,6 @@ int write_passes(Backend &backend, Session &s, const psx_sink *sink) {
     return PSX_OK;
 }
 
-// Scene compilation (LuisaPathTracerBackend::compile_scene,
-// src/luisa/path_tracer_scene.cpp:50-1995, triangle subset)
 // Triangles that an instance weighs in the world tree's split costs: entering
 // one is a change of space and a tree of its own.  Weights of 4 and 48 give
 // the same frame times within 0.3 %.
@@ -1707,6 +1705,8 @@ uint32_t bvh_width(const psx_backend_options &o) {
     return 4u;
 }
 
+// Scene compilation (LuisaPathTracerBackend::compile_scene,
+// src/luisa/path_tracer_scene.cpp:50-1995, triangle subset)
 int compile(Backend *backend, const psx_scene_desc *d, psx_diag_fn diag, void *diag_user, Scene **out) {
     auto fail = [&](const std::string &msg) {
         if (diag) diag(diag_user, msg.c_str());
@@ -2117,7 +2117,6 @@ int compile(Backend *backend, const psx_scene_desc *d, psx_diag_fn diag, void *d
     // upload
     Scene &s = *scene;
     s.nodes.upload(quantize_nodes(nodes));
-    tris.push_back(LeafTri{});  // padding: a leaf step fetches 64 bytes from its 48-byte triangle
     s.tris.upload(tris);
     s.instances_buf.upload(instances);
     s.meshes_buf.upload(scene->meshes);

@@ -396,7 +396,6 @@ hipError_t launch_material_tables(const SceneView &s, float4 *shadow, float4 *em
     return hipGetLastError();
 }
 
-// after launch_material_tables on the same stream (reads s.material_shadow)
 hipError_t launch_light_measures(const TreeNode *nodes, uint32_t node_count, const TreeEmitter *emitters,
                                  uint32_t emitter_count, LightMeasure *node_measures, LightMeasure *emitter_measures,
                                  hipStream_t stream) {
@@ -407,6 +406,7 @@ hipError_t launch_light_measures(const TreeNode *nodes, uint32_t node_count, con
     return hipGetLastError();
 }
 
+// after launch_material_tables on the same stream (reads s.material_shadow)
 hipError_t launch_instance_opacity(const SceneView &s, uint32_t *flags, uint32_t count, hipStream_t stream) {
     if (count == 0u) return hipSuccess;
     hipLaunchKernelGGL(instance_opacity_kernel, dim3((count + 63u) / 64u), dim3(64), 0, stream, s, flags, count);

@@ -82,7 +82,7 @@ def test_pass_pixels(width, height, channels):
         backend.close()
 
 
-@pytest.mark.parametrize("total", [1, 257, 1024, 2049, 8192])
+@pytest.mark.parametrize("total", [1, 257, 1024, 1025, 2049, 8192])
 def test_sampler_tables(total):
     """One table per size from 256 to 8192, in one session that is reset."""
     print(f"case: sampler table for {total} samples", flush=True)

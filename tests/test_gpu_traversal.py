@@ -123,8 +123,8 @@ def test_queries_match_oracle(name, n):
 
 @pytest.mark.parametrize("width,height,spp", [(1, 1, 1), (8, 8, 1), (17, 3, 2), (64, 64, 1), (257, 129, 3), (640, 400, 9)])
 def test_short_queues(width, height, spp):
-    """Queues from one entry to several reservations a wave (4096 waves, 16 to
-    128 entries each): the trace kernel deals them out; film and ray count are
+    """Queues from one entry to several reservations a wave (4096 waves, 64 to
+    256 entries each): the trace kernel deals them out; film and ray count are
     those of the one-lane-per-path kernel."""
     print(f"case: short queues {width}x{height}x{spp}", flush=True)
     snap = scenes.cornell_lamps()
@@ -139,6 +139,29 @@ def test_short_queues(width, height, spp):
         scene.close()
         backend.close()
     assert films[0] == films[1]
+
+
+@pytest.mark.parametrize("shape", [
+    {"trace_chunk": 16, "refill_lanes": 1}, {"trace_chunk": 16, "refill_lanes": 64, "list_chunk": 64},
+    {"trace_chunk": 4096, "list_chunk": 256}, {"queue_chunk": 128, "list_chunk": 256}])
+def test_long_queues_of_other_shapes(shape):
+    """Reservations of 32 to 8192 queue entries and 128 to 512 list entries,
+    on queues that hold many of the small ones and fewer than one of the large
+    ones a wave: film and ray count are those of the default shape."""
+    print(f"case: long queues, {shape}", flush=True)
+    backend = RendererBackend(0, integrator=abi.INTEGRATOR_WAVEFRONT, max_samples_per_dispatch=3)
+    scene = backend.compile_scene(scenes.cornell_lamps()).scene
+    films = []
+    for tuning in ({}, shape):
+        session = backend.create_session(scene, scenes.cornell_settings(643, 401))
+        if tuning:
+            session.set_tuning(tuning)
+        session.render_device(0, 3, 3)
+        films.append([a.tobytes() for a in session.read_film()] + [session.stats().rays])
+        session.close()
+    assert films[0] == films[1]
+    scene.close()
+    backend.close()
 
 
 @pytest.mark.parametrize("n", [1, 65, 4099, 300001])
