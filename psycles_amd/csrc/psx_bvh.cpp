@@ -360,44 +360,45 @@ std::vector<QNode4> quantize_nodes(const std::vector<Node4> &nodes) {
     return out;
 }
 
-void transformed_bounds(const std::vector<Node4> &nodes, const std::vector<LeafTri> &tris, uint32_t root,
-                        const float *transform, double lo[3], double hi[3]) {
-    std::vector<uint32_t> stack;
+uint32_t transformed_bounds(const std::vector<Node4> &nodes, const std::vector<LeafTri> &tris, uint32_t root,
+                            const float *transform, uint32_t budget, double lo[3], double hi[3]) {
+    struct Open {
+        double reach;
+        uint32_t node;
+        bool operator<(const Open &o) const { return reach < o.reach; }
+    };
+    std::vector<Open> heap;  // the node that reaches furthest is opened next
+    uint32_t all = 0u;
     for (int side = 0; side < 6; ++side) {
         const int axis = side >> 1;
         const double sign = (side & 1) != 0 ? -1.0 : 1.0;
         const double m[3] = {sign * transform[axis], sign * transform[4 + axis], sign * transform[8 + axis]};
         double best = -HUGE_VAL, tolerance = 0.0;
-        stack.assign(1, root);
-        while (!stack.empty()) {
-            const Node4 &n = nodes[stack.back()];
-            stack.pop_back();
+        heap.assign(1, Open{HUGE_VAL, root});
+        for (uint32_t opened = 0u; !heap.empty() && heap.front().reach > best + tolerance; ++opened, ++all) {
+            const Open top = heap.front();
+            if (opened == budget) {
+                best = top.reach;  // the rest of the mesh reaches no further
+                break;
+            }
+            std::pop_heap(heap.begin(), heap.end());
+            heap.pop_back();
+            const Node4 &n = nodes[top.node];
             const float *nlo[3] = {n.lo_x, n.lo_y, n.lo_z}, *nhi[3] = {n.hi_x, n.hi_y, n.hi_z};
-            double reach[4];
-            int order[4], k = 0;
             double widest = 0.0;
             for (int i = 0; i < 4; ++i) {
                 if (n.count[i] == kEmptySlot) continue;
-                reach[i] = 0.0;
-                double magnitude = 0.0, extent = 0.0;
+                double reach = 0.0, magnitude = 0.0, extent = 0.0;
                 for (int a = 0; a < 3; ++a) {
-                    reach[i] += std::max(m[a] * nlo[a][i], m[a] * nhi[a][i]);
+                    reach += std::max(m[a] * nlo[a][i], m[a] * nhi[a][i]);
                     magnitude += std::max(std::fabs(m[a] * nlo[a][i]), std::fabs(m[a] * nhi[a][i]));
                     extent += std::fabs(m[a] * nhi[a][i] - m[a] * nlo[a][i]);
                 }
                 widest = std::max(widest, 1.0e-4 * extent + 4.0e-5 * magnitude);
-                order[k++] = i;
-            }
-            // a flat mesh has all its boxes, which are padded, reach past
-            // its vertices: what is this near is not searched but allowed for
-            if (tolerance == 0.0) tolerance = widest;
-            // the furthest child is searched first: it is pushed last
-            std::sort(order, order + k, [&](int a, int b) { return reach[a] < reach[b]; });
-            for (int j = 0; j < k; ++j) {
-                const int i = order[j];
-                if (reach[i] <= best + tolerance) continue;
+                if (reach <= best + tolerance) continue;
                 if (n.count[i] == 0u) {
-                    stack.push_back(n.child[i]);
+                    heap.push_back(Open{reach, n.child[i]});
+                    std::push_heap(heap.begin(), heap.end());
                     continue;
                 }
                 for (uint32_t t = n.child[i]; t < n.child[i] + n.count[i]; ++t) {
@@ -407,6 +408,9 @@ void transformed_bounds(const std::vector<Node4> &nodes, const std::vector<LeafT
                     best = std::max(best, m[0] * l.p2x + m[1] * l.p2y + m[2] * l.p2z);
                 }
             }
+            // a flat mesh has all its boxes, which are padded, reach past
+            // its vertices: what is this near is not searched but allowed for
+            if (tolerance == 0.0) tolerance = widest;
         }
         best += tolerance;
         if (sign > 0.0)
@@ -414,6 +418,7 @@ void transformed_bounds(const std::vector<Node4> &nodes, const std::vector<LeafT
         else
             lo[axis] = transform[12 + axis] - best;
     }
+    return all;
 }
 
 }  // namespace psx

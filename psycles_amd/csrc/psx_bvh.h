@@ -38,10 +38,12 @@ QNode4 quantize_node(const Node4 &n);
 
 // Bounds of the triangles under `root` (leaves hold triangles only) after the
 // affine map `transform` (column-major 4x4), in double precision: six support
-// searches that descend only where a node's box reaches past the best vertex
-// so far.  A box of eight transformed corners is up to sqrt(3) times as wide
-// for a rotated instance.
-void transformed_bounds(const std::vector<Node4> &nodes, const std::vector<LeafTri> &tris, uint32_t root,
-                        const float *transform, double lo[3], double hi[3]);
+// searches that open the nodes whose boxes reach past the best vertex so far,
+// the furthest first and at most `budget` of them each; where more are left the
+// bound is the box of the furthest.  Returns how many were opened.  A box of
+// eight transformed corners is up to sqrt(3) times as wide for a rotated
+// instance.
+uint32_t transformed_bounds(const std::vector<Node4> &nodes, const std::vector<LeafTri> &tris, uint32_t root,
+                            const float *transform, uint32_t budget, double lo[3], double hi[3]);
 
 }  // namespace psx
