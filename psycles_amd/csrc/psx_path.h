@@ -727,12 +727,7 @@ __device__ __forceinline__ void traversal_advance(const SceneView &s, Traversal 
     const bool run_leaf = !run_change && n_leaf >= n_node;
     if (changes && run_change) traversal_change_space<ANYHIT>(s, t, st);
     if (leaf && run_leaf) traversal_leaf<COUNT, ANYHIT>(s, t, st, tri_count);
-    if (node && !run_change && !run_leaf) {
-        if (FAR && __builtin_amdgcn_ballot_w64(t.margin > 0.0f) != 0ull)
-            traversal_node<COUNT, true>(s, t, st, node_count);
-        else
-            traversal_node<COUNT, false>(s, t, st, node_count);
-    }
+    if (node && !run_change && !run_leaf) traversal_node<COUNT, FAR>(s, t, st, node_count);
 }
 
 template <bool COUNT>

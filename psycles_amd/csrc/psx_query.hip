@@ -11,6 +11,7 @@
 // probe_kernel evaluates one device function per input record, so tests can
 // hold the device code itself against the reference's function fixtures.
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/psx.h"
 #include "psx_launch.h"
@@ -116,9 +117,17 @@ __global__ __launch_bounds__(kQueryBlock, 4) void intersect_kernel(SceneView s, 
         // waves of one kind took 290: 60000 queries, 95 % shadows through up
         // to 50 transparent slabs).
         const uint32_t busy_min = !exhausted || res < res_end ? 64u - kQueryRefill : 0u;
-        do {
-            traversal_advance<false, true, true>(s, t, st, nodes, tris);
-        } while (static_cast<uint32_t>(__popcll(__ballot(traversal_busy(t, st)))) > busy_min);
+        auto advance = [&](auto far) {
+            do {
+                traversal_advance<false, true, decltype(far)::value>(s, t, st, nodes, tris);
+            } while (static_cast<uint32_t>(__popcll(__ballot(traversal_busy(t, st)))) > busy_min);
+        };
+        // a loop of its own for waves with a far ray: the choice at each node
+        // cost the others 1 %
+        if (__ballot(active && t.margin > 0.0f) != 0ull)
+            advance(std::true_type{});
+        else
+            advance(std::false_type{});
         if (active && !traversal_busy(t, st)) {
             const Hit b = traversal_result(t, st);
             ++passes;

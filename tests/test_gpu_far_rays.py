@@ -73,3 +73,24 @@ def test_silhouettes_from_far(distance):
     assert wrong == 0
     scene.close()
     backend.close()
+
+
+def test_near_and_far_rays_share_waves():
+    """Closest hits and shadows from near and far in one call: what a wave does
+    for its far rays changes nothing for the others."""
+    print("case: near and far rays together", flush=True)
+    snap = turned_cards()
+    backend = RendererBackend(0)
+    scene = backend.compile_scene(snap).scene
+    oracle = ob.OracleScene(snap, brute_force=True)
+    rays = [q for group in zip(*(silhouette_rays(snap, d, 7)[::3] for d in (10.0, 1.0e6, 30.0, 1.0e5))) for q in group]
+    for i, q in enumerate(rays):
+        if i % 8 in (2, 5):
+            q["kind"], q["visibility"] = abi.QUERY_SHADOW, abi.VIS_SHADOW
+    got, want = scene.intersect(rays), oracle.intersect(rays)
+    assert 0.2 < np.mean([w.hit for w in want]) < 0.8
+    for a, b in zip(got, want):
+        assert (a.hit, a.object, a.primitive) == (b.hit, b.object, b.primitive)
+        assert np.float32([a.t, *a.transmittance]).tobytes() == np.float32([b.t, *b.transmittance]).tobytes()
+    scene.close()
+    backend.close()
