@@ -606,6 +606,7 @@ struct PassStaging {
 struct StagingPool {
     std::mutex mutex;
     std::vector<std::unique_ptr<PassStaging>> idle;
+    StagingPool() { idle.reserve(2u); }  // giving one back allocates nothing
 };
 
 class StagingLease {
