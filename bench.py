@@ -449,7 +449,7 @@ def main() -> int:
             # WRITE_SIZE per ray) over the same launch time give the
             # bandwidth the kernel really draws
             "basis": "achieved: algorithmic B_ray = 48 + 32 N_node + 36 N_tri bytes per ray (binary SAH BVH); "
-                     "which the kernel's BVH4 undercuts, so frac can exceed 1; "
+                     "the kernel's BVH4 undercuts it, so frac can exceed 1; "
                      "traffic: measured HBM bytes per launch, of which traffic_frac is the share of the peak",
             "traffic_gbs": traffic_gbs,
             "traffic_frac": traffic_gbs / HBM_PEAK_GBS if traffic_gbs else None,

@@ -1978,12 +1978,12 @@ int compile(Backend *backend, const psx_scene_desc *d, psx_diag_fn diag, void *d
     // for 16 times as far cost 3 % of the many-light frame (243.9 -> 251.0 ms).
     double far_slack = 0.0;
     // Nodes that a support search of an instance may open, which bounds the
-    // boxes of any number of instances to about half a second.  A sphere of
+    // boxes of any number of instances to a quarter of a second.  A sphere of
     // 200000 triangles, the worst case, takes some 300 a side, 0.3 ms, for its
-    // exact box: 3 s for 10000 of them, whose boxes 52 nodes a side leave 0.5 %
-    // too wide.  Without any budget to speak of a box is still within the
+    // exact box: 3 s for 10000 of them, whose boxes 26 nodes a side leave 1 %
+    // too wide.  However few are left, a box lies within that of the
     // transformed corners of the mesh's.
-    const uint32_t budget = std::max(1u, (1u << 19) / std::max(d->instance_count, 1u));
+    const uint32_t budget = std::max(1u, (1u << 18) / std::max(d->instance_count, 1u));
     auto rounding_gain = [](const float *m, const Affine &w2o, int a) {
         double gain = 1.0;
         for (int o = 0; o < 3; ++o)
