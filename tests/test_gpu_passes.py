@@ -5,6 +5,8 @@ sums (bit for bit), for every rule and channel count, at pixel counts around
 a block's edge; a session that is reset keeps its table only while the sample
 total needs the same size; tables of every size against the oracle's sampler.
 """
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -95,5 +97,35 @@ def test_sampler_tables(total):
             assert np.array_equal(session.sampler_probe(sample, n, 0, 20), ob.sampler_probe(s, sample, n, 0, 20))
         session.reset(s)
     session.close()
+    scene.close()
+    backend.close()
+
+
+def test_concurrent_downloads():
+    """Six sessions of one backend read their passes at once, more than the
+    stagings that the backend keeps: every sink gets its own film's pixels."""
+    print("case: six sessions read their passes at once", flush=True)
+    kinds = ((abi.PASS_COMBINED, 4), (abi.PASS_NORMAL, 3), (abi.PASS_ALBEDO, 3), (abi.PASS_SAMPLE_COUNT, 1))
+    backend = RendererBackend(0, integrator=abi.INTEGRATOR_WAVEFRONT, graphs=False)
+    scene = backend.compile_scene(scenes.cornell_lamps()).scene
+
+    def render(seed):
+        s, keep = with_passes(scenes.cornell_settings(200 + 37 * seed, 150), kinds)
+        s.seed = seed
+        session = backend.create_session(scene, s)
+        out = []
+        for _ in range(4):
+            sink = MemoryOutputSink()
+            session.reset(s)
+            assert session.render_samples(SampleRange(0, 2, 0, 16), sink)
+            out.append({k: v.tobytes() for k, v in sink.passes.items()})
+        session.close()
+        return out
+
+    alone = [render(seed)[0] for seed in range(6)]
+    with ThreadPoolExecutor(6) as pool:
+        together = list(pool.map(render, range(6)))
+    for want, got in zip(alone, together):
+        assert all(g == want for g in got)
     scene.close()
     backend.close()
