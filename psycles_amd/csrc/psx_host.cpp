@@ -752,6 +752,25 @@ struct Scene {
         refresh_material_tables(*fresh);
         tables = std::move(fresh);
     }
+    // Binds parameters to a material as a new version; if a table of it cannot
+    // be had, the scene stays as it was.
+    void bind_parameters(uint32_t material, std::vector<float> params) {
+        HostMaterial &m = materials[material];
+        const SceneView before = view;
+        const bool emitted = m.may_emit;
+        m.params.swap(params);
+        try {
+            refresh_may_emit(m);
+            gpu_materials[material].may_emit = m.may_emit ? 1u : 0u;
+            apply_parameter_version(emitted || m.may_emit);
+        } catch (...) {
+            m.params.swap(params);
+            m.may_emit = emitted;
+            gpu_materials[material].may_emit = emitted ? 1u : 0u;
+            view = before;
+            throw;
+        }
+    }
     void rebuild_emitters(ParamTables &t);
 
     // Triangles whose material can emit for some parameter block (its
@@ -2610,15 +2629,10 @@ struct Server {
                     edits.erase(it);
                     editing.insert(op.scene);
                 }
-                HostMaterial &m = op.scene->materials[op.material];
-                m.params = op.params;
-                const bool emitted = m.may_emit;
-                refresh_may_emit(m);
-                op.scene->gpu_materials[op.material].may_emit = m.may_emit ? 1u : 0u;
                 // stream-ordered allocations and copies on the scene's
                 // table stream, which never synchronises with the null
                 // stream, so edits need not wait for the capture gate
-                op.scene->apply_parameter_version(emitted || m.may_emit);
+                op.scene->bind_parameters(op.material, std::move(op.params));
                 {
                     std::lock_guard<std::mutex> lock(mutex);
                     SceneVersions &v = versions_of(op.scene);
@@ -3082,16 +3096,10 @@ void psx_scene_destroy(psx_scene *s) {
 int psx_scene_update_parameters(psx_scene *handle, uint32_t material, const float *p, uint32_t count) {
     Scene *s = reinterpret_cast<Scene *>(handle);
     if (!s || !p || material >= s->materials.size()) return PSX_ERROR_INVALID_ARGUMENT;
-    HostMaterial &m = s->materials[material];
-    if (count != m.params.size()) return PSX_ERROR_INVALID_ARGUMENT;
+    if (count != s->materials[material].params.size()) return PSX_ERROR_INVALID_ARGUMENT;
     return guarded([&] {
         hip_check(hipSetDevice(s->backend->device));
-        m.params.assign(p, p + count);
-        const bool emitted = m.may_emit;
-        refresh_may_emit(m);
-        Material &g = s->gpu_materials[material];
-        g.may_emit = m.may_emit ? 1u : 0u;
-        s->apply_parameter_version(emitted || m.may_emit);
+        s->bind_parameters(material, std::vector<float>(p, p + count));
         hip_check(hipEventSynchronize(s->tables->ready));
         return static_cast<int>(PSX_OK);
     });

@@ -59,6 +59,24 @@ void need_tables(const char *kernel, const psx::KernelParams &k, const float4 *s
     need(kernel, "filter table", filter, 1024u * 4u);
 }
 
+// the tables of the scene's parameter version
+void need_scene(const char *kernel, const psx::SceneView &s) {
+    need(kernel, "parameters", s.params, 4u);
+    need(kernel, "materials", s.materials, s.material_count * sizeof(psx::Material));
+    need(kernel, "material shadow", s.material_shadow, s.material_count * 16u);
+    need(kernel, "material emission", s.material_emission, s.material_count * 16u);
+    need(kernel, "instance opacity", s.instance_opaque, s.instance_count * 4u);
+    if (s.emitter_count == 0u) return;
+    need(kernel, "emitters", s.emitters, s.emitter_count * sizeof(psx::Emitter));
+    need(kernel, "distribution", s.distribution, s.distribution_count * sizeof(psx::DistEntry));
+    need(kernel, "tree nodes", s.tree_nodes, s.tree_node_count * sizeof(psx::TreeNode));
+    need(kernel, "tree emitters", s.tree_emitters, s.tree_emitter_count * sizeof(psx::TreeEmitter));
+    need(kernel, "tree mapping", s.tree_mapping, s.tree_emitter_count * 8u);
+    need(kernel, "emitter primitives", s.emitter_cprim, s.emitter_count * 4u);
+    need(kernel, "node measures", s.node_measures, s.tree_node_count * sizeof(psx::LightMeasure));
+    need(kernel, "emitter measures", s.emitter_measures, s.tree_emitter_count * sizeof(psx::LightMeasure));
+}
+
 void need_film(const char *kernel, const psx::FilmView &f, size_t n) {
     need(kernel, "combined", f.combined, n * 16u);
     need(kernel, "normal", f.normal, n * 16u);
@@ -103,6 +121,7 @@ void run(const std::string &name, void **args) {
         const auto &p = arg<psx::KernelParams>(args, 1);
         const auto &film = arg<psx::FilmView>(args, 4);
         const size_t n = static_cast<size_t>(p.window_width) * p.window_height;
+        need_scene(k, arg<psx::SceneView>(args, 0));
         need_tables(k, p, arg<const float4 *>(args, 2), arg<const float *>(args, 3));
         need_film(k, film, n);
         if (fake().faults.empty()) fill_film(film, n, arg<uint32_t>(args, 6));
@@ -293,6 +312,7 @@ struct World {
     psx_render_settings settings{};
     std::vector<uint32_t> passes, channels;
     uint32_t samples_per_dispatch = 1u;
+    bool emissive = false;
 
     psx_render_settings sized(uint32_t width, uint32_t height) {
         psx_render_settings s = settings;
@@ -307,9 +327,11 @@ struct World {
         static const uint32_t triangle[3] = {0, 1, 2}, slot[1] = {0};
         static const float parameters[4] = {0.5f, 0.5f, 0.5f, 0.0f};
         psx_closure_instr diffuse{};
-        diffuse.op = PSX_CLOSURE_DIFFUSE;
-        diffuse.roughness = 3u;
-        psx_material material{&diffuse, 1u, 0u, parameters, 4u, PSX_EMISSION_SAMPLING_NONE};
+        diffuse.op = emissive ? PSX_CLOSURE_EMISSION : PSX_CLOSURE_DIFFUSE;
+        (emissive ? diffuse.strength : diffuse.roughness) = 3u;
+        static const float glow[4] = {0.5f, 0.5f, 0.5f, 1.0f};
+        psx_material material{&diffuse, 1u, 0u, emissive ? glow : parameters, 4u,
+                              emissive ? PSX_EMISSION_SAMPLING_FRONT_BACK : PSX_EMISSION_SAMPLING_NONE};
         psx_mesh mesh{positions, 3u, triangle, 1u, nullptr, nullptr, slot, 1u, nullptr};
         psx_instance instance{};
         instance.visibility_mask = PSX_VISIBILITY_ALL;
@@ -418,6 +440,28 @@ int film(std::vector<uint32_t> kinds) {
     return 1;
 }
 
+// new parameters of which a table cannot be had: the scene keeps its old ones,
+// and takes the new ones when there is memory again
+int parameters(bool emissive) {
+    for (long nth = 0; nth < 32; ++nth) {
+        World w;
+        w.emissive = emissive;
+        EXPECT(w.make(PSX_INTEGRATOR_MEGAKERNEL, {PSX_PASS_COMBINED}));
+        EXPECT(psx_session_render_device(w.session, 0, 1, 16) == PSX_OK);
+        const float other[4] = {0.25f, 0.5f, 0.75f, emissive ? 2.0f : 0.0f};
+        fake().fail_in = nth;
+        const int rc = psx_scene_update_parameters(w.scene, 0u, other, 4u);
+        const bool all_tried = fake().fail_in >= 0;
+        fake().fail_in = -1;
+        EXPECT(rc == (all_tried ? PSX_OK : PSX_ERROR_OUT_OF_MEMORY));
+        EXPECT(psx_session_render_device(w.session, 1, 1, 16) == PSX_OK);
+        EXPECT(psx_scene_update_parameters(w.scene, 0u, other, 4u) == PSX_OK);
+        EXPECT(psx_session_render_device(w.session, 2, 1, 16) == PSX_OK);
+        if (all_tried) return 0;
+    }
+    return 1;
+}
+
 struct Collected {
     int begun = 0, ended = 0, cancelled = 0;
     std::vector<uint32_t> kinds;
@@ -495,6 +539,7 @@ int main(int argc, char **argv) {
     if (scenario == "film") rc = film({PSX_PASS_COMBINED}) || film({PSX_PASS_COMBINED, PSX_PASS_DIFFUSE_DIRECT});
     if (scenario == "passes")
         rc = passes(64, 48, {4u, 1u, 3u, 9u}) || passes(1920, 1090, {4u, 2u, 4u}) || passes(4352, 4000, {1u, 4u, 4u, 2u});
+    if (scenario == "parameters") rc = parameters(false) || parameters(true);
     if (scenario == "broken") rc = broken(64, 48) || broken(4352, 4000);
     for (const std::string &f : fake().faults) std::printf("fault: %s\n", f.c_str());
     if (rc != 0 || !fake().faults.empty() || fake().launches == 0) return 1;

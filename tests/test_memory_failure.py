@@ -23,7 +23,7 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["table", "path-state", "film", "passes", "broken"])
+@pytest.mark.parametrize("scenario", ["table", "path-state", "film", "passes", "broken", "parameters"])
 def test_after_a_failed_allocation(driver, scenario):
     r = subprocess.run([str(driver), scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
